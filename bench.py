@@ -278,12 +278,10 @@ APPLY_KERNELS = {
 
 
 def query_kernel(geo, k):
-    """The query kernel the library launches for k results: the K bucket,
-    the one- or two-pass form (two passes from K = 32 for float and K = 16
-    for double coordinates) and the 22-entry LDS stack."""
-    kb = next(v for v in (1, 4, 8, 10, 16, 24, 32, 48, 64) if k <= v)
-    two = kb >= (32 if geo == "float" else 16)
-    return f"knn_query{'2' if two else ''}_kernel<{geo},{kb},22>"
+    """The query kernel the library launches for k results: the group search
+    with the row slots that k takes (16, 32, 64 or 128)."""
+    slots = 16 if k <= 8 else 32 if k <= 20 else 64 if k <= 42 else 128
+    return f"knn_group_kernel<{geo},{slots}>"
 
 
 def kernel_rooflines(form, r, n, m, kk, nnz, fields):

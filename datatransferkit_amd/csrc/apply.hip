@@ -180,7 +180,7 @@ __global__ void __launch_bounds__( kBlock )
 // whole-record reads. Stored straight from the rows, targets in random
 // caller order scatter one value per field and row: at 1M x 1M (k = 32,
 // 4 float fields) the apply took 0.211 ms against 0.142 ms for the same
-// targets given in Morton order, and 0.163 ms staged.
+// targets given in Hilbert order, and 0.163 ms staged.
 template <typename X, int NF>
 __global__ void __launch_bounds__( kBlock )
     records_to_caller_kernel( Pack<X, NF> const *__restrict__ rec,
@@ -231,7 +231,7 @@ void apply_pass( RowLayout const &g, C const *coeffs, X const *x,
 inline std::size_t align256( std::size_t b ) { return ( b + 255 ) & ~std::size_t( 255 ); }
 
 // The apply's two scratch arrays: the position-ordered gathered fields
-// (n_src records of the widest pass) and, when rows are in Morton order,
+// (n_src records of the widest pass) and, when rows are in Hilbert order,
 // the row results staged before they move to the targets.
 template <typename X, typename XS>
 void apply_scratch_sizes( RowLayout const &g, int n_fields, std::size_t &xs_bytes,
@@ -257,7 +257,7 @@ void launch_apply( RowLayout const &g, C const *coeffs, X const *x,
     DeviceBuffer<char> owned( ws ? 0 : xs_bytes + ys_bytes, s );
     char *const base = ws ? static_cast<char *>( ws ) : owned.get();
     XS *const scratch = reinterpret_cast<XS *>( base );
-    // rows in Morton order: results staged by row, then moved to targets
+    // rows in Hilbert order: results staged by row, then moved to targets
     X *const yscratch =
         ys_bytes ? reinterpret_cast<X *>( base + xs_bytes ) : nullptr;
     for ( int f0 = 0; f0 < n_fields; )
@@ -737,7 +737,7 @@ void crs_apply_transpose_f64( RowLayout const &g, CscIndex const &csc,
         (std::size_t)std::max<int64_t>( g.n_tgt, 1 ) *
             pass_width( n_fields ),
         s );
-    // columns in Morton position order: results staged by position, then
+    // columns in curve position order: results staged by position, then
     // moved to sources
     bool const staged = g.perm && g.spos;
     DeviceBuffer<double> xscratch(

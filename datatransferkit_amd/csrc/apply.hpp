@@ -10,8 +10,8 @@
 //            c(e) ybar[f][row(e)]; gathered through a column index (CSC)
 //            built once, so no atomics and a fixed order.
 //
-// Row layout. Rows are stored in the spatial (Morton) order of the targets
-// and column indices name source *positions* in the Morton order of the
+// Row layout. Rows are stored in the spatial (Hilbert curve) order of the targets
+// and column indices name source *positions* in the Hilbert order of the
 // sources: row r belongs to target order[r], position p is source perm[p].
 // Neighbouring rows then gather from neighbouring positions, so one pass
 // over the rows reads the values nearly sequentially. An apply first

@@ -76,8 +76,8 @@ struct dtkx_mls
     int64_t n_src = 0, n_tgt = 0;
     int m = 0, kk = 0;
     hipStream_t stream = nullptr;
-    // CRS rows in the Morton order of the targets (row r: target order[r],
-    // trow the inverse), columns as Morton positions of the sources
+    // CRS rows in the Hilbert order of the targets (row r: target order[r],
+    // trow the inverse), columns as curve positions of the sources
     // (position p: source perm[p]); empty buffers mean caller order
     dtkx::DeviceBuffer<int32_t> indices, order, trow, perm, spos;
     // create only: each row's largest neighbour distance (FP32 bulk)
@@ -1105,7 +1105,7 @@ struct dtkx_spline
     // order, as dtkx_spline_get_basis returns them
     dtkx::DeviceBuffer<int32_t> nbr;
     dtkx::DeviceBuffer<double> phi;
-    // the system the solver runs on: sources renumbered by Morton position
+    // the system the solver runs on: sources renumbered by curve position
     dtkx::DeviceBuffer<int32_t> perm; // position -> source
     dtkx::DeviceBuffer<int32_t> m_idx_p, n_idx_p;
     dtkx::DeviceBuffer<double> m_phi_p;
@@ -1236,7 +1236,7 @@ int dtkx_spline_create( const double *src_xyz, int64_t n_src,
         dtkx::spline_basis_weights( h->pts_d.get(), h->pts_d.get(), n_all, kk,
                                     h->nbr.get(), o.rbf, o.geometry,
                                     h->phi.get(), s );
-        // the solver's system: sources in Morton position order
+        // the solver's system: sources in curve position order
         h->m_idx_p.resize( (size_t)n_src * kk, s );
         h->m_phi_p.resize( (size_t)n_src * kk, s );
         h->n_idx_p.resize( (size_t)n_tgt * kk, s );
@@ -1459,7 +1459,7 @@ struct dtkx_mls_batch
     hipStream_t stream = nullptr;
     int64_t n_src = 0, n_tgt = 0, nnz = 0;
     std::vector<int64_t> tgt_count; // per problem
-    // concatenated problems: offsets, problem ids, Morton layout, CSR rows
+    // concatenated problems: offsets, problem ids, curve layout, CSR rows
     dtkx::DeviceBuffer<int32_t> src_off, tgt_off, src_prob, tgt_prob;
     dtkx::DeviceBuffer<int32_t> order, perm, pos, indices;
     dtkx::DeviceBuffer<int64_t> row_off;
@@ -1538,16 +1538,6 @@ struct dtkx_mls_batch
 
 namespace
 {
-
-// the K of the query kernel that holds up to k results
-int query_bucket( int k )
-{
-    int const ks[] = {1, 4, 8, 10, 16, 24, 32, 48, 64};
-    for ( int v : ks )
-        if ( k <= v )
-            return v;
-    return 64;
-}
 
 // Lanes per system of the classical solver for rows [r0, r1): the fastest
 // of the candidates on a sample of the rows (every candidate gives the same
@@ -1781,7 +1771,7 @@ int dtkx_mls_batch_create( int32_t n_problems, const dtkx_mls_problem *problems,
         std::stable_sort( rank.begin(), rank.end(), [&]( int a, int c ) {
             if ( m[a] != m[c] )
                 return m[a] < m[c];
-            return query_bucket( kk[a] ) < query_bucket( kk[c] );
+            return dtkx::knn_bucket( kk[a] ) < dtkx::knn_bucket( kk[c] );
         } );
         dtkx::KnnBatch &kb = b->kb;
         auto &groups = b->groups;
@@ -1793,11 +1783,11 @@ int dtkx_mls_batch_create( int32_t n_problems, const dtkx_mls_problem *problems,
             rstart[p] = static_cast<int32_t>( row );
             rbase[p] = nnz;
             int64_t const n = problems[p].n_tgt;
-            int const kb_p = query_bucket( kk[p] );
+            int const kb_p = dtkx::knn_bucket( kk[p] );
             if ( n > 0 )
             {
                 if ( !kb.launches.empty() && kb.launches.back().end == row &&
-                     query_bucket( kb.launches.back().kmax ) == kb_p )
+                     dtkx::knn_bucket( kb.launches.back().kmax ) == kb_p )
                 {
                     kb.launches.back().end = row + n;
                     kb.launches.back().kmax =

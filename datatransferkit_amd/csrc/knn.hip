@@ -1,31 +1,34 @@
-// LBVH k-nearest-neighbour search for gfx950.
+// k-nearest-neighbour search for gfx950.
 //
-// Build: scene box -> 63-bit Morton codes (21 bits per axis) with every
+// Build: scene box -> 63-bit Hilbert codes (21 bits per axis) with every
 // radix pass's digit counts -> the hand-written radix sort of (code, index)
-// (radix_sort.hpp; the targets' 30-bit codes sort in the same launches, and
+// (radix_sort.hpp; the targets' 48-bit codes sort in the same launches, and
 // the last pass writes both inverse permutations and the points in sorted
-// order) -> Karras hierarchy (duplicate codes split by index), in which each
-// internal node also writes both child boxes: exact for small children, the
-// Morton cell of the child's common prefix for large ones (a conservative
-// box needs no bottom-up pass, whose device-scope fences are costly across
-// the XCDs' separate L2 caches).
-// Query: one lane per target, targets processed in Morton order so a wave
-// walks a compact region; a per-lane stack in LDS; the k best candidates
-// stay sorted in registers as 64-bit keys (float distance bits << 32 |
-// index), so the ordering is (distance, index) with one integer compare.
-// Pruning uses squared distances against a threshold slightly above the
-// square of the current k-th distance, which never drops a candidate that
-// could tie or beat it; the kept set is therefore exactly the k smallest
-// (distance, index) pairs, as brute force gives. For larger k (and double
-// coordinates, whose key comparisons cost more) the list is replaced by two
-// traversals: the exact k-th squared distance from a list of distances
-// alone (one median-of-three per slot), then a fixed-radius pass that
-// collects the row, sorted at the end by (distance, index).
+// order) -> the boxes of 8, 64, 512, ... consecutive sources.
+// Query: groups of targets that are consecutive on the curve (knn_group.hpp).
+// The exact k smallest (distance, index) pairs of each target, as brute force
+// gives. 1M x 1M uniform points, build and query: k = 32 0.94 ms, k = 10
+// 0.72 ms, k = 1 0.65 ms (one tree traversal a lane over the hierarchy below
+// took 2.14, 1.00 and 0.64).
+//
+// The rows that the groups leave, and searches with fewer than 64 sources,
+// go to a tree search: a Karras hierarchy over the sorted codes (duplicate
+// codes split by index), in which each internal node also writes both child
+// boxes: exact for small children, the curve cell of the child's common
+// prefix for large ones (a conservative box needs no bottom-up pass). One
+// lane per target; a per-lane stack in LDS, or in global memory; the k best
+// candidates stay sorted in registers as 64-bit keys (float distance bits
+// << 32 | index), so the ordering is (distance, index) with one integer
+// compare. Pruning uses squared distances against a threshold slightly above
+// the square of the current k-th distance, which never drops a candidate
+// that could tie or beat it.
 #include "knn.hpp"
 #include "radix_sort.hpp"
 
 
+#include <algorithm>
 #include <cfloat>
+#include <cmath>
 #include <cstring>
 #include <vector>
 
@@ -138,7 +141,8 @@ __global__ void __launch_bounds__( kBlock )
             box[d] = sh[d][0];
 }
 
-// ---------------------------------------------------------- Morton codes
+// ----------------------------------------------------------- curve codes
+// Bits 0..20 of v spread to every third bit.
 __device__ inline uint64_t expand21( uint32_t v )
 {
     uint64_t x = v & 0x1fffffu;
@@ -150,42 +154,99 @@ __device__ inline uint64_t expand21( uint32_t v )
     return x;
 }
 
-// 63-bit Morton code of p (21 bits per axis) in the scene box
-// box[0..2] = lower corner, box[3..5] = upper corner.
-template <typename T, typename V>
-__device__ inline uint64_t morton63( V p, T const *box )
+// The 2^21 grid of a scene box (box[0..2] = lower corner, box[3..5] = upper
+// corner): cell = (p - lo) scale. One division an axis and box, not a point.
+struct CurveFrame
 {
-    double c[3] = {(double)p.x, (double)p.y, (double)p.z};
-    uint32_t q[3];
+    double lo[3], scale[3];
+};
+template <typename T>
+__device__ inline CurveFrame curve_frame( T const *box )
+{
+    CurveFrame f;
     for ( int d = 0; d < 3; ++d )
     {
-        double lo = box[d], ext = (double)box[3 + d] - lo;
-        double u = ext > 0 ? ( c[d] - lo ) / ext * 2097151.0 : 0.0;
+        f.lo[d] = box[d];
+        double const ext = (double)box[3 + d] - f.lo[d];
+        f.scale[d] = ext > 0 ? 2097151.0 / ext : 0.0;
+    }
+    return f;
+}
+
+// Cell of p on the grid of f.
+template <typename V>
+__device__ inline void curve_cell( V p, CurveFrame const &f, uint32_t *q )
+{
+    double const c[3] = {(double)p.x, (double)p.y, (double)p.z};
+    for ( int d = 0; d < 3; ++d )
+    {
+        double u = ( c[d] - f.lo[d] ) * f.scale[d];
         u = u < 0 ? 0 : ( u > 2097151.0 ? 2097151.0 : u );
         q[d] = (uint32_t)u;
     }
-    return ( expand21( q[0] ) << 2 ) | ( expand21( q[1] ) << 1 ) |
-           expand21( q[2] );
+}
+
+// Place on the Hilbert curve of the cell q of a 2^BITS grid (3 BITS bits),
+// by Skilling's transform (AIP Conf. Proc. 707, 2004): from the top bit
+// down, an axis' bit inverts or exchanges the lower bits of the first axis;
+// then a Gray decode across the axes. The code of q >> s is the code of q
+// without its last 3 s bits, so a prefix of 3 L bits names an octree cell,
+// one further bit a half and two a quarter of one. Consecutive cells share
+// a face: a run of consecutive points, unlike one in Hilbert order, never
+// jumps, and its box stays small (the sources within the k-th distance of
+// 16 consecutive targets number 223 against 360, the 8-point blocks they
+// lie in 55 against 102: uniform points, k = 32).
+template <int BITS>
+__device__ inline uint64_t hilbert_code( uint32_t const *q )
+{
+    uint32_t x = q[0], y = q[1], z = q[2];
+#pragma unroll
+    for ( int b = BITS - 1; b >= 1; --b )
+    {
+        uint32_t const Q = 1u << b, P = Q - 1u;
+        x ^= x & Q ? P : 0u;
+        uint32_t const ty = ( x ^ y ) & P;
+        uint32_t const iy = y & Q ? P : ty;
+        y ^= y & Q ? 0u : ty;
+        x ^= iy;
+        uint32_t const tz = ( x ^ z ) & P;
+        uint32_t const iz = z & Q ? P : tz;
+        z ^= z & Q ? 0u : tz;
+        x ^= iz;
+    }
+    y ^= x;
+    z ^= y;
+    uint32_t t = z >> 1;
+    t ^= t >> 1;
+    t ^= t >> 2;
+    t ^= t >> 4;
+    t ^= t >> 8;
+    t ^= t >> 16;
+    return ( expand21( x ^ t ) << 2 ) | ( expand21( y ^ t ) << 1 ) |
+           expand21( z ^ t );
 }
 
 // Radix passes of the two key kinds: the sources' 63-bit codes and the
-// targets' top 30 bits.
-constexpr int kSrcKeyBits = 63, kTgtKeyBits = 30;
+// targets' top 48 bits (a cell of 1.5e-5 of the scene: a group of targets
+// must be close together in terms of the sources around it. With 30 bits,
+// cells of 1e-3, the targets inside a cluster of that size were in no order,
+// and half of the rows of 1M points in 200 such clusters were left over).
+constexpr int kSrcKeyBits = 63, kTgtLevels = 16, kTgtKeyBits = 3 * kTgtLevels;
 constexpr int kSrcPasses = ( kSrcKeyBits + 7 ) / 8;
 constexpr int kTgtPasses = ( kTgtKeyBits + 7 ) / 8;
 constexpr int kHistWords = ( kSrcPasses + kTgtPasses ) * rsort::kDigits;
 
-// Morton codes of the sources (63-bit) and of the targets (top 30 bits) in
+// Hilbert codes of the sources (63-bit) and of the targets (top 30 bits) in
 // one launch, one sort tile of points a block (blocks [0, src_blocks) take
 // the sources), with the digit counts of every radix pass added into hist
 // (sources' passes first, zero on entry). src_prob / tgt_prob (nullable, a batch):
 // each point's problem, whose scene box is box + 6 problem.
 template <typename T, typename V>
 __global__ void __launch_bounds__( rsort::kThreads )
-    morton_hist_kernel( V const *src, int64_t n_src, V const *tgt,
+    curve_hist_kernel( V const *src, int64_t n_src, V const *tgt,
                         int64_t n_tgt, T const *box, int32_t const *src_prob,
                         int32_t const *tgt_prob, int src_blocks,
-                        uint64_t *scodes, uint32_t *tcodes, uint32_t *hist )
+                        uint64_t *scodes, uint64_t *tcodes, uint32_t *hist )
 {
     __shared__ uint32_t h[kSrcPasses * rsort::kDigits];
     bool const is_src = static_cast<int>( blockIdx.x ) < src_blocks;
@@ -199,15 +260,19 @@ __global__ void __launch_bounds__( rsort::kThreads )
     int64_t const n = is_src ? n_src : n_tgt;
     V const *pts = is_src ? src : tgt;
     int32_t const *prob = is_src ? src_prob : tgt_prob;
+    CurveFrame frame = curve_frame( box );
     for ( int s = 0; s < rsort::kItems; ++s )
     {
         int64_t const i = c0 + s * rsort::kThreads + threadIdx.x;
         if ( i >= n )
             break;
-        uint64_t const code =
-            morton63<T, V>( pts[i], prob ? box + 6 * prob[i] : box );
+        if ( prob )
+            frame = curve_frame( box + 6 * prob[i] );
+        uint32_t q[3];
+        curve_cell( pts[i], frame, q );
         if ( is_src )
         {
+            uint64_t const code = hilbert_code<21>( q );
             scodes[i] = code;
 #pragma unroll
             for ( int p = 0; p < kSrcPasses; ++p )
@@ -216,7 +281,10 @@ __global__ void __launch_bounds__( rsort::kThreads )
         }
         else
         {
-            uint32_t const c = static_cast<uint32_t>( code >> 33 );
+            // the top bits of the full code
+            constexpr int kCut = 21 - kTgtLevels;
+            uint32_t const cut[3] = {q[0] >> kCut, q[1] >> kCut, q[2] >> kCut};
+            uint64_t const c = hilbert_code<kTgtLevels>( cut );
             tcodes[i] = c;
 #pragma unroll
             for ( int p = 0; p < kTgtPasses; ++p )
@@ -248,46 +316,45 @@ __device__ inline int prefix_delta( uint64_t const *codes, int64_t n,
     return 64 + __clz( (uint32_t)i ^ (uint32_t)j );
 }
 
-__device__ inline uint32_t compact21( uint64_t x )
-{
-    x &= 0x1249249249249249ull;
-    x = ( x | x >> 2 ) & 0x10c30c30c30c30c3ull;
-    x = ( x | x >> 4 ) & 0x100f00f00f00f00full;
-    x = ( x | x >> 8 ) & 0x1f0000ff0000ffull;
-    x = ( x | x >> 16 ) & 0x1f00000000ffffull;
-    x = ( x | x >> 32 ) & 0x1fffffull;
-    return (uint32_t)x;
-}
-
 __device__ inline float round_down( double v ) { return __double2float_rd( v ); }
 __device__ inline float round_up( double v ) { return __double2float_ru( v ); }
-__device__ inline double round_down_d( double v ) { return v; }
 
-// Conservative box of every point whose Morton code shares the first
-// `delta` bits of `code` (bit 63 is always 0): the quantisation cell of the
-// prefix, mapped back to world coordinates with a margin and outward
-// rounding, so it contains the points whatever the rounding of the forward
-// quantisation (morton63).
+// Conservative box of the points between two points of the curve order
+// whose cells are qb and qe (qm: a point between them) and whose codes share
+// the first `delta` bits (bit 63 is always 0): the octree cell of the
+// prefix's whole digits, cut to the two octants that it then holds when the
+// prefix ends two bits into a digit (those of qb and qe), and to their half
+// of the cell when it ends one bit in and the three points show two of the
+// half's axes. (The curve enters and leaves a half through octants that
+// differ in one axis only, so its middle names the other.) Mapped back to
+// world coordinates with a margin and outward rounding, so it contains the
+// points whatever the rounding of the forward quantisation (curve_cell).
 template <typename T>
-__device__ inline void cell_box( uint64_t code, int delta, T const *scene,
+__device__ inline void cell_box( uint32_t const *qb, uint32_t const *qm,
+                                 uint32_t const *qe, int delta, T const *scene,
                                  T *lo, T *hi )
 {
     int const nb = delta >= 64 ? 63 : ( delta - 1 ); // known bits below 63
-    uint64_t const all = ( 1ull << 63 ) - 1;
-    uint64_t const mask = nb <= 0 ? 0ull : ( all & ~( ( 1ull << ( 63 - nb ) ) - 1 ) );
-    uint64_t const pmin = code & mask;
-    uint64_t const pmax = ( code & mask ) | ( all & ~mask );
-    uint32_t const qmin[3] = {compact21( pmin >> 2 ), compact21( pmin >> 1 ),
-                              compact21( pmin )};
-    uint32_t const qmax[3] = {compact21( pmax >> 2 ), compact21( pmax >> 1 ),
-                              compact21( pmax )};
+    int const digits = nb > 0 ? nb / 3 : 0, part = nb > 0 ? nb % 3 : 0;
+    int const sh = 21 - digits;
+    uint32_t diff[3];
+    int n_diff = 0;
     for ( int d = 0; d < 3; ++d )
     {
+        uint32_t const x = ( qb[d] ^ qe[d] ) | ( qb[d] ^ qm[d] );
+        diff[d] = part ? ( x >> ( sh - 1 ) ) & 1u : 1u;
+        n_diff += (int)diff[d];
+    }
+    bool const cut = part == 2 || ( part == 1 && n_diff == 2 );
+    for ( int d = 0; d < 3; ++d )
+    {
+        int const s = cut && !diff[d] ? sh - 1 : sh;
+        uint32_t const qmin = ( qb[d] >> s ) << s;
         double const s0 = scene[d], ext = (double)scene[3 + d] - s0;
         double const h = ext / 2097151.0;
         double const margin = 1e-9 * ext + 1e-300;
-        double l = s0 + qmin[d] * h - margin;
-        double u = s0 + ( qmax[d] + 1.0 ) * h + margin;
+        double l = s0 + qmin * h - margin;
+        double u = s0 + ( (double)qmin + (double)( 1u << s ) ) * h + margin;
         if ( sizeof( T ) == 4 )
         {
             lo[d] = (T)round_down( l );
@@ -304,10 +371,7 @@ __device__ inline void cell_box( uint64_t code, int delta, T const *scene,
 // Children of internal node i: ranges, codes, parents and child boxes.
 // A child that is a leaf gets its point as a degenerate box and the code
 // ~source_index; an internal child covering at most kTight points gets its
-// exact box, a larger one the Morton cell of its common prefix. Query at
-// 1M x 1M for kTight 8 / 16 / 32: k = 32 2.11 / 2.08 / 2.07 ms, k = 16
-// 1.03 / 1.01 / 1.00, 1M clustered (k = 32) 2.06 / 2.03 / 2.21 (the build
-// takes longer at 32).
+// exact box, a larger one the curve cell of its common prefix.
 #ifndef DTKX_KNN_TIGHT
 #define DTKX_KNN_TIGHT 16
 #endif
@@ -332,7 +396,8 @@ __device__ inline int node_problem( int32_t const *src_off, int n_prob,
 }
 
 // One problem (src_off null): n points, internal nodes [0, n - 1).
-// Batch: n_int internal nodes in all; node i belongs to problem p, whose
+// wanted (nullable): nothing is built when it is 0 (no query is left to the
+// hierarchy). Batch: n_int internal nodes in all; node i belongs to problem p, whose
 // sorted points are [src_off[p], src_off[p + 1]) with scene box scene + 6 p;
 // the hierarchy of each problem is built over its own range (child node
 // indices and leaf codes are global).
@@ -341,8 +406,10 @@ __global__ void __launch_bounds__( kBlock )
     karras_kernel( uint64_t const *codes_all, int32_t const *sorted_all,
                    V const *pts, V const *sorted_pts_all, int64_t n_int,
                    T const *scenes, int32_t const *src_off, int n_prob,
-                   Node<T> *nodes, int32_t *sizes )
+                   Node<T> *nodes, int32_t *sizes, int32_t const *wanted )
 {
+    if ( wanted && *wanted == 0 )
+        return;
     int64_t const gi = blockIdx.x * (int64_t)kBlock + threadIdx.x;
     if ( gi >= n_int )
         return;
@@ -427,8 +494,15 @@ __global__ void __launch_bounds__( kBlock )
             }
         }
         else
-            cell_box<T>( codes[b], prefix_delta( codes, n, b, e ), scene,
+        {
+            CurveFrame const frame = curve_frame( scene );
+            uint32_t qb[3], qm[3], qe[3];
+            curve_cell( point( b ), frame, qb );
+            curve_cell( point( ( b + e ) / 2 ), frame, qm );
+            curve_cell( point( e ), frame, qe );
+            cell_box<T>( qb, qm, qe, prefix_delta( codes, n, b, e ), scene,
                          nd.lo[c], nd.hi[c] );
+        }
     }
     nodes[gi] = nd;
 }
@@ -649,86 +723,29 @@ __device__ inline double sqrt_rn( double s ) { return __builtin_sqrt( s ); }
 
 constexpr int kQueryBlock = 64;
 
-// Seed the two-pass search's k-th distance from the deepest node on the
-// query's path holding k sources.
+// Seed the k-th distance from the deepest node on the query's path holding
+// k sources.
 #ifndef DTKX_KNN_SEED
 #define DTKX_KNN_SEED 1
 #endif
 constexpr bool kSeed = DTKX_KNN_SEED != 0;
 
-// Queries run with an LDS stack of kLdsStack entries; the rare one whose
-// descent needs more is re-run with a global stack of kMaxDepth entries.
-// The LDS stack bounds the occupancy (8 bytes per entry and lane). With
-// the seeded k-th distance (seed_far_sq) a descent pushes only far
-// children inside the seed's bound, so shallow stacks suffice: 22 entries
-// (14 waves per CU) against 24 at 1M x 1M: k = 32 2.11 / 2.12 ms, k = 16
-// 1.03 / 1.13, k = 10 0.73 / 0.81; 20 entries (with an 8-entry second
-// pass) 13 % slower at k = 32, and 82 clustered queries overflow. Before
-// seeding, 24 entries were needed, and 40 % of the queries of 1M points in
-// 200 Gaussian clusters (sigma 1e-3) overflowed them; none do now.
+// Queries run with an LDS stack of kLdsStack entries (14 waves per CU); the
+// rare one whose descent needs more is re-run with a global stack of
+// kMaxDepth entries. With the seeded k-th distance (seed_far_sq) a descent
+// pushes only far children inside the seed's bound, so shallow stacks
+// suffice.
 // Every level of the hierarchy lengthens the common prefix of the node's
-// keys (63 Morton bits, then 32 index bits for equal codes), so no path
+// keys (63 curve bits, then 32 index bits for equal codes), so no path
 // from the root has more than 96 internal levels.
 #ifndef DTKX_KNN_LDS_STACK
 #define DTKX_KNN_LDS_STACK 22
 #endif
 constexpr int kLdsStack = DTKX_KNN_LDS_STACK;
-// The one-pass search (K below two_pass_k) keeps no row in its stack's
-// slots, so its stack could be shorter: 16 entries took 0.63 ms against
-// 0.72 at k = 10 and 0.90 against 1.00 at k = 16 (1M x 1M uniform), but on
-// 1M points in 200 clusters (sigma 1e-3) 15 and 65 queries overflowed and
-// their re-run's serial tail made the search 0.86 against 0.73 and 1.23
-// against 0.98 ms; 22 overflows none there.
-#ifndef DTKX_KNN_LDS_STACK1
-#define DTKX_KNN_LDS_STACK1 22
-#endif
-constexpr int kLdsStack1 = DTKX_KNN_LDS_STACK1;
-// stack entries of the fixed-radius pass of a two-pass search when its row
-// is collected in the LDS stack's other slots (its radius is final, so it
-// descends far less deep than the first pass); the row needs
-// K <= 2 kLdsStack - kPass2Stack slots for float coordinates
-#ifndef DTKX_KNN_PASS2_STACK
-#define DTKX_KNN_PASS2_STACK 12
-#endif
-constexpr int kPass2Stack = DTKX_KNN_PASS2_STACK;
 constexpr int kMaxDepth = 97;
-// the largest K whose two-pass rows are sorted inside the traversal kernel
-#ifndef DTKX_KNN_FUSED_SORT_K
-#define DTKX_KNN_FUSED_SORT_K 32
-#endif
-constexpr int kFusedSortK = DTKX_KNN_FUSED_SORT_K;
-// collect the rows of K > kFusedSortK in LDS too (an extra array beside
-// the dead stack slots), written out in one burst per row. Off: the extra
-// LDS costs more occupancy than the scattered row stores cost traffic
-// (1M x 1M query, k = 64: 5.30 against 4.09 ms; k = 48: 3.83 against 3.22).
-#ifndef DTKX_KNN_BIG_ROW_LDS
-#define DTKX_KNN_BIG_ROW_LDS 0
-#endif
-constexpr bool kBigRowLds = DTKX_KNN_BIG_ROW_LDS != 0;
-
-// launch mode of the separate row sort
-constexpr int kSortRows = -1;
-// The smallest K searched in two passes. Measured for 1M uniform sources
-// and targets with the 24-entry LDS stack: with float coordinates one pass
-// is faster up to k = 24 (1.35 against 1.67 ms at k = 16, 1.93 against
-// 2.09 ms at k = 24) and two passes from k = 32 (2.53 against 2.68 ms);
-// with double coordinates, whose (distance, index) comparisons cost three
-// operations, two passes win from k = 16 (with the 32-entry stack: 3.2
-// against 4.2 ms at k = 16, 5.1 against 11.9 ms at k = 32). With the
-// seeded k-th distance and the 22-entry stack the crossover is unchanged:
-// one pass 1.54 against 1.75 ms at k = 24, two passes 2.12 against 2.21 ms
-// at k = 32.
-#ifndef DTKX_KNN_TWO_PASS_KF
-#define DTKX_KNN_TWO_PASS_KF 32
-#endif
-template <typename T>
-constexpr int two_pass_k()
-{
-    return sizeof( T ) == 4 ? DTKX_KNN_TWO_PASS_KF : 16;
-}
 
 // Arguments of a query launch. One problem: rows [row0, row0 + n_rows) of
-// the Morton-ordered targets against n_src sources, kk results per row.
+// the Hilbert-ordered targets against n_src sources, kk results per row.
 // Batch (src_off set): target t belongs to problem tgt_prob[t], whose
 // sources are [src_off[p], src_off[p + 1]), whose hierarchy is rooted at
 // internal node src_off[p] - p and whose rows hold kk_prob[p] results at
@@ -749,7 +766,7 @@ struct QueryArgs
     int64_t const *row_off = nullptr;
     int32_t *out_idx = nullptr;
     double *out_dist = nullptr;
-    // Morton layout: row r written at row r with indices as positions
+    // curve layout: row r written at row r with indices as positions
     int32_t const *src_pos = nullptr;
     // nullable: row r's largest neighbour distance, written at row r
     float *row_max = nullptr;
@@ -768,7 +785,7 @@ struct QueryArgs
     int64_t gstride = 0;
 };
 
-// One row of a one-pass search: lane qi (its global-stack slot), row r;
+// One row of the tree search: lane qi (its global-stack slot), row r;
 // st_node and st_d are the block's LDS stack. STACK > 0: an LDS stack of
 // that many entries per lane (a query that would need more is listed for
 // the re-run); STACK == 0: a per-lane stack in global memory (gstack, laid
@@ -916,93 +933,23 @@ __global__ void __launch_bounds__( kQueryBlock )
     __shared__ T st_d[LS * kQueryBlock];
     int64_t const qi = xcd_tile<0>() * kQueryBlock + threadIdx.x;
     if constexpr ( STACK == 0 )
-        if ( a.rows )
-        {
-            // re-run of listed rows: the grid's n_rows lanes stride over
-            // the list, whose length only the device knows
-            int64_t const n = *a.n_rows_dev;
-            if ( a.n_rows_total && qi == 0 )
-                atomicAdd( a.n_rows_total, (int32_t)n );
-            for ( int64_t i = qi; i < n; i += a.n_rows )
-                query_row<T, K, STACK>( a, qi, a.rows[i], st_node, st_d );
-            return;
-        }
+    {
+        // listed rows: the grid's n_rows lanes stride over the list, whose
+        // length only the device knows
+        int64_t const n = *a.n_rows_dev;
+        if ( a.n_rows_total && qi == 0 )
+            atomicAdd( a.n_rows_total, (int32_t)n );
+        for ( int64_t i = qi; i < n; i += a.n_rows )
+            query_row<T, K, STACK>( a, qi, a.rows[i], st_node, st_d );
+        return;
+    }
     // LDS-stack launches run rows [row0, row0 + n_rows), one per lane
     if ( qi >= a.n_rows )
         return;
     query_row<T, K, STACK>( a, qi, a.row0 + qi, st_node, st_d );
 }
 
-// ------------------------------------------------- two-pass k-best search
-// For larger k the sorted (distance, index) list costs five operations per
-// slot for every candidate, and a wave runs it whenever any of its lanes
-// meets one. Two traversals do the same work with fewer operations:
-// pass 1 keeps only the k smallest SQUARED distances, a sorted register
-// array updated with one median-of-three per slot; its last entry s_k gives
-// the k-th distance d_k = sqrt(s_k) (a correctly rounded square root is
-// monotone, so it maps order statistics to order statistics). Exactly the
-// pass-1 entries whose root is below d_k are sources at distance < d_k, say
-// c_lt of them. Pass 2 is a fixed-radius traversal that writes those c_lt
-// sources and the k - c_lt smallest indices among the sources at distance
-// == d_k to the row; the row is then sorted by (distance, index) in
-// registers. The result is the set and order the sorted list gives.
-template <typename T>
-__device__ inline T med3( T a, T b, T c );
-template <>
-__device__ inline float med3( float a, float b, float c )
-{
-    return __builtin_amdgcn_fmed3f( a, b, c );
-}
-template <>
-__device__ inline double med3( double a, double b, double c )
-{
-    return fmin( c, fmax( a, b ) ); // a <= c
-}
-
-// The k smallest squared distances, ascending. Slots below K - kk hold -1,
-// so the last slot is the kk-th smallest for any kk <= K.
-template <typename T, int K>
-struct KthList
-{
-    T d[K];
-    __device__ void init( int kk )
-    {
-#pragma unroll
-        for ( int j = 0; j < K; ++j )
-            d[j] = j < K - kk ? T( -1 ) : T( INFINITY );
-    }
-    // new d[j] = clamp(s, d[j - 1], d[j]): the j-th of the sorted union
-    __device__ void insert( T s )
-    {
-#pragma unroll
-        for ( int j = K - 1; j > 0; --j )
-            d[j] = med3( d[j - 1], s, d[j] );
-        d[0] = fmin( d[0], s );
-    }
-    __device__ T last() const { return d[K - 1]; }
-    // kk entries of value b (padding stays -1): b acts as kk candidates
-    // at squared distance b, so the list ends at the true kk-th value
-    // whenever at least kk sources lie at or below b
-    __device__ void seed( int kk, T b )
-    {
-#pragma unroll
-        for ( int j = 0; j < K; ++j )
-            if ( j >= K - kk )
-                d[j] = b;
-    }
-};
-
-// A squared-distance bound above every s whose rounded root is <= w.
-__device__ inline float root_bound( float w )
-{
-    return w * w * 1.00000095367431640625f; // (1 + 2^-20)
-}
-__device__ inline double root_bound( double w )
-{
-    return w * w * 1.0000000000000009; // (1 + 2^-50)
-}
-
-// (distance, index) keys of the final sort
+// (distance, index) keys
 template <typename T>
 struct SortKey;
 template <>
@@ -1040,406 +987,7 @@ struct SortKey<double>
     __device__ static double distance( type a ) { return a.d; }
 };
 
-constexpr int pow2_at_least( int k )
-{
-    int n = 1;
-    while ( n < k )
-        n <<= 1;
-    return n;
-}
-
-// ascending bitonic sorting network, all indices compile-time constants
-template <typename T, int N>
-__device__ inline void bitonic_sort( typename SortKey<T>::type ( &a )[N] )
-{
-    using SK = SortKey<T>;
-#pragma unroll
-    for ( int k = 2; k <= N; k <<= 1 )
-#pragma unroll
-        for ( int j = k >> 1; j > 0; j >>= 1 )
-#pragma unroll
-            for ( int i = 0; i < N; ++i )
-            {
-                int const l = i ^ j;
-                if ( l > i )
-                {
-                    bool const up = ( i & k ) == 0;
-                    auto const x = a[i], y = a[l];
-                    bool const swap = up ? SK::less( y, x ) : SK::less( x, y );
-                    a[i] = swap ? y : x;
-                    a[l] = swap ? x : y;
-                }
-            }
-}
-
-// A two-pass row (its unordered indices read through get(j)) sorted by
-// (distance, index) into row, distances recomputed exactly as the
-// traversals computed them, indices then mapped to positions for the Morton
-// layout. (Fused: the LDS stack, not the network's registers, limits the
-// kernel's occupancy.)
-template <typename T, int K, typename Get>
-__device__ inline void sort_row( QueryArgs<T> const &a, T const *q,
-                                 int64_t r, int64_t base, int kk,
-                                 int32_t *row, Get const &get )
-{
-    using SK = SortKey<T>;
-    constexpr int N = pow2_at_least( K );
-    typename SK::type key[N];
-#pragma unroll
-    for ( int j = 0; j < N; ++j )
-    {
-        key[j] = SK::none();
-        if ( j < kk )
-        {
-            int32_t const id = get( j );
-            typename Vec4<T>::type const p = a.src[id];
-            T const b[3] = {p.x, p.y, p.z};
-            key[j] = SK::make( sqrt_rn( box_sq( q, b, b ) ), id );
-        }
-    }
-    bitonic_sort<T, N>( key );
-#pragma unroll
-    for ( int j = 0; j < K; ++j )
-        if ( j < kk )
-        {
-            int32_t const id = SK::index( key[j] );
-            row[j] = a.src_pos ? a.src_pos[id] : id;
-            if ( a.out_dist )
-                a.out_dist[base + j] = SK::distance( key[j] );
-            if ( a.row_max && j == kk - 1 )
-                a.row_max[r] = (float)SK::distance( key[j] );
-        }
-}
-
-// One row of a two-pass search: lane qi (its global-stack slot), row r;
-// st_node and st_d are the block's LDS stack.
-template <typename T, int K, int STACK>
-__device__ inline void query2_row( QueryArgs<T> const &a, int64_t const qi,
-                                  int64_t const r, int32_t *st_node, T *st_d )
-{
-    using SK = SortKey<T>;
-    int32_t const t = a.order[r];
-    int64_t so = 0, np = a.n_src;
-    int32_t root = 0;
-    int kk = a.kk;
-    if ( a.src_off )
-    {
-        int const pb = a.tgt_prob[t];
-        so = a.src_off[pb];
-        np = a.src_off[pb + 1] - so;
-        root = (int32_t)( so - pb );
-        kk = a.kk_prob[pb];
-    }
-    typename Vec4<T>::type qp = a.tgt[t];
-    T const q[3] = {qp.x, qp.y, qp.z};
-    int64_t const base =
-        a.row_off ? a.row_off[r] : ( a.src_pos ? r : (int64_t)t ) * kk;
-    int32_t *row = a.out_idx + base;
-
-    auto overflow = [&]() {
-        a.overflow_rows[atomicAdd( a.n_overflow, 1 )] = (int32_t)r;
-    };
-
-    // pass 1: the kk-th smallest squared distance
-    KthList<T, K> list;
-    list.init( kk );
-    if ( a.node_size && np > 1 )
-        // pruning starts at the seed, so the descent pushes no far child
-        // beyond it
-        list.seed( kk, root_bound( sqrt_rn(
-                           seed_far_sq( a.nodes, a.node_size, root, q, kk ) ) ) );
-    if ( np == 1 )
-    {
-        typename Vec4<T>::type sp0 = a.src[so];
-        T const b[3] = {sp0.x, sp0.y, sp0.z};
-        list.insert( box_sq( q, b, b ) );
-    }
-    else
-    {
-        T thr = list.last();
-        int sp = 0;
-        int32_t node = root;
-        while ( node >= 0 )
-        {
-            Node<T> const nd = a.nodes[node];
-            T const s0 = box_sq( q, nd.lo[0], nd.hi[0] );
-            T const s1 = box_sq( q, nd.lo[1], nd.hi[1] );
-            int32_t const c0 = nd.child[0], c1 = nd.child[1];
-            // an entry equal to the bound leaves the list's values unchanged
-            if ( c0 < 0 && s0 < thr )
-            {
-                list.insert( s0 );
-                thr = list.last();
-            }
-            if ( c1 < 0 && s1 < thr )
-            {
-                list.insert( s1 );
-                thr = list.last();
-            }
-            bool const g0 = c0 >= 0 && s0 < thr;
-            bool const g1 = c1 >= 0 && s1 < thr;
-            int32_t next = -1;
-            if ( g0 && g1 )
-            {
-                bool const near0 = s0 <= s1;
-                int32_t const far = near0 ? c1 : c0;
-                T const fs = near0 ? s1 : s0;
-                next = near0 ? c0 : c1;
-                if ( STACK > 0 )
-                {
-                    if ( sp == STACK )
-                    {
-                        overflow();
-                        return;
-                    }
-                    st_node[sp * kQueryBlock + threadIdx.x] = far;
-                    st_d[sp * kQueryBlock + threadIdx.x] = fs;
-                }
-                else
-                {
-                    int2 e;
-                    e.x = far;
-                    e.y = __float_as_int( (float)fs );
-                    a.gstack[sp * a.gstride + qi] = e;
-                }
-                ++sp;
-            }
-            else if ( g0 )
-                next = c0;
-            else if ( g1 )
-                next = c1;
-            else
-            {
-                while ( sp > 0 )
-                {
-                    --sp;
-                    int32_t cand;
-                    T cs;
-                    if ( STACK > 0 )
-                    {
-                        cand = st_node[sp * kQueryBlock + threadIdx.x];
-                        cs = st_d[sp * kQueryBlock + threadIdx.x];
-                    }
-                    else
-                    {
-                        int2 e = a.gstack[sp * a.gstride + qi];
-                        cand = e.x;
-                        // a rounded copy of a double bound only orders
-                        cs = sizeof( T ) == 4 ? (T)__int_as_float( e.y ) : 0;
-                    }
-                    if ( cs < thr )
-                    {
-                        next = cand;
-                        break;
-                    }
-                }
-            }
-            node = next;
-        }
-    }
-
-    // pass 2: the sources at distance < d_k, and the smallest indices among
-    // those at distance == d_k, written to the row unordered
-    T const dk = sqrt_rn( list.last() );
-    int c_lt = 0;
-#pragma unroll
-    for ( int j = 0; j < K; ++j )
-        c_lt += ( list.d[j] >= 0 && sqrt_rn( list.d[j] ) < dk ) ? 1 : 0;
-    T const s_hi = root_bound( dk );
-    // The row is collected in LDS when it fits beside pass 2's stack (whose
-    // pass-1 distances are dead): the stack keeps the first kPass2Stack node
-    // slots, the row takes the distance slots (as ints) and the node slots
-    // above. Scattered 4-byte stores to the row in global memory, spread
-    // over the traversal, would leave partly written lines for the L2 to
-    // evict (8 times the row's bytes, measured).
-    constexpr int kDistSlots = STACK * (int)( sizeof( T ) / 4 );
-    constexpr int kDeadSlots = kDistSlots + STACK - kPass2Stack;
-    // rows of K > kFusedSortK: the slots beyond the dead ones in an LDS
-    // array of their own, the row copied out at the end
-    constexpr bool kBigRow = kBigRowLds && STACK > kPass2Stack &&
-                             K > kFusedSortK;
-    constexpr bool kRowLds = STACK > kPass2Stack &&
-                             ( kBigRow || ( K <= kFusedSortK && K <= kDeadSlots ) );
-    constexpr int kExtra = kBigRow && K > kDeadSlots ? K - kDeadSlots : 1;
-    __shared__ int32_t st_extra[kBigRow ? kExtra * kQueryBlock : 1];
-    constexpr int kStack2 = kRowLds ? kPass2Stack : STACK;
-    int32_t *const ids_d = reinterpret_cast<int32_t *>( st_d );
-    auto slot = [&]( int j ) -> int32_t & {
-        if constexpr ( kRowLds )
-        {
-            if ( j < kDistSlots )
-                return ids_d[j * kQueryBlock + threadIdx.x];
-            if ( !kBigRow || j < kDeadSlots )
-                return st_node[( kPass2Stack + j - kDistSlots ) * kQueryBlock +
-                               threadIdx.x];
-            return st_extra[( j - kDeadSlots ) * kQueryBlock + threadIdx.x];
-        }
-        else
-            return row[j];
-    };
-    int n_lt = 0, n_eq = 0;
-    auto take = [&]( T s, int32_t id ) {
-        T const d = sqrt_rn( s );
-        if ( d < dk )
-        {
-            if ( n_lt < c_lt )
-                slot( n_lt++ ) = id;
-        }
-        else if ( d == dk )
-        {
-            if ( c_lt + n_eq < kk )
-                slot( c_lt + n_eq++ ) = id;
-            else
-            {
-                // all tie slots taken: replace the largest index if larger
-                int jm = c_lt;
-                for ( int j = c_lt + 1; j < kk; ++j )
-                    jm = slot( j ) > slot( jm ) ? j : jm;
-                if ( id < slot( jm ) )
-                    slot( jm ) = id;
-            }
-        }
-    };
-    if ( np == 1 )
-    {
-        typename Vec4<T>::type sp0 = a.src[so];
-        T const b[3] = {sp0.x, sp0.y, sp0.z};
-        take( box_sq( q, b, b ), (int32_t)so );
-    }
-    else
-    {
-        int sp = 0;
-        int32_t node = root;
-        while ( node >= 0 )
-        {
-            Node<T> const nd = a.nodes[node];
-            T const s0 = box_sq( q, nd.lo[0], nd.hi[0] );
-            T const s1 = box_sq( q, nd.lo[1], nd.hi[1] );
-            int32_t const c0 = nd.child[0], c1 = nd.child[1];
-            if ( c0 < 0 && s0 <= s_hi )
-                take( s0, ~c0 );
-            if ( c1 < 0 && s1 <= s_hi )
-                take( s1, ~c1 );
-            bool const g0 = c0 >= 0 && s0 <= s_hi;
-            bool const g1 = c1 >= 0 && s1 <= s_hi;
-            int32_t next = -1;
-            if ( g0 && g1 )
-            {
-                next = c0;
-                if ( STACK > 0 )
-                {
-                    if ( sp == kStack2 )
-                    {
-                        overflow();
-                        return;
-                    }
-                    st_node[sp * kQueryBlock + threadIdx.x] = c1;
-                }
-                else
-                    a.gstack[sp * a.gstride + qi].x = c1;
-                ++sp;
-            }
-            else if ( g0 )
-                next = c0;
-            else if ( g1 )
-                next = c1;
-            else if ( sp > 0 )
-            {
-                --sp;
-                next = STACK > 0 ? st_node[sp * kQueryBlock + threadIdx.x]
-                                 : a.gstack[sp * a.gstride + qi].x;
-            }
-            node = next;
-        }
-    }
-    if constexpr ( K <= kFusedSortK )
-        sort_row<T, K>( a, q, r, base, kk, row, slot );
-    else if constexpr ( kBigRow )
-        for ( int j = 0; j < kk; ++j )
-            row[j] = slot( j );
-}
-
-// Registers for four waves per SIMD (128): the float K = 32 kernel then
-// spills 52 bytes a lane, and its LDS stack admits 14 waves per CU against
-// the 12 that 135 registers allowed: 1.92 ms against 2.02 for the 1M x 1M,
-// k = 32 query. (Kernels whose LDS already allows fewer waves, the double
-// ones, keep their registers.)
-template <typename T, int K, int STACK>
-__global__ void __launch_bounds__( kQueryBlock )
-    __attribute__( ( amdgpu_waves_per_eu( 4 ) ) )
-    knn_query2_kernel( QueryArgs<T> const a )
-{
-    constexpr int LS = STACK > 0 ? STACK : 1;
-    __shared__ int32_t st_node[LS * kQueryBlock];
-    __shared__ T st_d[LS * kQueryBlock];
-    int64_t const qi = xcd_tile<0>() * kQueryBlock + threadIdx.x;
-    if constexpr ( STACK == 0 )
-        if ( a.rows )
-        {
-            // re-run of listed rows: the grid's n_rows lanes stride over
-            // the list, whose length only the device knows
-            int64_t const n = *a.n_rows_dev;
-            if ( a.n_rows_total && qi == 0 )
-                atomicAdd( a.n_rows_total, (int32_t)n );
-            for ( int64_t i = qi; i < n; i += a.n_rows )
-                query2_row<T, K, STACK>( a, qi, a.rows[i], st_node, st_d );
-            return;
-        }
-    // LDS-stack launches run rows [row0, row0 + n_rows), one per lane
-    if ( qi >= a.n_rows )
-        return;
-    query2_row<T, K, STACK>( a, qi, a.row0 + qi, st_node, st_d );
-}
-
-// The row sort of a two-pass launch for K > kFusedSortK, whose sorting
-// network would take the traversal's registers. A row's 64 slots (entries
-// past the row's length hold keys that sort last) are spread over a group
-// of 64 / E lanes, lane g of the group holding slots g E .. g E + E - 1, so
-// a wave sorts E rows. The bitonic network of sort_row then runs its
-// stages of distance j < E inside each lane and the others across the
-// group's lanes (ds_bpermute). The row's index loads and stores are
-// contiguous per group. 1M rows of 64 (float, uniform points) take 0.40 ms
-// with E = 4, against 0.42 / 0.50 / 0.93 ms with E = 2 / 8 / 16 (fewer
-// VALU per row with more slots per lane, but more registers and fewer
-// rows in flight), 0.59 ms with one row per wave, and 1.19 ms with one row
-// per lane (64 keys in 268 registers, one wave per SIMD, each lane's loads
-// and stores touching 64 cache lines).
-#ifndef DTKX_SORT_ROWS_E
-#define DTKX_SORT_ROWS_E 4
-#endif
-constexpr int kSortE = DTKX_SORT_ROWS_E;   // slots per lane
-constexpr int kSortWaves = 4;              // waves per block
-constexpr int kSortSlots = 64;             // slots per row
-
-// the 32-bit value of the lane whose byte address is given (every lane of
-// the wave is active)
-__device__ inline int lane_read( int v, int addr )
-{
-    return __builtin_amdgcn_ds_bpermute( addr, v );
-}
-
-template <typename T>
-__device__ inline typename SortKey<T>::type
-lane_read_key( typename SortKey<T>::type k, int addr )
-{
-    if constexpr ( sizeof( T ) == 4 )
-    {
-        uint32_t const lo = (uint32_t)lane_read( (int)( k & 0xffffffffu ), addr );
-        uint32_t const hi = (uint32_t)lane_read( (int)( k >> 32 ), addr );
-        return ( (uint64_t)hi << 32 ) | lo;
-    }
-    else
-    {
-        int64_t const b = __double_as_longlong( k.d );
-        int const lo = lane_read( (int)( b & 0xffffffff ), addr );
-        int const hi = lane_read( (int)( b >> 32 ), addr );
-        return {__longlong_as_double( ( (int64_t)hi << 32 ) | (uint32_t)lo ),
-                lane_read( k.id, addr )};
-    }
-}
-
 // a < b and (c ? a : b) field by field, without short-circuit branches
-__device__ inline bool key_less( uint64_t a, uint64_t b ) { return a < b; }
 __device__ inline bool key_less( DKey const &a, DKey const &b )
 {
     return ( a.d < b.d ) | ( ( a.d == b.d ) & ( a.id < b.id ) );
@@ -1453,112 +1001,15 @@ __device__ inline DKey key_pick( bool c, DKey const &a, DKey const &b )
     return {c ? a.d : b.d, c ? a.id : b.id};
 }
 
-template <typename T, int K>
-__global__ void __launch_bounds__( 64 * kSortWaves )
-    knn_sort_rows_kernel( QueryArgs<T> const a )
+} // namespace
+} // namespace dtkx
+
+#include "knn_group.hpp"
+
+namespace dtkx
 {
-    constexpr int E = kSortE, G = kSortSlots / E;
-    static_assert( K <= kSortSlots && G >= 1 && G * E == kSortSlots,
-                   "a row's slots fill its lane group" );
-    using SK = SortKey<T>;
-    int const lane = threadIdx.x & 63;
-    int const g = lane % G; // lane within the row's group
-    int64_t const qi = ( xcd_tile<0>() * kSortWaves + threadIdx.x / 64 ) * E +
-                       lane / G;
-    // rows past the launch's end still run the network (every lane takes
-    // part in the cross-lane reads) with keys that sort last
-    bool const valid = qi < a.n_rows;
-    int64_t const r = a.row0 + ( valid ? qi : 0 );
-    int kk = 0;
-    typename SK::type key[E];
-#pragma unroll
-    for ( int e = 0; e < E; ++e )
-        key[e] = SK::none();
-    int32_t *row = nullptr;
-    int64_t base = 0;
-    if ( valid )
-    {
-        int32_t const t = a.order[r];
-        kk = a.kk;
-        if ( a.src_off )
-            kk = a.kk_prob[a.tgt_prob[t]];
-        typename Vec4<T>::type qp = a.tgt[t];
-        T const q[3] = {qp.x, qp.y, qp.z};
-        base = a.row_off ? a.row_off[r] : ( a.src_pos ? r : (int64_t)t ) * kk;
-        row = a.out_idx + base;
-#pragma unroll
-        for ( int e = 0; e < E; ++e )
-        {
-            int const j = g * E + e;
-            if ( j < kk )
-            {
-                int32_t const id = row[j];
-                typename Vec4<T>::type const p = a.src[id];
-                T const b[3] = {p.x, p.y, p.z};
-                key[e] = SK::make( sqrt_rn( box_sq( q, b, b ) ), id );
-            }
-        }
-    }
-    // slot i = g E + e; of a pair (i, i ^ j), the lower slot of an
-    // ascending block (i & k == 0) keeps the smaller key
-#pragma unroll
-    for ( int k = 2; k <= kSortSlots; k <<= 1 )
-#pragma unroll
-        for ( int j = k >> 1; j > 0; j >>= 1 )
-        {
-            if ( j < E )
-            {
-#pragma unroll
-                for ( int e = 0; e < E; ++e )
-                {
-                    int const f = e ^ j;
-                    if ( f > e )
-                    {
-                        bool const up = ( ( g * E + e ) & k ) == 0;
-                        auto const x = key[e], y = key[f];
-                        bool const lt = key_less( y, x ), gt = key_less( x, y );
-                        bool const swap = ( up & lt ) | ( !up & gt );
-                        key[e] = key_pick( swap, y, x );
-                        key[f] = key_pick( swap, x, y );
-                    }
-                }
-            }
-            else
-            {
-                int const addr = ( lane ^ ( j / E ) ) << 2;
-                // (i & k) and (i & j) depend on the lane only: e < E <= j < k
-                bool const keep_min =
-                    ( ( ( g * E ) & k ) == 0 ) == ( ( ( g * E ) & j ) == 0 );
-#pragma unroll
-                for ( int e = 0; e < E; ++e )
-                {
-                    typename SK::type const other = lane_read_key<T>( key[e], addr );
-                    bool const lt = key_less( other, key[e] );
-                    bool const gt = key_less( key[e], other );
-                    // both comparisons, combined without a branch per lane
-                    bool const take = ( keep_min & lt ) | ( !keep_min & gt );
-                    key[e] = key_pick( take, other, key[e] );
-                }
-            }
-        }
-    if ( valid )
-    {
-#pragma unroll
-        for ( int e = 0; e < E; ++e )
-        {
-            int const j = g * E + e;
-            if ( j < kk )
-            {
-                int32_t const id = SK::index( key[e] );
-                row[j] = a.src_pos ? a.src_pos[id] : id;
-                if ( a.out_dist )
-                    a.out_dist[base + j] = SK::distance( key[e] );
-                if ( a.row_max && j == kk - 1 )
-                    a.row_max[r] = (float)SK::distance( key[e] );
-            }
-        }
-    }
-}
+namespace
+{
 
 template <typename T>
 struct QueryLauncher
@@ -1567,20 +1018,9 @@ struct QueryLauncher
     static void run( int stack, QueryArgs<T> const &a, hipStream_t s )
     {
         dim3 grid( ceil_div( a.n_rows, kQueryBlock ) ), block( kQueryBlock );
-        if constexpr ( K >= two_pass_k<T>() )
-        {
-            if ( stack == kLdsStack )
-                knn_query2_kernel<T, K, kLdsStack><<<grid, block, 0, s>>>( a );
-            else if ( stack == 0 )
-                knn_query2_kernel<T, K, 0><<<grid, block, 0, s>>>( a );
-            else if ( K > kFusedSortK && stack == kSortRows )
-                knn_sort_rows_kernel<T, K>
-                    <<<ceil_div( a.n_rows, kSortWaves * kSortE ),
-                       64 * kSortWaves, 0, s>>>( a );
-        }
-        else if ( stack == kLdsStack )
-            knn_query_kernel<T, K, kLdsStack1><<<grid, block, 0, s>>>( a );
-        else if ( stack == 0 )
+        if ( stack == kLdsStack )
+            knn_query_kernel<T, K, kLdsStack><<<grid, block, 0, s>>>( a );
+        else
             knn_query_kernel<T, K, 0><<<grid, block, 0, s>>>( a );
         DTKX_HIP( hipGetLastError() );
     }
@@ -1596,51 +1036,167 @@ struct QueryLauncher
         run<KV>( stack, a, s );                                                \
         return;                                                                \
     }
-        DTKX_KNN_CASE( 1 )
         DTKX_KNN_CASE( 4 )
-        DTKX_KNN_CASE( 8 )
-        DTKX_KNN_CASE( 10 )
         DTKX_KNN_CASE( 16 )
-        DTKX_KNN_CASE( 24 )
         DTKX_KNN_CASE( 32 )
-        DTKX_KNN_CASE( 48 )
         DTKX_KNN_CASE( 64 )
 #undef DTKX_KNN_CASE
         DTKX_REQUIRE( k <= knn_max_k, DTKX_ERR_UNSUPPORTED );
     }
 };
 
-// the K of the query kernel instantiated for up to k results
-inline int query_bucket( int k )
+// Targets a group and a wave (per_target sources a target). Groups of as
+// many rows as a sort takes, fewer where so many sources lie within the k-th
+// distance of a group (estimated for evenly spread points) that a wave's
+// registers would not hold them. 64 targets a wave, half of that from
+// k = 17, where a wave works long enough for the last ones to show (1M x 1M,
+// search with build: k = 32 0.939 ms against 0.961, k = 10 0.749 against
+// 0.726), and fewer where the launch would have less than 8192 waves (1e5 x
+// 1e5, k = 32: 0.310 ms against 0.332 with 2048 waves at least).
+template <typename T, int S>
+void plan_groups( double per_target, int64_t n_rows, int kk, GroupArgs<T> &g )
 {
-    int const ks[] = {1, 4, 8, 10, 16, 24, 32, 48, 64};
-    for ( int v : ks )
-        if ( k <= v )
-            return v;
-    return 64;
+    double const reach = 2.2 * std::cbrt( 0.2387 * kk );
+    auto candidates = [&]( int n ) {
+        double const e = std::cbrt( n * per_target ) + reach;
+        return e * e * e;
+    };
+    using Shape = GroupShape<T, S>;
+    g.group = Shape::kRows;
+    while ( g.group > 1 &&
+            candidates( g.group ) > 0.7 * Shape::kCand )
+        g.group /= 2;
+    g.per_wave = kk > 16 ? 32 : 64;
+    while ( g.per_wave > 1 && n_rows / g.per_wave < 8192 )
+        g.per_wave /= 2;
+    g.group = std::min( g.group, g.per_wave );
+    g.spacing = (float)( 1.0 / std::cbrt( (double)kk ) );
+    g.root_k = (float)( 1.0 / std::sqrt( (double)kk ) );
 }
 
-// blocks of the global-stack re-run (16k lanes, 12.7 MB of stack)
-constexpr int64_t kRerunBlocks = 256;
+template <typename T, int S>
+void launch_group( GroupArgs<T> g, double per_target, int kk, hipStream_t s )
+{
+    plan_groups<T, S>( per_target, g.a.n_rows, kk, g );
+    knn_group_kernel<T, S>
+        <<<ceil_div( g.a.n_rows, g.per_wave ), 64, 0, s>>>( g );
+    DTKX_HIP( hipGetLastError() );
+}
 
-// The query launch with the LDS stack, then the re-run of its overflow.
-template <typename T>
-void run_queries( int kmax, QueryArgs<T> qa, int64_t n_rows, KnnInfo *info,
+// Boxes of the n sorted sources, level by level (box_levels launches of
+// three levels each). ids (nullable): pts are read through it, and copied
+// in order to sorted.
+template <typename T, typename V>
+void build_boxes( V const *pts, int32_t const *ids, V *sorted, int64_t n,
+                  DeviceBuffer<CurveBox<T>> &buf, BoxLevels<T> &out,
                   hipStream_t s )
 {
-    if ( n_rows == 0 )
+    int64_t count[kMaxBoxLevels] = {};
+    out.n_levels = box_levels( n, count );
+    int64_t total = 0;
+    for ( int l = 0; l < out.n_levels; ++l )
+        total += count[l];
+    buf.resize( total, s );
+    CurveBox<T> *p = buf.get();
+    for ( int l = 0; l < out.n_levels; ++l )
+    {
+        out.level[l] = p;
+        p += count[l];
+    }
+    auto level = [&]( int l ) {
+        return l < out.n_levels ? out.level[l] : nullptr;
+    };
+    box_levels_kernel<T, V, true><<<ceil_div( n, 512 ), 512, 0, s>>>(
+        pts, ids, sorted, nullptr, n, level( 0 ), level( 1 ), level( 2 ) );
+    DTKX_HIP( hipGetLastError() );
+    for ( int l = 3; l < out.n_levels; l += 3 )
+    {
+        box_levels_kernel<T, V, false>
+            <<<ceil_div( count[l - 1], 512 ), 512, 0, s>>>(
+                nullptr, nullptr, nullptr, level( l - 1 ), count[l - 1],
+                level( l ), level( l + 1 ), level( l + 2 ) );
+        DTKX_HIP( hipGetLastError() );
+    }
+}
+
+// the smallest source set searched by groups: one 64-point node
+constexpr int64_t kGroupSources = 64;
+
+// blocks of the global-stack re-run (at most 131k lanes, 102 MB of stack:
+// clouds with hundreds of copies of a point leave every row near them to it)
+constexpr int64_t kRerunBlocks = 2048;
+
+// The queries of a search, in launches of rows with up to kmax results.
+// With boxes, rows are searched by groups of targets (knn_group.hpp);
+// without, the tree search with its LDS stack runs over every row. Rows that
+// either leaves (too many sources at equal distances for the groups'
+// registers, a descent past the LDS stack) are run again by the tree search
+// with a global stack. After the groups the hierarchy is built only if there
+// are such rows: the device decides, the launch returns at once otherwise
+// (5 us, where the hierarchy of 1M sources takes 80).
+// build_tree( wanted ): launches karras_kernel, for *wanted != 0 if given.
+template <typename T, typename BuildTree>
+void run_queries( std::vector<KnnBatch::Launch> const &launches,
+                  QueryArgs<T> qa, int64_t n_tgt, double per_target,
+                  BoxLevels<T> const *boxes, typename Vec4<T>::type const *pts,
+                  int32_t const *ids, BuildTree &&build_tree, KnnInfo *info,
+                  hipStream_t s )
+{
+    if ( n_tgt == 0 )
         return;
-    DeviceBuffer<int32_t> rows( n_rows, s ), count( 1, s );
+    DeviceBuffer<int32_t> rows( n_tgt, s ), count( 1, s );
     zero_async( count.get(), sizeof( int32_t ), s );
     qa.overflow_rows = rows.get();
     qa.n_overflow = count.get();
-    QueryLauncher<T>::dispatch( kmax, kLdsStack, qa, s );
+    int kmax = 1;
+    for ( auto const &l : launches )
+        kmax = std::max( kmax, l.kmax );
+    if ( boxes )
+    {
+        for ( auto const &l : launches )
+        {
+            GroupArgs<T> g;
+            g.a = qa;
+            g.a.row0 = l.begin;
+            g.a.n_rows = l.end - l.begin;
+            g.boxes = *boxes;
+            g.pts = pts;
+            g.ids = ids;
+            if ( g.a.n_rows == 0 )
+                continue;
+            switch ( group_slots( l.kmax ) )
+            {
+            case 16:
+                launch_group<T, 16>( g, per_target, l.kmax, s );
+                break;
+            case 32:
+                launch_group<T, 32>( g, per_target, l.kmax, s );
+                break;
+            case 64:
+                launch_group<T, 64>( g, per_target, l.kmax, s );
+                break;
+            default:
+                launch_group<T, 128>( g, per_target, l.kmax, s );
+            }
+        }
+        build_tree( static_cast<int32_t const *>( count.get() ) );
+    }
+    else
+    {
+        build_tree( nullptr );
+        for ( auto const &l : launches )
+        {
+            qa.row0 = l.begin;
+            qa.n_rows = l.end - l.begin;
+            QueryLauncher<T>::dispatch( l.kmax, kLdsStack, qa, s );
+        }
+    }
     // The re-run is launched without reading the list's length back (a
     // stream synchronisation, 60 us of idle GPU at 1M x 1M): a bounded grid
     // whose lanes stride over the list, each with its own global stack.
     // Almost always the list is empty and the launch costs a few us.
     int64_t const lanes =
-        std::min<int64_t>( ceil_div( n_rows, kQueryBlock ), kRerunBlocks ) *
+        std::min<int64_t>( ceil_div( n_tgt, kQueryBlock ), kRerunBlocks ) *
         kQueryBlock;
     DeviceBuffer<int2> gstack( static_cast<std::size_t>( kMaxDepth ) * lanes,
                                s );
@@ -1663,9 +1219,6 @@ void run_queries( int kmax, QueryArgs<T> qa, int64_t n_rows, KnnInfo *info,
         DTKX_HIP( hipStreamSynchronize( s ) );
         info->n_overflow += n_over;
     }
-    // two-pass rows of large K are written unordered: sort them (a no-op
-    // launch mode for every other K)
-    QueryLauncher<T>::dispatch( kmax, kSortRows, qa, s );
 }
 
 template <typename T>
@@ -1707,11 +1260,11 @@ void knn_impl( void const *src_v, int64_t n_src, void const *tgt_v,
     bbox_final<T><<<1, kBlock, 0, s>>>( partial.get(), nparts, box.get() );
     DTKX_HIP( hipGetLastError() );
 
-    // Morton codes of both point sets (the targets' order only has to be
+    // Hilbert codes of both point sets (the targets' order only has to be
     // local, so their top 30 bits do) with every pass's digit counts
     DeviceBuffer<uint64_t> scodes( n_src, s ), scodes1( n_src, s );
-    DeviceBuffer<uint32_t> tcodes( n_tgt, s ), tcodes1( n_tgt, s );
-    morton_hist_kernel<T, V><<<src_tiles + tgt_tiles, rsort::kThreads, 0, s>>>(
+    DeviceBuffer<uint64_t> tcodes( n_tgt, s ), tcodes1( n_tgt, s );
+    curve_hist_kernel<T, V><<<src_tiles + tgt_tiles, rsort::kThreads, 0, s>>>(
         src, n_src, tgt, n_tgt, box.get(), nullptr, nullptr, src_tiles,
         scodes.get(), tcodes.get(), hist );
     DTKX_HIP( hipGetLastError() );
@@ -1793,25 +1346,30 @@ void knn_impl( void const *src_v, int64_t n_src, void const *tgt_v,
         b.tiles = tgt_tiles;
         b.passes = kTgtPasses;
         b.key_bits = kTgtKeyBits;
-        b.key_bytes = 4;
+        b.key_bytes = 8;
     }
     rsort::sort( pa, s );
     // the sorted codes are back in scodes after an even number of passes
     static_assert( kSrcPasses % 2 == 0, "sorted codes in scodes" );
 
-    // hierarchy
+    if ( n_tgt == 0 )
+        return;
     int64_t const n_int = n_src - 1;
     DeviceBuffer<Node<T>> nodes( std::max<int64_t>( n_int, 1 ), s );
     DeviceBuffer<int32_t> sizes( std::max<int64_t>( n_int, 1 ), s );
-    if ( n_int > 0 )
-    {
+    auto build_tree = [&]( int32_t const *wanted ) {
+        if ( n_int == 0 )
+            return;
         karras_kernel<T, V><<<ceil_div( n_int, kBlock ), kBlock, 0, s>>>(
             scodes.get(), ids_sorted, src, spts, n_int, box.get(), nullptr, 1,
-            nodes.get(), sizes.get() );
+            nodes.get(), sizes.get(), wanted );
         DTKX_HIP( hipGetLastError() );
-    }
-    if ( n_tgt == 0 )
-        return;
+    };
+    bool const grouped = n_src >= kGroupSources;
+    DeviceBuffer<CurveBox<T>> box_buf;
+    BoxLevels<T> boxes;
+    if ( grouped )
+        build_boxes<T, V>( spts, nullptr, nullptr, n_src, box_buf, boxes, s );
 
     QueryArgs<T> qa;
     qa.nodes = nodes.get();
@@ -1819,8 +1377,6 @@ void knn_impl( void const *src_v, int64_t n_src, void const *tgt_v,
     qa.src = src;
     qa.tgt = tgt;
     qa.order = order;
-    qa.row0 = 0;
-    qa.n_rows = n_tgt;
     qa.n_src = n_src;
     qa.kk = kk;
     qa.out_idx = out.indices;
@@ -1829,7 +1385,9 @@ void knn_impl( void const *src_v, int64_t n_src, void const *tgt_v,
     qa.row_max = out.morton_layout ? out.row_max : nullptr;
     if ( info && info->query_begin )
         DTKX_HIP( hipEventRecord( info->query_begin, s ) );
-    run_queries<T>( k, qa, n_tgt, info, s );
+    run_queries<T>( {{0, n_tgt, kk}}, qa, n_tgt, (double)n_src / (double)n_tgt,
+                    grouped ? &boxes : nullptr, spts, ids_sorted, build_tree,
+                    info, s );
     if ( info && info->query_end )
         DTKX_HIP( hipEventRecord( info->query_end, s ) );
     // buffers are released at scope exit, ordered on the stream
@@ -1971,7 +1529,7 @@ void knn_batched_impl( void const *src_v, int64_t n_src, void const *tgt_v,
     DTKX_HIP( hipGetLastError() );
 
     // Two stable radix sorts of both point sets, in shared launches
-    // (radix_sort.hpp): by Morton code in the problem's box (sources 63 bits,
+    // (radix_sort.hpp): by Hilbert code in the problem's box (sources 63 bits,
     // targets 30, as one problem's search orders them), then by the
     // problem's key (sources: the problem; targets: its row key). The second
     // sorts positions of the first, and its last pass gathers the first's
@@ -1998,8 +1556,8 @@ void knn_batched_impl( void const *src_v, int64_t n_src, void const *tgt_v,
 
     DeviceBuffer<uint64_t> scodes( n_src, s ), scodes1( n_src, s ),
         codes_sorted( n_src, s );
-    DeviceBuffer<uint32_t> tcodes( n_tgt, s ), tcodes1( n_tgt, s );
-    morton_hist_kernel<T, V><<<src_tiles + tgt_tiles, rsort::kThreads, 0, s>>>(
+    DeviceBuffer<uint64_t> tcodes( n_tgt, s ), tcodes1( n_tgt, s );
+    curve_hist_kernel<T, V><<<src_tiles + tgt_tiles, rsort::kThreads, 0, s>>>(
         src, n_src, tgt, n_tgt, boxes.get(), b.src_prob, b.tgt_prob,
         src_tiles, scodes.get(), tcodes.get(), st1.hist );
     DTKX_HIP( hipGetLastError() );
@@ -2034,7 +1592,7 @@ void knn_batched_impl( void const *src_v, int64_t n_src, void const *tgt_v,
         t.tiles = tgt_tiles;
         t.passes = kTgtPasses;
         t.key_bits = kTgtKeyBits;
-        t.key_bytes = 4;
+        t.key_bytes = 8;
     };
     rsort::PassArgs pa1;
     pa1.tickets = st1.tickets;
@@ -2098,53 +1656,60 @@ void knn_batched_impl( void const *src_v, int64_t n_src, void const *tgt_v,
     rsort::sort( pa2, s );
     invert_permutation( out.src_perm, n_src, out.src_pos, s );
 
+    if ( n_tgt == 0 )
+        return;
     // one hierarchy per problem, all in one launch
     int64_t const n_int = n_src - P;
     DeviceBuffer<Node<T>> nodes( std::max<int64_t>( n_int, 1 ), s );
     DeviceBuffer<int32_t> sizes( std::max<int64_t>( n_int, 1 ), s );
-    if ( n_int > 0 )
-    {
+    auto build_tree = [&]( int32_t const *wanted ) {
+        if ( n_int == 0 )
+            return;
         karras_kernel<T, V><<<ceil_div( n_int, kBlock ), kBlock, 0, s>>>(
             codes_sorted.get(), out.src_perm, src, nullptr, n_int,
-            boxes.get(), b.src_off, P, nodes.get(), sizes.get() );
+            boxes.get(), b.src_off, P, nodes.get(), sizes.get(), wanted );
         DTKX_HIP( hipGetLastError() );
-    }
-    codes_sorted.release();
-    if ( n_tgt == 0 )
-        return;
+    };
 
-    // rows: ordered by (row key of the problem, Morton code)
+    // rows: ordered by (row key of the problem, Hilbert code)
     row_offsets_kernel<<<ceil_div( n_tgt + 1, kBlock ), kBlock, 0, s>>>(
         out.order, b.tgt_prob, b.row_base, b.row_start, b.kk_prob, n_tgt,
         b.nnz, out.row_off );
     DTKX_HIP( hipGetLastError() );
 
+    bool const grouped = n_src >= kGroupSources;
+    DeviceBuffer<V> spts( grouped ? n_src : 0, s );
+    DeviceBuffer<CurveBox<T>> box_buf;
+    BoxLevels<T> levels;
+    if ( grouped )
+        build_boxes<T, V>( src, out.src_perm, spts.get(), n_src, box_buf, levels,
+                           s );
+
     if ( info && info->query_begin )
         DTKX_HIP( hipEventRecord( info->query_begin, s ) );
-    for ( auto const &l : b.launches )
-    {
-        QueryArgs<T> qa;
-        qa.nodes = nodes.get();
-        qa.node_size = kSeed ? sizes.get() : nullptr;
-        qa.src = src;
-        qa.tgt = tgt;
-        qa.order = out.order;
-        qa.row0 = l.begin;
-        qa.n_rows = l.end - l.begin;
-        qa.src_off = b.src_off;
-        qa.tgt_prob = b.tgt_prob;
-        qa.kk_prob = b.kk_prob;
-        qa.row_off = out.row_off;
-        qa.out_idx = out.indices;
-        qa.src_pos = out.src_pos;
-        qa.row_max = out.row_max;
-        run_queries<T>( l.kmax, qa, l.end - l.begin, info, s );
-    }
+    QueryArgs<T> qa;
+    qa.nodes = nodes.get();
+    qa.node_size = kSeed ? sizes.get() : nullptr;
+    qa.src = src;
+    qa.tgt = tgt;
+    qa.order = out.order;
+    qa.src_off = b.src_off;
+    qa.tgt_prob = b.tgt_prob;
+    qa.kk_prob = b.kk_prob;
+    qa.row_off = out.row_off;
+    qa.out_idx = out.indices;
+    qa.src_pos = out.src_pos;
+    qa.row_max = out.row_max;
+    run_queries<T>( b.launches, qa, n_tgt, (double)n_src / (double)n_tgt,
+                    grouped ? &levels : nullptr, spts.get(), out.src_perm,
+                    build_tree, info, s );
     if ( info && info->query_end )
         DTKX_HIP( hipEventRecord( info->query_end, s ) );
 }
 
 } // namespace
+
+int knn_bucket( int k ) { return group_slots( k ); }
 
 void knn_search_batched( int geometry, void const *src, int64_t n_src,
                          void const *tgt, int64_t n_tgt, KnnBatch const &b,

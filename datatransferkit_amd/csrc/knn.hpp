@@ -29,10 +29,10 @@ struct KnnInfo
 
 // Results of a search. indices: [n_tgt][kk], kk = min(k, n_src); dist
 // (nullable): matching distances. query_order (nullable): the targets in
-// the Morton order the queries ran in (row r of a Morton layout holds
+// the Hilbert order the queries ran in (row r of a curve layout holds
 // target query_order[r]). src_perm / src_pos (nullable): the sources in
-// Morton order and its inverse. With morton_layout, row r of indices/dist
-// is the r-th query and every index is the source's Morton position
+// Hilbert order and its inverse. With morton_layout, row r of indices/dist
+// is the r-th query and every index is the source's curve position
 // (src_pos[source]); otherwise row t is target t and indices are source
 // indices. Either way a row is ordered by (distance, source index).
 struct KnnOutput
@@ -43,13 +43,13 @@ struct KnnOutput
     int32_t *src_perm = nullptr;
     int32_t *src_pos = nullptr;
     bool morton_layout = false;
-    // nullable, Morton layout: each row's largest neighbour distance (the
+    // nullable, curve layout: each row's largest neighbour distance (the
     // k-th, as the search computes it)
     float *row_max = nullptr;
     // nullable: the inverse of query_order (query_pos[target] = row)
     int32_t *query_pos = nullptr;
     // nullable: sorted_src[position] = src4[source], a double4 copy of the
-    // sources in Morton order (src4 may be the search's own points)
+    // sources in Hilbert order (src4 may be the search's own points)
     double4 const *src4 = nullptr;
     double4 *sorted_src = nullptr;
 };
@@ -65,7 +65,7 @@ void knn_search( int geometry, void const *src, int64_t n_src,
 // [tgt_off[p], tgt_off[p + 1]) of the concatenated arrays (every problem has
 // at least one source). Each problem's hierarchy is built over its own
 // sorted range inside one set of kernels, and each query starts at its
-// problem's root. Output rows are ordered by (row_key[problem], Morton code
+// problem's root. Output rows are ordered by (row_key[problem], Hilbert code
 // of the target in its problem's box); row r holds kk_prob[p] neighbours at
 // CSR offset row_off[r] = row_base[p] + (r - row_start[p]) kk_prob[p], as
 // global source positions (the sorted order is problem-major, so problem p's
@@ -106,6 +106,10 @@ void knn_search_batched( int geometry, void const *src, int64_t n_src,
                          void const *tgt, int64_t n_tgt, KnnBatch const &b,
                          KnnBatchOutput const &out, KnnInfo *info,
                          hipStream_t s );
+
+// Rows of equal buckets can share a query launch (the row slots of the
+// group search).
+int knn_bucket( int k );
 
 // Largest k the query kernels are instantiated for.
 constexpr int knn_max_k = 64;

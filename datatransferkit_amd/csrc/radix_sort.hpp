@@ -1,4 +1,4 @@
-// Stable LSD radix sort of (key, index) pairs for the kNN build's Morton
+// Stable LSD radix sort of (key, index) pairs for the kNN build's curve
 // codes, written for gfx950 wave64.
 //
 // One launch per 8-bit digit. A block takes a tile of 8192 keys (a ticket
@@ -19,7 +19,7 @@
 // of each digit) come from the kernel that writes the keys; the look-back
 // words of the first pass and the tickets start at zero (cleared by an
 // earlier kernel of the chain). Pass p clears the words pass p + 1 uses.
-// Two independent arrays (the sources' 63-bit codes and the targets' 30-bit
+// Two independent arrays (the sources' 63-bit codes and the targets' 48-bit
 // ones) share the launches. The last pass can also write the inverse
 // permutation and gather up to two per-index records into sorted order.
 #ifndef DTKX_RADIX_SORT_HPP

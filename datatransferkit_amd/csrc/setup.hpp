@@ -49,7 +49,7 @@ struct SetupParams
 // the eigen-solver; accumulated atomically.
 // Row r of indices and coeffs belongs to target order[r] (identity when
 // order is null); indices address src, which may be the sources in a
-// permuted (Morton) order.
+// permuted (curve) order.
 
 // Classical max-pivot two-sided Jacobi, reference operation order.
 int setup_classical( double4 const *src, double4 const *tgt, int64_t n_tgt,

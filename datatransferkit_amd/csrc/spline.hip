@@ -391,7 +391,7 @@ __global__ void __launch_bounds__( kBlock )
 }
 
 // ------------------------------------------------------ renumbering
-// Sources renumbered by their Morton position (perm: position -> source,
+// Sources renumbered by their curve position (perm: position -> source,
 // pos: source -> position): row p of the position-ordered M is row
 // perm[p] with its indices mapped through pos, and the point rows follow.
 template <typename Pt>

@@ -46,7 +46,7 @@ void spline_basis_weights( double4 const *src, double4 const *pts, int64_t n,
                            int kk, int32_t const *idx, int rbf, int geometry,
                            double *phi, hipStream_t s );
 
-// The sources renumbered by their Morton position (perm: position ->
+// The sources renumbered by their curve position (perm: position ->
 // source, pos: its inverse), so that the operator's gathers stay local:
 // M's rows and the source points are reordered and their indices mapped,
 // N's indices are mapped. Every buffer is device memory.
