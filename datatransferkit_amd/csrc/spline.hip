@@ -14,6 +14,7 @@
 #include <algorithm>
 #include <cfloat>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 namespace dtkx
@@ -23,29 +24,20 @@ namespace
 
 constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / 64;
-// Krylov kernels. Dots (gemv_t): each block takes kRowsT rows per thread
-// and a group of kGroup basis vectors, so a thread has kGroup
-// independent loads per row and two wave reductions per vector for kRowsT
-// rows. Updates (gemv_n, dcgs2_update, residual): kRowsN rows per thread,
-// many waves. Solve at 1M sources (91 iterations), rows x group:
-// 8 x 16 21.6 ms, 4 x 16 22.6, 8 x 8 20.0, 4 x 8 20.5, 16 x 8 19.9,
-// 32 x 8 20.4, 8 x 4 19.8, 16 x 4 19.8; kRowsN 1, 2, 4: 21.8, 21.6, 21.9.
-#ifndef DTKX_SPLINE_ROWS_T
-#define DTKX_SPLINE_ROWS_T 16
-#endif
-#ifndef DTKX_SPLINE_GROUP
-#define DTKX_SPLINE_GROUP 8
-#endif
-#ifndef DTKX_SPLINE_ROWS_N
-#define DTKX_SPLINE_ROWS_N 2
-#endif
-constexpr int kRowsT = DTKX_SPLINE_ROWS_T;
-constexpr int kTileT = kBlock * kRowsT;
-constexpr int kGroup = DTKX_SPLINE_GROUP;
-constexpr int kRowsN = DTKX_SPLINE_ROWS_N;
-constexpr int kTileN = kBlock * kRowsN;
+// Krylov kernels. Dots (gemv_t): each block takes rows_t rows per thread
+// and a group of kGroup basis vectors, so a thread has kGroup independent
+// loads per row and two wave reductions per vector for its rows. Updates
+// (gemv_n, dcgs2_update, residual): rows_n rows per thread, many waves.
+// Solve at 1M sources (91 iterations), rows x group: 8 x 16 21.6 ms, 4 x 16
+// 22.6, 8 x 8 20.0, 4 x 8 20.5, 16 x 8 19.9, 32 x 8 20.4, 8 x 4 19.8,
+// 16 x 4 19.8; rows_n 1, 2, 4: 21.8, 21.6, 21.9. Below that size the rows a
+// thread fall with n (rows_t, rows_n), to keep the chip full: see there.
+constexpr int kGroup = 8;
 // largest number of basis vectors one orthogonalisation pass handles
 constexpr int kMaxVectors = 512;
+// rows a thread of the cycle-end kernels
+constexpr int kRowsN = 2;
+constexpr int kTileN = kBlock * kRowsN;
 // grid of the operator kernels (grid-stride over the rows)
 constexpr int kRowBlocks = 2048;
 
@@ -157,9 +149,11 @@ __global__ void __launch_bounds__( kBlock )
     }
 }
 
-// out[v] = sum_b partial[v][b] over nb blocks, one wave per v.
+// out[v] = sum_b partial[v][b] over nb blocks, one wave per v; also to
+// host_out (nullable, pinned host memory).
 __global__ void __launch_bounds__( kBlock )
-    reduce_kernel( double const *partial, int nb, int nv, double *out )
+    reduce_kernel( double const *partial, int nb, int nv, double *out,
+                   double *host_out = nullptr )
 {
     int const v = blockIdx.x * kWaves + ( threadIdx.x >> 6 );
     int const lane = threadIdx.x & 63;
@@ -170,12 +164,20 @@ __global__ void __launch_bounds__( kBlock )
         a += partial[(int64_t)v * nb + b];
     a = wave_sum( a );
     if ( lane == 0 )
+    {
         out[v] = a;
+        if ( host_out )
+        {
+            host_out[v] = a;
+            __threadfence_system();
+        }
+    }
 }
 
 // partial[2 v + k][row block] = sum over the block's rows of q_v[i] r_k[i]
 // for the two right-hand sides r_0, r_1 and the vectors v of the block's
 // group (blockIdx.y), v < nv.
+template <int ROWS>
 __global__ void __launch_bounds__( kBlock )
     gemv_t_kernel( double const *basis, int64_t ld, int nv, int64_t n,
                    double const *r0, double const *r1, double *partial )
@@ -183,7 +185,7 @@ __global__ void __launch_bounds__( kBlock )
     __shared__ double lds[kWaves][2 * kGroup];
     int const v0 = blockIdx.y * kGroup;
     int const cnt = min( kGroup, nv - v0 );
-    int64_t const base = blockIdx.x * (int64_t)kTileT + threadIdx.x;
+    int64_t const base = blockIdx.x * (int64_t)( kBlock * ROWS ) + threadIdx.x;
     double a0[kGroup], a1[kGroup];
 #pragma unroll
     for ( int g = 0; g < kGroup; ++g )
@@ -198,7 +200,7 @@ __global__ void __launch_bounds__( kBlock )
     for ( int g = 0; g < kGroup; ++g )
         q[g] = basis + min( v0 + g, nv - 1 ) * ld;
 #pragma unroll 2
-    for ( int r = 0; r < kRowsT; ++r )
+    for ( int r = 0; r < ROWS; ++r )
     {
         int64_t const i = base + r * kBlock;
         int64_t const ic = min( i, n - 1 );
@@ -237,28 +239,59 @@ __global__ void __launch_bounds__( kBlock )
     }
 }
 
-// One step of the delayed reorthogonalisation, rows of kRowsN per thread:
+// One step of the delayed reorthogonalisation, ROWS rows per thread:
 //   q_j = (u - sum_{v<j} q_v s_v) / rho      (u is basis vector j)
 //   v   = (w - sum_{v<j} q_v t_v - q_j gamma) / rho   (w is vector j + 1)
-// with s_v = st[2 v], t_v = st[2 v + 1]; q_j and v overwrite u and w.
+// with s_v = st[2 v], t_v = st[2 v + 1], rho^2 = st[2 j] - |s|^2 (0 if that
+// is not positive) and gamma = (st[2 j + 1] - s^T t) / rho, which every
+// block forms for itself, so that the host need not have seen the dots;
+// q_j and v overwrite u and w. scalars: rho and gamma, for the host.
+template <int ROWS>
 __global__ void __launch_bounds__( kBlock )
     dcgs2_update_kernel( double *basis, int64_t ld, int j, int64_t n,
-                         double const *st, double inv_rho, double gamma )
+                         double const *st, double *scalars )
 {
     __shared__ double ss[kMaxVectors], ts[kMaxVectors];
+    __shared__ double sums[2];
     for ( int v = threadIdx.x; v < j; v += kBlock )
     {
         ss[v] = st[2 * v];
         ts[v] = st[2 * v + 1];
     }
     __syncthreads();
+    if ( threadIdx.x < 64 )
+    {
+        double a = 0., b = 0.;
+        for ( int v = threadIdx.x; v < j; v += 64 )
+        {
+            a += ss[v] * ss[v];
+            b += ss[v] * ts[v];
+        }
+        a = wave_sum( a );
+        b = wave_sum( b );
+        if ( threadIdx.x == 0 )
+        {
+            double const rho2 = st[2 * j] - a;
+            double const rho = rho2 > 0. ? sqrt( rho2 ) : 0.;
+            sums[0] = 1. / rho;
+            sums[1] = ( st[2 * j + 1] - b ) / rho;
+            if ( blockIdx.x == 0 )
+            {
+                scalars[0] = rho;
+                scalars[1] = sums[1];
+                __threadfence_system();
+            }
+        }
+    }
+    __syncthreads();
+    double const inv_rho = sums[0], gamma = sums[1];
     double *const u = basis + j * ld;
     double *const w = u + ld;
-    int64_t const base = blockIdx.x * (int64_t)kTileN + threadIdx.x;
-    int64_t ii[kRowsN];
-    double au[kRowsN], aw[kRowsN];
+    int64_t const base = blockIdx.x * (int64_t)( kBlock * ROWS ) + threadIdx.x;
+    int64_t ii[ROWS];
+    double au[ROWS], aw[ROWS];
 #pragma unroll
-    for ( int r = 0; r < kRowsN; ++r )
+    for ( int r = 0; r < ROWS; ++r )
     {
         // rows past n read row n - 1 and are not written back
         ii[r] = min( base + r * kBlock, n - 1 );
@@ -271,7 +304,7 @@ __global__ void __launch_bounds__( kBlock )
         double const *q = basis + v * ld;
         double const sv = ss[v], tv = ts[v];
 #pragma unroll
-        for ( int r = 0; r < kRowsN; ++r )
+        for ( int r = 0; r < ROWS; ++r )
         {
             double const qv = q[ii[r]];
             au[r] -= qv * sv;
@@ -279,7 +312,7 @@ __global__ void __launch_bounds__( kBlock )
         }
     }
 #pragma unroll
-    for ( int r = 0; r < kRowsN; ++r )
+    for ( int r = 0; r < ROWS; ++r )
     {
         int64_t const i = base + r * kBlock;
         if ( i < n )
@@ -477,7 +510,27 @@ void system_apply( SplineSystem const &sys, double const *z, double *y,
     DTKX_HIP( hipGetLastError() );
 }
 
-int tiles_t( int64_t n ) { return (int)( ( n + kTileT - 1 ) / kTileT ); }
+// Rows a thread of the dots: 16, halved down to 2 while there are fewer than
+// 128 row tiles (a launch has one block a tile and group of 8 vectors; 150k
+// sources have 37 tiles of 16 rows a thread). Solve with 16 / this rule:
+// 30k sources 2.27 / 1.74 ms, 150k 4.05 / 3.35, 400k 7.28 / 6.90 (with 4 rows
+// 7.24), the update at its rows below.
+int rows_t( int64_t n )
+{
+    int r = 16;
+    while ( r > 2 && n < (int64_t)128 * kBlock * r )
+        r /= 2;
+    return r;
+}
+int tiles_t( int64_t n )
+{
+    int const tile = kBlock * rows_t( n );
+    return (int)( ( n + tile - 1 ) / tile );
+}
+// Rows a thread of the basis update: with 2, 150k sources are 293 blocks
+// whose threads walk the basis with too few loads in flight (solve 4.05 ms
+// against 3.35 with 1).
+int rows_n( int64_t n ) { return n < 500000 ? 1 : 2; }
 int tiles_n( int64_t n ) { return (int)( ( n + kTileN - 1 ) / kTileN ); }
 int groups( int nv ) { return ( nv + kGroup - 1 ) / kGroup; }
 
@@ -561,6 +614,9 @@ SplineSolver::~SplineSolver()
 {
     if ( host_ )
         (void)hipHostFree( host_ );
+    for ( auto e : events_ )
+        if ( e )
+            (void)hipEventDestroy( e );
 }
 
 void SplineSolver::reserve( int64_t n, int restart, hipStream_t s )
@@ -583,8 +639,15 @@ void SplineSolver::reserve( int64_t n, int restart, hipStream_t s )
     if ( host_ )
         DTKX_HIP( hipHostFree( host_ ) );
     host_ = nullptr;
-    DTKX_HIP( hipHostMalloc( (void **)&host_, 3 * nv * sizeof( double ),
+    // a slot: the dots of restart + 1 vectors, rho and gamma
+    slot_ = 2 * nv + 2;
+    DTKX_HIP( hipHostMalloc( (void **)&host_,
+                             ( kSlots * slot_ + nv ) * sizeof( double ),
                              hipHostMallocDefault ) );
+    host_y_ = host_ + kSlots * slot_;
+    for ( auto &e : events_ )
+        if ( !e )
+            DTKX_HIP( hipEventCreateWithFlags( &e, hipEventDisableTiming ) );
 }
 
 GmresInfo SplineSolver::solve( SplineSystem const &sys, double const *x,
@@ -602,16 +665,34 @@ GmresInfo SplineSolver::solve( SplineSystem const &sys, double const *x,
     double *const part = partial_.get();
     double *const dots = dots_.get();
     auto fetch = [&]( double const *src, int count ) {
-        DTKX_HIP( hipMemcpyAsync( host_, src, count * sizeof( double ),
+        DTKX_HIP( hipMemcpyAsync( host_y_, src, count * sizeof( double ),
                                   hipMemcpyDeviceToHost, s ) );
         DTKX_HIP( hipStreamSynchronize( s ) );
     };
-    // dots[2 v + k] = Q[v]^T r_k, v < nv
-    auto project = [&]( int nv, double const *r0, double const *r1 ) {
-        gemv_t_kernel<<<dim3( nbt, groups( nv ) ), kBlock, 0, s>>>(
-            Q, ld, nv, n, r0, r1, part );
+    // dots[2 v + k] = q_v^T r_k for the nv vectors q_v at q, and to host
+    auto project = [&]( double const *q, int nv, double const *r0,
+                        double const *r1, double *host ) {
+        auto run = [&]( auto rows ) {
+            gemv_t_kernel<decltype( rows )::value>
+                <<<dim3( nbt, groups( nv ) ), kBlock, 0, s>>>( q, ld, nv, n,
+                                                               r0, r1, part );
+        };
+        switch ( rows_t( n ) )
+        {
+        case 2:
+            run( std::integral_constant<int, 2>{} );
+            break;
+        case 4:
+            run( std::integral_constant<int, 4>{} );
+            break;
+        case 8:
+            run( std::integral_constant<int, 8>{} );
+            break;
+        default:
+            run( std::integral_constant<int, 16>{} );
+        }
         reduce_kernel<<<( 2 * nv + kWaves - 1 ) / kWaves, kBlock, 0, s>>>(
-            part, nbt, 2 * nv, dots );
+            part, nbt, 2 * nv, dots, host );
         DTKX_HIP( hipGetLastError() );
     };
     // b = S x = [x; 0], z = 0 (def.hpp:200-203, 286-291)
@@ -622,11 +703,9 @@ GmresInfo SplineSolver::solve( SplineSystem const &sys, double const *x,
     DTKX_HIP( hipMemsetAsync( z, 0, n * sizeof( double ), s ) );
     GmresInfo info;
     // |b|^2: b as the only basis vector of a projection
-    gemv_t_kernel<<<dim3( nbt, 1 ), kBlock, 0, s>>>( b, ld, 1, n, b, b, part );
-    reduce_kernel<<<1, kBlock, 0, s>>>( part, nbt, 1, dots );
-    DTKX_HIP( hipGetLastError() );
+    project( b, 1, b, b, nullptr );
     fetch( dots, 1 );
-    double const beta = std::sqrt( host_[0] );
+    double const beta = std::sqrt( host_y_[0] );
     if ( !( beta > 0. ) )
     {
         info.converged = std::isfinite( beta );
@@ -653,7 +732,35 @@ GmresInfo SplineSolver::solve( SplineSystem const &sys, double const *x,
     double rnorm = beta;
     int total = 0;
     int const gblocks = (int)( ( n + kBlock - 1 ) / kBlock );
-    int const ublocks = tiles_n( n );
+    int const rn = rows_n( n );
+    int const ublocks =
+        (int)( ( n + kBlock * rn - 1 ) / ( (int64_t)kBlock * rn ) );
+    // Iteration j on the stream: everything it needs of the earlier ones is
+    // on the device, so the host queues up to kAhead iterations past the
+    // one whose column it is forming (each ends with an event; its dots,
+    // rho and gamma lie in a pinned slot of their own). Iterations queued
+    // past the last one used write basis vectors that are not read.
+    auto slot = [&]( int j ) { return host_ + ( j % kSlots ) * slot_; };
+    auto enqueue = [&]( int j ) {
+        bool const last = j == m; // only column m - 1 is left to finalise
+        double *const u = Q + j * ld;
+        double *const w = u + ld;
+        double *const h = slot( j );
+        if ( !last )
+            system_apply( sys, u, w, part, s );
+        project( Q, j + 1, u, last ? u : w, h );
+        if ( !last )
+        {
+            if ( rn == 1 )
+                dcgs2_update_kernel<1><<<ublocks, kBlock, 0, s>>>(
+                    Q, ld, j, n, dots, h + 2 * ( j + 1 ) );
+            else
+                dcgs2_update_kernel<2><<<ublocks, kBlock, 0, s>>>(
+                    Q, ld, j, n, dots, h + 2 * ( j + 1 ) );
+            DTKX_HIP( hipGetLastError() );
+        }
+        DTKX_HIP( hipEventRecord( events_[j % kSlots], s ) );
+    };
     while ( true )
     {
         // u = r / |r|
@@ -662,27 +769,28 @@ GmresInfo SplineSolver::solve( SplineSystem const &sys, double const *x,
         std::fill( g.begin(), g.end(), 0. );
         int j = 0; // u = Q[j]
         int k = 0; // final columns
-        while ( true )
+        int queued = 0;
+        // no further ahead than the residual's last step lets expect
+        int ahead = 0;
+        int const end = std::min( m, opt.max_iterations - total );
+        while ( total < opt.max_iterations )
         {
-            // j == m: only column m - 1 is left to finalise
             bool const last = j == m;
-            if ( j == 0 && total >= opt.max_iterations )
-                break;
-            double *const u = Q + j * ld;
-            double *const w = u + ld;
-            if ( !last )
-                system_apply( sys, u, w, part, s );
-            project( j + 1, u, last ? u : w );
-            fetch( dots, 2 * ( j + 1 ) );
-            double ss = 0., st = 0.;
-            for ( int v = 0; v < j; ++v )
+            for ( ; queued <= std::min( end, j + ahead ); ++queued )
+                enqueue( queued );
+            DTKX_HIP( hipEventSynchronize( events_[j % kSlots] ) );
+            double const *const dot = slot( j );
+            double rho = dot[2 * ( j + 1 )];
+            double const gamma = dot[2 * ( j + 1 ) + 1];
+            if ( last )
             {
-                ss += host_[2 * v] * host_[2 * v];
-                st += host_[2 * v] * host_[2 * v + 1];
+                // (no update, which forms it)
+                double ss = 0.;
+                for ( int v = 0; v < j; ++v )
+                    ss += dot[2 * v] * dot[2 * v];
+                double const rho2 = dot[2 * j] - ss;
+                rho = rho2 > 0. ? std::sqrt( rho2 ) : 0.;
             }
-            double const sigma = host_[2 * j], tau = host_[2 * j + 1];
-            double const rho2 = sigma - ss;
-            double const rho = rho2 > 0. ? std::sqrt( rho2 ) : 0.;
             if ( j == 0 )
                 g[0] = rnorm * rho; // r = rnorm u = rnorm rho q_0
             else
@@ -690,7 +798,7 @@ GmresInfo SplineSolver::solve( SplineSystem const &sys, double const *x,
                 // column j - 1 is final
                 int const c = j - 1;
                 for ( int v = 0; v < j; ++v )
-                    at( Ha, v, c ) += host_[2 * v];
+                    at( Ha, v, c ) += dot[2 * v];
                 at( Ha, j, c ) = rho;
                 for ( int v = 0; v <= j; ++v )
                     at( R, v, c ) = at( Ha, v, c );
@@ -715,25 +823,24 @@ GmresInfo SplineSolver::solve( SplineSystem const &sys, double const *x,
                 if ( !std::isfinite( rho ) || std::fabs( g[j] ) <= target ||
                      !( rho > 0. ) || last || total >= opt.max_iterations )
                     break; // converged, invariant Krylov space, or done
+                double e = std::fabs( g[j] );
+                for ( ahead = 0; ahead < kAhead && e > target; ++ahead )
+                    e *= std::fabs( sn[c] );
             }
             if ( !( rho > 0. ) || !std::isfinite( rho ) )
                 break;
             // provisional column j: ([t; gamma] - H(0:j, 0:j-1) s) / rho
-            double const gamma = ( tau - st ) / rho;
             for ( int v = 0; v <= j; ++v )
             {
                 double a = 0.;
                 for ( int c = 0; c < j && c + 1 >= v; ++c )
-                    a += at( Ha, v, c ) * host_[2 * c];
+                    a += at( Ha, v, c ) * dot[2 * c];
                 hs[v] = a;
             }
             for ( int v = 0; v < j; ++v )
-                at( Ha, v, j ) = ( host_[2 * v + 1] - hs[v] ) / rho;
+                at( Ha, v, j ) = ( dot[2 * v + 1] - hs[v] ) / rho;
             at( Ha, j, j ) = ( gamma - hs[j] ) / rho;
             at( Ha, j + 1, j ) = 1.;
-            dcgs2_update_kernel<<<ublocks, kBlock, 0, s>>>( Q, ld, j, n, dots,
-                                                            1. / rho, gamma );
-            DTKX_HIP( hipGetLastError() );
             ++j;
         }
         // z += Q_k y, R(0:k, 0:k) y = g(0:k)
@@ -746,9 +853,10 @@ GmresInfo SplineSolver::solve( SplineSystem const &sys, double const *x,
         }
         if ( k > 0 )
         {
+            // (the slots may still be written by iterations queued ahead)
             for ( int i = 0; i < k; ++i )
-                host_[i] = -yv[i];
-            DTKX_HIP( hipMemcpyAsync( dots, host_, k * sizeof( double ),
+                host_y_[i] = -yv[i];
+            DTKX_HIP( hipMemcpyAsync( dots, host_y_, k * sizeof( double ),
                                       hipMemcpyHostToDevice, s ) );
             gemv_n_kernel<<<nbn, kBlock, 0, s>>>( Q, ld, k, n, dots, z,
                                                   nullptr );
@@ -760,7 +868,7 @@ GmresInfo SplineSolver::solve( SplineSystem const &sys, double const *x,
         reduce_kernel<<<1, kBlock, 0, s>>>( part, nbn, 1, dots );
         DTKX_HIP( hipGetLastError() );
         fetch( dots, 1 );
-        rnorm = std::sqrt( host_[0] );
+        rnorm = std::sqrt( host_y_[0] );
         info.iterations = total;
         info.residual = rnorm / beta;
         info.converged = rnorm <= target;

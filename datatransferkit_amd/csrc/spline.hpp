@@ -107,7 +107,13 @@ class SplineSolver
     int64_t ld_ = 0;
     int restart_ = 0;
     DeviceBuffer<double> basis_, rhs_, res_, partial_, dots_;
-    double *host_ = nullptr; // pinned: projections and norms
+    // iterations queued past the one whose column the host is forming (the
+    // GPU idled for 15 us an iteration without), and their pinned slots
+    static constexpr int kAhead = 2, kSlots = kAhead + 1;
+    std::size_t slot_ = 0;
+    double *host_ = nullptr;   // pinned: kSlots slots, then host_y_
+    double *host_y_ = nullptr; // pinned: the cycle's combination, norms
+    hipEvent_t events_[kSlots] = {};
 };
 
 } // namespace dtkx
