@@ -302,6 +302,16 @@ __global__ void __launch_bounds__( rsort::kThreads )
     }
 }
 
+} // namespace
+} // namespace dtkx
+
+#include "knn_small.hpp"
+
+namespace dtkx
+{
+namespace
+{
+
 // ------------------------------------------------------ Karras hierarchy
 // delta(i, j): common prefix length of keys i and j, with the index used
 // to break ties between equal codes; -1 outside [0, n).
@@ -1231,44 +1241,6 @@ void knn_impl( void const *src_v, int64_t n_src, void const *tgt_v,
     V const *tgt = static_cast<V const *>( tgt_v );
     int const kk = static_cast<int>( k < n_src ? k : n_src );
 
-    // Sort state, one buffer: the digit counts of every pass, the tile
-    // tickets and the look-back words of the first pass (all cleared by the
-    // scene-box launch), then those of the second pass (cleared by the
-    // first pass).
-    int const src_tiles = rsort::tiles_for( n_src );
-    int const tgt_tiles = rsort::tiles_for( n_tgt );
-    std::size_t const head = ( kHistWords + 4 * rsort::kMaxPasses ) * 4;
-    std::size_t const look_src = (std::size_t)src_tiles * rsort::kDigits * 8;
-    std::size_t const look_tgt = (std::size_t)tgt_tiles * rsort::kDigits * 8;
-    std::size_t const zero_bytes = head + look_src + look_tgt;
-    static_assert( ( kHistWords + 4 * rsort::kMaxPasses ) * 4 % 16 == 0,
-                   "uint4 clearing" );
-    DeviceBuffer<uint4> state( ( zero_bytes + look_src + look_tgt ) / 16, s );
-    char *const st = reinterpret_cast<char *>( state.get() );
-    uint32_t *const hist = reinterpret_cast<uint32_t *>( st );
-    uint32_t *const tickets = hist + kHistWords;
-    uint64_t *const look0 = reinterpret_cast<uint64_t *>( st + head );
-    uint64_t *const look1 = reinterpret_cast<uint64_t *>( st + zero_bytes );
-
-    // scene box of the sources
-    int nparts = static_cast<int>( std::min<int64_t>(
-        1024, std::max<int64_t>( 1, ceil_div( n_src, kBlock ) ) ) );
-    DeviceBuffer<T> partial( 6 * nparts, s ), box( 6, s );
-    bbox_partial<T, V><<<nparts, kBlock, 0, s>>>(
-        src, n_src, partial.get(), state.get(),
-        static_cast<int64_t>( zero_bytes / 16 ) );
-    bbox_final<T><<<1, kBlock, 0, s>>>( partial.get(), nparts, box.get() );
-    DTKX_HIP( hipGetLastError() );
-
-    // Hilbert codes of both point sets (the targets' order only has to be
-    // local, so their top 30 bits do) with every pass's digit counts
-    DeviceBuffer<uint64_t> scodes( n_src, s ), scodes1( n_src, s );
-    DeviceBuffer<uint64_t> tcodes( n_tgt, s ), tcodes1( n_tgt, s );
-    curve_hist_kernel<T, V><<<src_tiles + tgt_tiles, rsort::kThreads, 0, s>>>(
-        src, n_src, tgt, n_tgt, box.get(), nullptr, nullptr, src_tiles,
-        scodes.get(), tcodes.get(), hist );
-    DTKX_HIP( hipGetLastError() );
-
     // outputs of the sort: the permutations, their inverses, the points in
     // sorted order (the hierarchy's copy, and the caller's double4 copy,
     // one buffer when they coincide)
@@ -1301,56 +1273,120 @@ void knn_impl( void const *src_v, int64_t n_src, void const *tgt_v,
         spts_buf.resize( n_src, s );
         spts = spts_buf.get();
     }
-    DeviceBuffer<int32_t> svals( 2 * n_src, s ), tvals( 2 * n_tgt, s );
+    DeviceBuffer<T> box( 6, s );
+    DeviceBuffer<uint64_t> scodes( n_src, s );
+    if ( n_src <= kSmallSort && n_tgt <= kSmallSort )
+    {
+        SmallSortArgs<T, V> g;
+        g.src = src;
+        g.tgt = tgt;
+        g.n_src = static_cast<int>( n_src );
+        g.n_tgt = static_cast<int>( n_tgt );
+        g.box = box.get();
+        g.codes = scodes.get();
+        g.src_ids = ids_sorted;
+        g.src_pos = src_pos;
+        g.tgt_ids = order;
+        g.tgt_pos = out.query_pos;
+        g.src_sorted = spts;
+        if ( out.sorted_src && !share )
+        {
+            g.src4 = out.src4;
+            g.src4_sorted = out.sorted_src;
+        }
+        small_sort( g, s );
+    }
+    else
+    {
+        // Sort state, one buffer: the digit counts of every pass, the tile
+        // tickets and the look-back words of the first pass (all cleared by the
+        // scene-box launch), then those of the second pass (cleared by the
+        // first pass).
+        int const src_tiles = rsort::tiles_for( n_src );
+        int const tgt_tiles = rsort::tiles_for( n_tgt );
+        std::size_t const head = ( kHistWords + 4 * rsort::kMaxPasses ) * 4;
+        std::size_t const look_src = (std::size_t)src_tiles * rsort::kDigits * 8;
+        std::size_t const look_tgt = (std::size_t)tgt_tiles * rsort::kDigits * 8;
+        std::size_t const zero_bytes = head + look_src + look_tgt;
+        static_assert( ( kHistWords + 4 * rsort::kMaxPasses ) * 4 % 16 == 0,
+                       "uint4 clearing" );
+        DeviceBuffer<uint4> state( ( zero_bytes + look_src + look_tgt ) / 16, s );
+        char *const st = reinterpret_cast<char *>( state.get() );
+        uint32_t *const hist = reinterpret_cast<uint32_t *>( st );
+        uint32_t *const tickets = hist + kHistWords;
+        uint64_t *const look0 = reinterpret_cast<uint64_t *>( st + head );
+        uint64_t *const look1 = reinterpret_cast<uint64_t *>( st + zero_bytes );
 
-    rsort::PassArgs pa;
-    pa.tickets = tickets;
-    rsort::Array &a = pa.a[0];
-    a.keys[0] = scodes.get();
-    a.keys[1] = scodes1.get();
-    a.vals[0] = svals.get();
-    a.vals[1] = svals.get() + n_src;
-    a.vals_out = ids_sorted;
-    a.pos_out = src_pos;
-    a.gather_in[0] = src;
-    a.gather_out[0] = spts;
-    a.gather_bytes[0] = sizeof( V );
-    if ( out.sorted_src && !share )
-    {
-        a.gather_in[1] = out.src4;
-        a.gather_out[1] = out.sorted_src;
-        a.gather_bytes[1] = sizeof( double4 );
+        // scene box of the sources
+        int nparts = static_cast<int>( std::min<int64_t>(
+            1024, std::max<int64_t>( 1, ceil_div( n_src, kBlock ) ) ) );
+        DeviceBuffer<T> partial( 6 * nparts, s );
+        bbox_partial<T, V><<<nparts, kBlock, 0, s>>>(
+            src, n_src, partial.get(), state.get(),
+            static_cast<int64_t>( zero_bytes / 16 ) );
+        bbox_final<T><<<1, kBlock, 0, s>>>( partial.get(), nparts, box.get() );
+        DTKX_HIP( hipGetLastError() );
+
+        // Hilbert codes of both point sets (the targets' order only has to be
+        // local, so their top 48 bits do) with every pass's digit counts
+        DeviceBuffer<uint64_t> scodes1( n_src, s );
+        DeviceBuffer<uint64_t> tcodes( n_tgt, s ), tcodes1( n_tgt, s );
+        curve_hist_kernel<T, V><<<src_tiles + tgt_tiles, rsort::kThreads, 0, s>>>(
+            src, n_src, tgt, n_tgt, box.get(), nullptr, nullptr, src_tiles,
+            scodes.get(), tcodes.get(), hist );
+        DTKX_HIP( hipGetLastError() );
+
+        DeviceBuffer<int32_t> svals( 2 * n_src, s ), tvals( 2 * n_tgt, s );
+
+        rsort::PassArgs pa;
+        pa.tickets = tickets;
+        rsort::Array &a = pa.a[0];
+        a.keys[0] = scodes.get();
+        a.keys[1] = scodes1.get();
+        a.vals[0] = svals.get();
+        a.vals[1] = svals.get() + n_src;
+        a.vals_out = ids_sorted;
+        a.pos_out = src_pos;
+        a.gather_in[0] = src;
+        a.gather_out[0] = spts;
+        a.gather_bytes[0] = sizeof( V );
+        if ( out.sorted_src && !share )
+        {
+            a.gather_in[1] = out.src4;
+            a.gather_out[1] = out.sorted_src;
+            a.gather_bytes[1] = sizeof( double4 );
+        }
+        a.hist = hist;
+        a.look[0] = look0;
+        a.look[1] = look1;
+        a.n = n_src;
+        a.tiles = src_tiles;
+        a.passes = kSrcPasses;
+        a.key_bits = kSrcKeyBits;
+        a.key_bytes = 8;
+        a.keep_keys = true;
+        rsort::Array &b = pa.a[1];
+        if ( n_tgt > 0 )
+        {
+            b.keys[0] = tcodes.get();
+            b.keys[1] = tcodes1.get();
+            b.vals[0] = tvals.get();
+            b.vals[1] = tvals.get() + n_tgt;
+            b.vals_out = order;
+            b.pos_out = out.query_pos;
+            b.hist = hist + kSrcPasses * rsort::kDigits;
+            b.look[0] = look0 + (std::size_t)src_tiles * rsort::kDigits;
+            b.look[1] = look1 + (std::size_t)src_tiles * rsort::kDigits;
+            b.n = n_tgt;
+            b.tiles = tgt_tiles;
+            b.passes = kTgtPasses;
+            b.key_bits = kTgtKeyBits;
+            b.key_bytes = 8;
+        }
+        rsort::sort( pa, s );
+        // the sorted codes are back in scodes after an even number of passes
+        static_assert( kSrcPasses % 2 == 0, "sorted codes in scodes" );
     }
-    a.hist = hist;
-    a.look[0] = look0;
-    a.look[1] = look1;
-    a.n = n_src;
-    a.tiles = src_tiles;
-    a.passes = kSrcPasses;
-    a.key_bits = kSrcKeyBits;
-    a.key_bytes = 8;
-    a.keep_keys = true;
-    rsort::Array &b = pa.a[1];
-    if ( n_tgt > 0 )
-    {
-        b.keys[0] = tcodes.get();
-        b.keys[1] = tcodes1.get();
-        b.vals[0] = tvals.get();
-        b.vals[1] = tvals.get() + n_tgt;
-        b.vals_out = order;
-        b.pos_out = out.query_pos;
-        b.hist = hist + kSrcPasses * rsort::kDigits;
-        b.look[0] = look0 + (std::size_t)src_tiles * rsort::kDigits;
-        b.look[1] = look1 + (std::size_t)src_tiles * rsort::kDigits;
-        b.n = n_tgt;
-        b.tiles = tgt_tiles;
-        b.passes = kTgtPasses;
-        b.key_bits = kTgtKeyBits;
-        b.key_bytes = 8;
-    }
-    rsort::sort( pa, s );
-    // the sorted codes are back in scodes after an even number of passes
-    static_assert( kSrcPasses % 2 == 0, "sorted codes in scodes" );
 
     if ( n_tgt == 0 )
         return;

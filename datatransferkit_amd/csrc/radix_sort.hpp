@@ -155,6 +155,26 @@ __device__ inline uint32_t lanes_below( uint64_t m )
         __builtin_amdgcn_mbcnt_lo( static_cast<uint32_t>( m ), 0u ) );
 }
 
+// The lanes among `ok` whose digit (8 bits) equals this lane's: one ballot a
+// bit, each taken as it is or inverted by the lane's own bit spread over a
+// word, so that a bit costs four vector instructions (a choice of the ballot
+// or its complement costs eight, and this is most of a pass' arithmetic).
+__device__ inline uint64_t same_digit( uint32_t d, uint64_t ok )
+{
+    uint32_t lo = static_cast<uint32_t>( ok ),
+             hi = static_cast<uint32_t>( ok >> 32 );
+#pragma unroll
+    for ( int b = 0; b < 8; ++b )
+    {
+        uint32_t const bit =
+            static_cast<uint32_t>( static_cast<int32_t>( d << ( 31 - b ) ) >> 31 );
+        uint64_t const bal = __ballot( bit != 0 );
+        lo &= ~( static_cast<uint32_t>( bal ) ^ bit );
+        hi &= ~( static_cast<uint32_t>( bal >> 32 ) ^ bit );
+    }
+    return ( static_cast<uint64_t>( hi ) << 32 ) | lo;
+}
+
 __device__ inline uint32_t wave_inclusive_scan( uint32_t v )
 {
     int const lane = threadIdx.x & 63;
@@ -254,15 +274,8 @@ __device__ void sort_tile( Array const &A, int pass, int tile, Smem &sm )
     {
         bool const ok = w0 + s * 64 + lane < A.n;
         uint32_t const d = static_cast<uint32_t>( key[s] >> shift ) & dmask;
-        uint64_t m = __ballot( ok );
-#pragma unroll
-        for ( int b = 0; b < 8; ++b )
-            if ( b < nbits )
-            {
-                bool const bit = ( d >> b ) & 1u;
-                uint64_t const bal = __ballot( bit );
-                m &= bit ? bal : ~bal;
-            }
+        // (bits past nbits are 0 in every digit)
+        uint64_t const m = same_digit( d, __ballot( ok ) );
         uint32_t const below = lanes_below( m );
         uint32_t prior = 0;
         if ( ok )
