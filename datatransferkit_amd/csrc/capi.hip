@@ -80,8 +80,6 @@ struct dtkx_mls
     // trow the inverse), columns as curve positions of the sources
     // (position p: source perm[p]); empty buffers mean caller order
     dtkx::DeviceBuffer<int32_t> indices, order, trow, perm, spos;
-    // create only: each row's largest neighbour distance (FP32 bulk)
-    dtkx::DeviceBuffer<float> row_max;
     dtkx::DeviceBuffer<double> coeffs;
     // per-row pseudo-inverse, packed upper triangle (store_pinv)
     dtkx::DeviceBuffer<double> pinv;
@@ -122,16 +120,6 @@ struct dtkx_mls
         return g;
     }
 };
-
-// 1: the FP32-bulk setup takes each row's radius from the search's k-th
-// distance instead of a pass over the neighbours. That distance is formed
-// from float-rounded absolute coordinates, so far from the origin it is
-// off by the coordinates' rounding: on a shell of radius 1 with k = 32
-// (neighbours ~4e-3 apart) the FP32-bulk error against FP64 rose from
-// 2.3e-7 to 1.04e-6; at the 1M x 1M cube it saved 2.7 % of a step.
-#ifndef DTKX_FP32_KNN_RADIUS
-#define DTKX_FP32_KNN_RADIUS 0
-#endif
 
 namespace
 {
@@ -284,23 +272,18 @@ __global__ void offsets_kernel( int32_t *off, int64_t n, int kk )
         off[i] = (int32_t)( i * kk );
 }
 
-__global__ void to_f32_kernel( double const *a, float *b, int64_t n )
-{
-    int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if ( i < n )
-        b[i] = (float)a[i];
-}
-
 // Create counters: the setup's four (underdetermined, unconverged,
 // rotations, eigen fallbacks) and the search's re-run count, read back
 // together at the end of the create.
 constexpr int kCounters = 5;
 
-// Shared tail of the two create paths: neighbours are in h->indices.
-void run_setup( dtkx_mls *h, unsigned long long *counters_d )
+// Shared tail of the two create paths: neighbours are in h->indices
+// (by_distance: as the search orders them).
+void run_setup( dtkx_mls *h, unsigned long long *counters_d, bool by_distance )
 {
     dtkx::SetupParams p;
     p.m = h->m;
+    p.by_distance = by_distance;
     p.kk = h->kk;
     p.rbf = h->opts.rbf;
     p.geometry = h->opts.geometry;
@@ -315,7 +298,6 @@ void run_setup( dtkx_mls *h, unsigned long long *counters_d )
         // the FP32-bulk form uses the cyclic solver unless Cholesky is asked
         p.max_rot = h->opts.max_rotations; // sweeps; 0 = default
         bool const f32 = h->opts.precision == DTKX_PRECISION_FP32_BULK;
-        p.row_max = DTKX_FP32_KNN_RADIUS && f32 ? h->row_max.get() : nullptr;
         auto *setup = h->opts.solver == DTKX_SOLVER_CHOLESKY
                           ? &dtkx::setup_fast
                           : &dtkx::setup_cyclic;
@@ -510,13 +492,6 @@ int dtkx_mls_create( const double *src_xyz, int64_t n_src,
             dtkx::KnnOutput kout;
             h->perm.resize( n_src, h->stream );
             h->spos.resize( n_src, h->stream );
-            // the FP32-bulk setup may take its radius from the search
-            if ( DTKX_FP32_KNN_RADIUS &&
-                 opts->precision == DTKX_PRECISION_FP32_BULK )
-            {
-                h->row_max.resize( n_tgt, h->stream );
-                kout.row_max = h->row_max.get();
-            }
             kout.indices = h->indices.get();
             kout.query_order = h->order.get();
             kout.src_perm = h->perm.get();
@@ -545,8 +520,7 @@ int dtkx_mls_create( const double *src_xyz, int64_t n_src,
                                   h->stream );
             h->src_d = std::move( sorted );
             ev.mark( 1 );
-            run_setup( h.get(), counters.get() );
-            h->row_max = {};
+            run_setup( h.get(), counters.get(), true );
             ev.mark( 2 );
         }
         finish_create( h.get(), std::move( counters ), std::move( events ) );
@@ -597,7 +571,7 @@ int dtkx_mls_create_with_neighbors( const double *src_xyz, int64_t n_src,
         if ( n_tgt > 0 )
         {
             events->mark( 1 );
-            run_setup( h.get(), counters.get() );
+            run_setup( h.get(), counters.get(), false );
             events->mark( 2 );
         }
         finish_create( h.get(), std::move( counters ), std::move( events ) );
@@ -1479,7 +1453,6 @@ struct dtkx_mls_batch
         int group_size; // classical solver; 0 until chosen
     };
     std::vector<Group> groups;
-    dtkx::DeviceBuffer<float> row_max;
     // [0..3] the setup's counters, [4] the search's overflow count (int32)
     dtkx::DeviceBuffer<unsigned long long> counters;
     // apply: gathered values and the per-problem pointer arrays the
@@ -1591,7 +1564,6 @@ int autotune_group( dtkx_mls_batch *b, dtkx::SetupParams p, double4 const *src,
 void enqueue_build( dtkx_mls_batch *b, StageEvents *ev )
 {
     hipStream_t const s = b->stream;
-    int const P = b->n_prob;
     int64_t const ns = b->n_src, nt = b->n_tgt;
     dtkx_mls_options const &o = b->opts;
     dtkx::zero_async( b->counters.get(), 5 * sizeof( uint64_t ), s );
@@ -1609,7 +1581,6 @@ void enqueue_build( dtkx_mls_batch *b, StageEvents *ev )
     ko.src_pos = b->pos.get();
     ko.row_off = b->row_off.get();
     ko.indices = b->indices.get();
-    ko.row_max = b->row_max.get(); // null unless the FP32-bulk radius
     dtkx::KnnInfo info;
     info.n_overflow_dev = reinterpret_cast<int32_t *>( b->counters.get() + 4 );
     if ( ev && nt > 0 )
@@ -1651,7 +1622,7 @@ void enqueue_build( dtkx_mls_batch *b, StageEvents *ev )
         if ( cyclic )
         {
             p.max_rot = o.max_rotations;
-            p.row_max = b->row_max.get();
+            p.by_distance = true;
             auto *setup = o.solver == DTKX_SOLVER_CHOLESKY ? &dtkx::setup_fast
                                                             : &dtkx::setup_cyclic;
             setup( src_d.get(), tgt_d.get(), g.r1, b->indices.get(),
@@ -1839,10 +1810,6 @@ int dtkx_mls_batch_create( int32_t n_problems, const dtkx_mls_problem *problems,
             b->coeffs32.resize( std::max<int64_t>( nnz, 1 ), s );
         else
             b->coeffs.resize( std::max<int64_t>( nnz, 1 ), s );
-        // the FP32-bulk setup may take its radius from the search
-        if ( DTKX_FP32_KNN_RADIUS &&
-             opts->precision == DTKX_PRECISION_FP32_BULK && nt > 0 )
-            b->row_max.resize( nt, s );
         kb.n_problems = P;
         kb.src_off = b->src_off.get();
         kb.src_prob = b->src_prob.get();

@@ -778,8 +778,6 @@ struct QueryArgs
     double *out_dist = nullptr;
     // curve layout: row r written at row r with indices as positions
     int32_t const *src_pos = nullptr;
-    // nullable: row r's largest neighbour distance, written at row r
-    float *row_max = nullptr;
     // LDS-stack launch: rows whose descent would push past the LDS stack
     // are listed here (and written by the re-run) instead of finished
     int32_t *overflow_rows = nullptr;
@@ -929,8 +927,6 @@ __device__ inline void query_row( QueryArgs<T> const &a, int64_t const qi,
             a.out_idx[base + j] = a.src_pos ? a.src_pos[id] : id;
             if ( a.out_dist )
                 a.out_dist[base + j] = best.distance( j );
-            if ( a.row_max && j == kk - 1 )
-                a.row_max[r] = (float)best.distance( j );
         }
 }
 
@@ -1418,7 +1414,6 @@ void knn_impl( void const *src_v, int64_t n_src, void const *tgt_v,
     qa.out_idx = out.indices;
     qa.out_dist = out.dist;
     qa.src_pos = out.morton_layout ? src_pos : nullptr;
-    qa.row_max = out.morton_layout ? out.row_max : nullptr;
     if ( info && info->query_begin )
         DTKX_HIP( hipEventRecord( info->query_begin, s ) );
     run_queries<T>( {{0, n_tgt, kk}}, qa, n_tgt, (double)n_src / (double)n_tgt,
@@ -1735,7 +1730,6 @@ void knn_batched_impl( void const *src_v, int64_t n_src, void const *tgt_v,
     qa.row_off = out.row_off;
     qa.out_idx = out.indices;
     qa.src_pos = out.src_pos;
-    qa.row_max = out.row_max;
     run_queries<T>( b.launches, qa, n_tgt, (double)n_src / (double)n_tgt,
                     grouped ? &levels : nullptr, spts.get(), out.src_perm,
                     build_tree, info, s );

@@ -43,9 +43,6 @@ struct KnnOutput
     int32_t *src_perm = nullptr;
     int32_t *src_pos = nullptr;
     bool morton_layout = false;
-    // nullable, curve layout: each row's largest neighbour distance (the
-    // k-th, as the search computes it)
-    float *row_max = nullptr;
     // nullable: the inverse of query_order (query_pos[target] = row)
     int32_t *query_pos = nullptr;
     // nullable: sorted_src[position] = src4[source], a double4 copy of the
@@ -99,7 +96,6 @@ struct KnnBatchOutput
     int32_t *src_pos = nullptr;  // [n_src] source -> position
     int64_t *row_off = nullptr;  // [n_tgt + 1]
     int32_t *indices = nullptr;  // [nnz]
-    float *row_max = nullptr;    // nullable [n_tgt]: largest distance per row
 };
 
 void knn_search_batched( int geometry, void const *src, int64_t n_src,

@@ -1158,7 +1158,7 @@ __global__ void __launch_bounds__( 64 )
                 if ( e >= mine )
                     pos[e] = (int32_t)beg;
             }
-            if ( a.out_dist || a.row_max )
+            if ( a.out_dist )
             {
                 V const tq = a.tgt[rt];
                 T const qq[3] = {tq.x, tq.y, tq.z};
@@ -1168,10 +1168,8 @@ __global__ void __launch_bounds__( 64 )
                     V const p = g.pts[pos[e]];
                     T const b[3] = {p.x, p.y, p.z};
                     T const d = sqrt_rn( point_sq( qq, b ) );
-                    if ( a.out_dist && e < mine )
+                    if ( e < mine )
                         a.out_dist[base + sl * E + e] = (double)d;
-                    if ( a.row_max && e == mine - 1 )
-                        a.row_max[r] = (float)d;
                     if ( e % 4 == 3 )
                         __builtin_amdgcn_sched_barrier( 0 );
                 }
@@ -1233,8 +1231,6 @@ __global__ void __launch_bounds__( 64 )
                         a.out_idx[cr_base + j] = a.src_pos ? a.src_pos[id] : id;
                         if ( a.out_dist )
                             a.out_dist[cr_base + j] = SK::distance( fk[e] );
-                        if ( a.row_max && j == kk - 1 )
-                            a.row_max[cr_row] = (float)SK::distance( fk[e] );
                     }
                 }
             }

@@ -31,9 +31,8 @@ struct SetupParams
     // i < *n_rows (device count, at most n_tgt - row0) instead of a range
     int32_t const *rows = nullptr;
     int32_t const *n_rows = nullptr;
-    // FP32 bulk (nullable): each row's largest neighbour distance from the
-    // kNN, which then gives the radius without a pass over the neighbours
-    float const *row_max = nullptr;
+    // every row is in the search's order, ascending by distance
+    bool by_distance = false;
     // cyclic solver over a row list (nullable): rows whose eigenvalues all
     // pass the truncation test are appended here (device count n_refine)
     int32_t *refine_rows = nullptr;

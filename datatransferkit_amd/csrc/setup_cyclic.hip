@@ -53,7 +53,7 @@ __device__ __forceinline__ SystemRow
                     int32_t const *__restrict__ indices,
                     int32_t const *__restrict__ order,
                     int64_t const *__restrict__ row_off, int kk_uniform,
-                    int rbf, int geometry, float const *__restrict__ row_max,
+                    int rbf, int geometry, bool by_distance,
                     double *A )
 {
     using S = SymIdx<M>;
@@ -66,18 +66,7 @@ __device__ __forceinline__ SystemRow
     int32_t const *nbr = indices + rbeg;
     double4 const tp = valid ? tgt[t] : double4{0, 0, 0, 0};
 
-    double dmax = 10. * DBL_EPSILON;
-    if ( F32 && row_max )
-    {
-        double const d = valid ? (double)row_max[slot] : 0.0;
-        dmax = d > dmax ? d : dmax;
-    }
-    else if ( valid )
-        for ( int l = 0; l < kk; ++l )
-        {
-            double const d = nbr_distance<M, F32>( geometry, src[nbr[l]], tp );
-            dmax = d > dmax ? d : dmax;
-        }
+    double const dmax = row_reach<M, F32>( geometry, by_distance, src, nbr, kk, tp );
     double const radius = F32 ? (double)( 1.1f * (float)dmax ) : 1.1 * dmax;
 
 #pragma unroll
@@ -146,7 +135,7 @@ __device__ __forceinline__ void
                          float *__restrict__ coeffs32,
                          double *__restrict__ pinv_out,
                          unsigned long long *__restrict__ counters,
-                         float const *__restrict__ row_max,
+                         bool by_distance,
                          int32_t *__restrict__ refine_rows,
                          int32_t *__restrict__ n_refine, bool screened )
 {
@@ -168,7 +157,7 @@ __device__ __forceinline__ void
     double A[S::size];
     SystemRow const sr =
         system_moments<M, F32>( valid, slot, src, tgt, indices, order, row_off,
-                                kk_uniform, rbf, geometry, row_max, A );
+                                kk_uniform, rbf, geometry, by_distance, A );
     int const kk = sr.kk;
     int64_t const rbeg = sr.rbeg;
     int32_t const *nbr = sr.nbr;
@@ -346,7 +335,7 @@ __global__ void __launch_bounds__( kBlock )
                          float *__restrict__ coeffs32,
                          double *__restrict__ pinv_out,
                          unsigned long long *__restrict__ counters,
-                         float const *__restrict__ row_max,
+                         bool by_distance,
                          int32_t *__restrict__ refine_rows,
                          int32_t *__restrict__ n_refine, bool screened )
 {
@@ -355,7 +344,7 @@ __global__ void __launch_bounds__( kBlock )
         cyclic_system<M, H, F32, STORE>(
             tile * SPB + threadIdx.x / H, src, tgt, n_tgt, indices, order, row0,
             row_off, rows, n_rows, kk_uniform, rbf, geometry, truncation, rcond,
-            max_sweeps, coeffs, coeffs32, pinv_out, counters, row_max,
+            max_sweeps, coeffs, coeffs32, pinv_out, counters, by_distance,
             refine_rows, n_refine, screened );
     };
     if constexpr ( LIST )
@@ -407,7 +396,7 @@ void launch_cyclic( double4 const *src, double4 const *tgt, int64_t n_tgt,
                                      p.row_off, p.rows, p.n_rows, p.kk,
                                      p.rbf, p.geometry, p.truncation, p.rcond,
                                      sweeps, coeffs, coeffs32, pinv, counters,
-                                     p.row_max, p.refine_rows, p.n_refine,
+                                     p.by_distance, p.refine_rows, p.n_refine,
                                      p.screened );
     };
     using T = std::true_type;
@@ -441,7 +430,7 @@ __global__ void __launch_bounds__( kBlock )
                          int rbf, int geometry, int truncation, double rcond,
                          int max_sweeps,
                          unsigned long long *__restrict__ counters,
-                         float const *__restrict__ row_max,
+                         bool by_distance,
                          int32_t *__restrict__ refine_rows,
                          int32_t *__restrict__ n_refine,
                          int32_t *__restrict__ full_rows,
@@ -459,7 +448,7 @@ __global__ void __launch_bounds__( kBlock )
         double A[S::size];
         (void)system_moments<M, F32>( valid, slot, src, tgt, indices, order,
                                       row_off, kk_uniform, rbf, geometry,
-                                      row_max, A );
+                                      by_distance, A );
         double no_v[1];
         int sweeps = 0;
         bool done = !valid || converged<M>( A );
@@ -509,7 +498,7 @@ void setup_screen( double4 const *src, double4 const *tgt, int64_t n_tgt,
             <<<blocks, kBlock, 0, s>>>(
                 src, tgt, indices, order, p.row_off, p.rows, p.n_rows, p.kk,
                 p.rbf, p.geometry, p.truncation, p.rcond, sweeps, counters,
-                p.row_max, p.refine_rows, p.n_refine, full_rows, n_full );
+                p.by_distance, p.refine_rows, p.n_refine, full_rows, n_full );
     };
     using T = std::true_type;
     using F = std::false_type;

@@ -67,7 +67,7 @@ __global__ void __launch_bounds__( kBlock, 2 )
                            int32_t *__restrict__ fallback,
                            int32_t *__restrict__ n_fallback,
                            unsigned long long *__restrict__ counters,
-                           float const *__restrict__ row_max )
+                           bool by_distance )
 {
     using S = SymIdx<M>;
     __shared__ RowShare<M> sh;
@@ -92,29 +92,8 @@ __global__ void __launch_bounds__( kBlock, 2 )
             p[j] = src[nbr[l0 + j < kk ? l0 + j : kk - 1]];
     };
 
-    // radius (Impl.hpp:118-134); the FP32-bulk form may take the largest
-    // distance from the kNN
-    double dmax = 10. * DBL_EPSILON;
-    if ( F32 && row_max )
-    {
-        double const d = valid ? (double)row_max[slot] : 0.0;
-        dmax = d > dmax ? d : dmax;
-    }
-    else
-    {
-        for ( int l0 = 0; l0 < kk; l0 += kGather )
-        {
-            double4 p[kGather];
-            gather( l0, p );
-#pragma unroll
-            for ( int j = 0; j < kGather; ++j )
-            {
-                double const d = nbr_distance<M, F32>( geometry, p[j], tp );
-                // a repeated last entry changes nothing
-                dmax = d > dmax ? d : dmax;
-            }
-        }
-    }
+    // radius (Impl.hpp:118-134)
+    double const dmax = row_reach<M, F32>( geometry, by_distance, src, nbr, kk, tp );
     double const radius = F32 ? (double)( 1.1f * (float)dmax ) : 1.1 * dmax;
 
     // moments, upper triangle
@@ -259,7 +238,7 @@ __global__ void __launch_bounds__( kBlock )
                    int rbf, int geometry, int32_t const *__restrict__ rows,
                    int32_t const *__restrict__ n_rows,
                    double *__restrict__ coeffs, float *__restrict__ coeffs32,
-                   float const *__restrict__ row_max,
+                   bool by_distance,
                    int32_t *__restrict__ full_rows,
                    int32_t *__restrict__ n_full )
 {
@@ -275,19 +254,8 @@ __global__ void __launch_bounds__( kBlock )
             row_off ? (int)( row_off[slot + 1] - rbeg ) : kk_uniform;
         int32_t const *nbr = indices + rbeg;
         double4 const tp = tgt[t];
-        double dmax = 10. * DBL_EPSILON;
-        if ( F32 && row_max )
-        {
-            double const d = (double)row_max[slot];
-            dmax = d > dmax ? d : dmax;
-        }
-        else
-            for ( int l = 0; l < kk; ++l )
-            {
-                double const d =
-                    nbr_distance<M, F32>( geometry, src[nbr[l]], tp );
-                dmax = d > dmax ? d : dmax;
-            }
+        double const dmax =
+            row_reach<M, F32>( geometry, by_distance, src, nbr, kk, tp );
         double const radius =
             F32 ? (double)( 1.1f * (float)dmax ) : 1.1 * dmax;
         double A[S::size];
@@ -355,7 +323,7 @@ void launch_fast( double4 const *src, double4 const *tgt, int64_t n_tgt,
             <<<grid, block, 0, s>>>( src, tgt, n_tgt, indices, order, p.row0,
                                      p.row_off, p.kk, p.rbf, p.geometry,
                                      p.truncation, p.rcond, coeffs, coeffs32,
-                                     pinv, list, count, counters, p.row_max );
+                                     pinv, list, count, counters, p.by_distance );
     };
     using T = std::true_type;
     using F = std::false_type;
@@ -430,7 +398,7 @@ void setup_fast( double4 const *src, double4 const *tgt, int64_t n_tgt,
                 <<<blocks, kBlock, 0, s>>>(
                     src, tgt, indices, order, p.row_off, p.kk, p.rbf,
                     p.geometry, rlist.get(), counts.get(), coeffs, coeffs32,
-                    p.row_max, flist.get(), counts.get() + 2 );
+                    p.by_distance, flist.get(), counts.get() + 2 );
         };
         using T = std::true_type;
         using F = std::false_type;
