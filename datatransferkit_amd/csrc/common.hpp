@@ -105,31 +105,9 @@ void cache_release();
 hipStream_t library_stream();
 // A second stream of the library's own on the current device (default
 // priority, non-blocking: it does not wait for the null stream), created
-// on first use and kept: forked work, and reads that must wait for one
-// event only, not for later work queued on a caller's stream.
+// on first use and kept: reads that must wait for one event only, not for
+// later work queued on a caller's stream.
 hipStream_t side_stream();
-
-// Work forked from stream s onto a stream of the library's own (default
-// priority, non-blocking, one per device, not side_stream()): it first
-// waits for everything queued on s so far, and join() (or the destructor)
-// makes s wait for everything queued on the forked stream since. Buffers
-// the forked work uses are allocated on s before the fork and released on
-// s after the join, so the block cache's stream order holds for them.
-class Fork
-{
-  public:
-    explicit Fork( hipStream_t s );
-    ~Fork();
-    Fork( Fork const & ) = delete;
-    Fork &operator=( Fork const & ) = delete;
-    hipStream_t side() const { return side_; }
-    void join();
-
-  private:
-    hipStream_t main_, side_;
-    hipEvent_t fork_ = nullptr, join_ = nullptr;
-    bool joined_ = false;
-};
 
 // Owning device buffer, move-only. With a stream it draws from the block
 // cache of that stream; without one it uses hipMalloc / hipFree.

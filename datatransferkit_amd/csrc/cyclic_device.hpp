@@ -150,8 +150,15 @@ __device__ inline double nbr_row( int geometry, int rbf, double radius,
 // zero, so the eigenvalues and vectors keep their bits without a branch
 // around the straight-line sweep; only A(p, q), already negligible and read
 // by nothing after convergence, is cleared as usual.
-template <int M, int R, int P_, int Q_>
-__device__ inline void rotate( double *A, double *V, bool skip )
+// KEEP: the tangent goes to kept, one a rotation in sweep order, kLanes apart
+// (sweep_vectors takes them).
+constexpr int kLanes = 64;
+
+template <int M>
+constexpr int rotations = M * ( M - 1 ) / 2;
+
+template <int M, int R, int P_, int Q_, bool KEEP>
+__device__ inline void rotate( double *A, double *V, bool skip, double *kept )
 {
     using S = SymIdx<M>;
     double const apq = A[S::at( P_, Q_ )];
@@ -174,6 +181,8 @@ __device__ inline void rotate( double *A, double *V, bool skip )
     double const s = t * c;
     double const tau = s / ( 1.0 + c );
     double const h = t * apq;
+    if constexpr ( KEEP )
+        kept[( P_ * ( 2 * M - P_ - 1 ) / 2 + Q_ - P_ - 1 ) * kLanes] = t;
     A[S::at( P_, P_ )] = app - h;
     A[S::at( Q_, Q_ )] = aqq + h;
     A[S::at( P_, Q_ )] = 0.0;
@@ -198,24 +207,73 @@ __device__ inline void rotate( double *A, double *V, bool skip )
 }
 
 // one cyclic sweep in row order (0,1), (0,2), ..., (M-2, M-1)
-template <int M, int R, int P_, int Q_>
+template <int M, int R, int P_, int Q_, bool KEEP>
 struct Sweep
 {
-    __device__ static inline void run( double *A, double *V, bool skip )
+    __device__ static inline void run( double *A, double *V, bool skip,
+                                       double *kept )
     {
-        rotate<M, R, P_, Q_>( A, V, skip );
+        rotate<M, R, P_, Q_, KEEP>( A, V, skip, kept );
         if constexpr ( Q_ + 1 < M )
-            Sweep<M, R, P_, Q_ + 1>::run( A, V, skip );
+            Sweep<M, R, P_, Q_ + 1, KEEP>::run( A, V, skip, kept );
         else if constexpr ( P_ + 2 < M )
-            Sweep<M, R, P_ + 1, P_ + 2>::run( A, V, skip );
+            Sweep<M, R, P_ + 1, P_ + 2, KEEP>::run( A, V, skip, kept );
     }
 };
 
-template <int M, int R>
-__device__ inline void sweep_all( double *A, double *V, bool skip )
+template <int M, int R, bool KEEP = false>
+__device__ inline void sweep_all( double *A, double *V, bool skip,
+                                  double *kept = nullptr )
 {
     if constexpr ( M >= 2 )
-        Sweep<M, R, 0, 1>::run( A, V, skip );
+        Sweep<M, R, 0, 1, KEEP>::run( A, V, skip, kept );
+}
+
+// V <- V J_1 ... J_n for a sweep's rotations from their kept tangents, with
+// rotate's operations and so its bits. The tangents are loaded a group ahead
+// of their use.
+template <int M>
+__device__ inline void sweep_vectors( double *V, double const *kept )
+{
+    constexpr int kN = rotations<M>, kG = kN < 5 ? kN : 5;
+    if constexpr ( M >= 2 )
+    {
+        double next[kG];
+#pragma unroll
+        for ( int i = 0; i < kG; ++i )
+            next[i] = kept[i * kLanes];
+        double cur[kG];
+        int i = 0;
+#pragma unroll
+        for ( int p = 0; p < M - 1; ++p )
+#pragma unroll
+            for ( int q = p + 1; q < M; ++q, ++i )
+            {
+                if ( i % kG == 0 )
+                {
+#pragma unroll
+                    for ( int g = 0; g < kG; ++g )
+                        cur[g] = next[g];
+#pragma unroll
+                    for ( int g = 0; g < kG; ++g )
+                        if ( i + kG + g < kN )
+                            next[g] = kept[( i + kG + g ) * kLanes];
+                }
+                double const t = cur[i % kG];
+                double const c = 1.0 / __builtin_sqrt( fma( t, t, 1.0 ) );
+                double const s = t * c;
+                double const tau = s / ( 1.0 + c );
+#pragma unroll
+                for ( int r = 0; r < M; ++r )
+                {
+                    double const vrp = V[r * M + p];
+                    double const vrq = V[r * M + q];
+                    V[r * M + p] = vrp - s * ( vrq + tau * vrp );
+                    V[r * M + q] = vrq + s * ( vrp - tau * vrq );
+                }
+                __builtin_amdgcn_sched_barrier( 0 );
+            }
+    }
 }
 
 template <int M>

@@ -37,9 +37,9 @@ struct SetupParams
     // pass the truncation test are appended here (device count n_refine)
     int32_t *refine_rows = nullptr;
     int32_t *n_refine = nullptr;
-    // cyclic solver over a list that setup_screen made: the sweeps and
-    // unconverged systems are counted for truncated rows only (the screen
-    // counted the others)
+    // cyclic solver over rows that setup_listed left: the sweeps and
+    // unconverged systems are counted for truncated rows only (it counted
+    // the others)
     bool screened = false;
 };
 
@@ -70,24 +70,24 @@ void setup_cyclic( double4 const *src, double4 const *tgt, int64_t n_tgt,
                    SetupParams const &p, double *coeffs, float *coeffs32,
                    double *pinv, unsigned long long *counters, hipStream_t s );
 
-// Eigenvalue screen of the listed rows p.rows[0 .. *p.n_rows): the cyclic
-// Jacobi of setup_cyclic without eigenvectors (the same rotations of A, so
-// the same eigenvalues, sweeps and convergence). Rows whose eigenvalues all
-// pass the truncation test are appended to p.refine_rows, the others to
-// full_rows; counters[1] and [2] are taken for the first kind. f32: the
-// FP32-bulk form's geometry and weights.
-void setup_screen( double4 const *src, double4 const *tgt, int64_t n_tgt,
+// The listed rows p.rows[0 .. *p.n_rows) by their eigenvalues: the cyclic
+// Jacobi of setup_cyclic (the same rotations of A, so the same eigenvalues,
+// sweeps and convergence) without V. Rows whose eigenvalues all pass the
+// truncation test are appended to p.refine_rows; the others' coefficients
+// are written, but for the few appended to full_rows, which its counters
+// leave out. coeffs32 as in setup_cyclic; *queue is zero before.
+void setup_listed( double4 const *src, double4 const *tgt, int64_t n_tgt,
                    int32_t const *indices, int32_t const *order,
-                   SetupParams const &p, bool f32, int32_t *full_rows,
-                   int32_t *n_full, unsigned long long *counters,
-                   hipStream_t s );
+                   SetupParams const &p, double *coeffs, float *coeffs32,
+                   int32_t *full_rows, int32_t *n_full, int32_t *queue,
+                   unsigned long long *counters, hipStream_t s );
 
 // Certified Cholesky fast path (DTKX_SOLVER_CHOLESKY): each system is
 // factored A = U^T U in FP64; when the bound lambda_min(A) >= 1 / |U^-1|_F^2
 // proves that no eigenvalue reaches the truncation threshold (with a margin
 // for the eigen-solver's rounding), A^+ = A^-1 and a0 = U^-1 U^-T e_0 is
 // used. The other systems are listed; those of them with no eigenvalue
-// below the threshold (setup_screen) have A^+ = A^-1 as well and are solved
+// below the threshold (setup_listed) have A^+ = A^-1 as well and are solved
 // again by Cholesky, whose rounding error follows the equilibrated matrix,
 // not the eigen-decomposition's eps |A| / lambda (measured on 10-neighbour
 // quadratic systems: 5e-10 against 2e-4 from the operator in extended

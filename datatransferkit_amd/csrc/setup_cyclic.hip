@@ -22,6 +22,7 @@
 #include "cyclic_device.hpp"
 #include "setup.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace dtkx
@@ -33,10 +34,8 @@ using namespace cyc;
 constexpr int kBlock = 64;
 
 // One listed or ranged row's neighbour list, target and radius
-// (Impl.hpp:118-134: the largest neighbour distance, for the FP32-bulk form
-// possibly taken from the kNN), with its moments (upper triangle) written
-// to A. Shared by the eigen-solver and the eigenvalue screen, so both form
-// the same bits.
+// (row_reach), with its moments (upper triangle) written
+// to A. Shared by the eigen-solver's two kernels, so both form the same bits.
 struct SystemRow
 {
     int64_t rbeg;
@@ -319,7 +318,6 @@ __device__ __forceinline__ void
 // device) runs a bounded grid that strides over the list, so an empty list
 // costs a few thousand empty blocks, not one per row of the operator.
 constexpr int kListBlocks = 2048;
-constexpr int kScreenBlocks = 16384;
 
 template <int M, int H, bool F32, bool STORE, bool LIST>
 __global__ void __launch_bounds__( kBlock )
@@ -358,15 +356,6 @@ __global__ void __launch_bounds__( kBlock )
         for ( int64_t tile = blockIdx.x; tile * SPB < n; tile += gridDim.x )
             one( tile );
     }
-    else if ( rows )
-    {
-        // a row list over a grid for its whole capacity: blocks past the
-        // device-side count return at once
-        int64_t const tile = blockIdx.x;
-        if ( tile * SPB >= *n_rows )
-            return;
-        one( tile );
-    }
     else
         one( xcd_tile() );
 }
@@ -378,11 +367,7 @@ void launch_cyclic( double4 const *src, double4 const *tgt, int64_t n_tgt,
                     double *pinv, unsigned long long *counters, hipStream_t s )
 {
     int const sweeps = p.max_rot > 0 ? static_cast<int>( p.max_rot ) : 30;
-    // A screened list (the rows the eigenvalue screen found truncated, a
-    // few percent of the listed rows) runs without the strided loop, whose
-    // registers spilled (364 bytes a lane for m = 10), over a grid for the
-    // list's whole capacity; other lists stride over a bounded grid.
-    bool const strided = p.rows && !p.screened;
+    bool const strided = p.rows != nullptr;
     int64_t blocks = ceil_div( n_tgt - p.row0, kBlock / H );
     if ( strided )
         blocks = blocks < kListBlocks ? blocks : kListBlocks;
@@ -408,19 +393,31 @@ void launch_cyclic( double4 const *src, double4 const *tgt, int64_t n_tgt,
     DTKX_HIP( hipGetLastError() );
 }
 
-// Eigenvalues only, one lane per listed row: the cyclic Jacobi on A
-// without eigenvectors. A rotation of A never reads V, and a converged
-// system's rotations are exact no-ops whatever its wave, so the
-// eigenvalues, the sweep count and the convergence flag are those
-// cyclic_system computes for the row. Rows whose eigenvalues all pass the
-// truncation test go to refine_rows (solved again by Cholesky, with their
-// sweeps and convergence counted here), the others to full_rows (the
-// eigen-solver with eigenvectors). Most rows the Cholesky setup lists are
-// of the first kind: on 10-neighbour quadratic systems (1M targets), 466k
-// of the 493k listed rows.
+// Listed rows, one lane each: the cyclic Jacobi of cyclic_system on A, whose
+// rotations never read V. Rows whose eigenvalues all pass the truncation test
+// go to refine_rows (solved again by Cholesky). For the others V is formed
+// afterwards, in the registers that A leaves, from the rotations' tangents
+// (kept for each wave and sweep; the last region takes all later sweeps and
+// is not read). The operations are cyclic_system's and a converged system's
+// rotations exact no-ops whatever its wave, so all results are its bit for
+// bit. Truncated rows that need more sweeps than are kept, or that hold a
+// value that is not finite, go to full_rows (cyclic_system, from their start).
+//
+// Bound by the FP64 of the rotations (a division chain and 64 fused
+// operations on A, 45 a sweep). A and V together (155 doubles) took two lanes
+// a system that both rotated A, at one wave a SIMD, after a first pass over
+// the list for the eigenvalues: a transfer with 300,000 such rows of 32 (a
+// shell) 2.26 ms, now 1.45. Measured on the way: the stores of the tangents
+// cost nothing beside the rotations; tiles from a queue instead of a stride
+// 797 -> 688 us of the kernel, as 4,688 tiles over 2,048 blocks leave some
+// with a third; gathers four neighbours at a time gave nothing.
+constexpr int kKeptSweeps = 10;
+// two waves a SIMD at this kernel's registers
+constexpr int kListedBlocks = 2048;
+
 template <int M, bool F32>
-__global__ void __launch_bounds__( kBlock )
-    eigen_screen_kernel( double4 const *__restrict__ src,
+__global__ void __launch_bounds__( kBlock, 2 )
+    eigen_listed_kernel( double4 const *__restrict__ src,
                          double4 const *__restrict__ tgt,
                          int32_t const *__restrict__ indices,
                          int32_t const *__restrict__ order,
@@ -428,77 +425,139 @@ __global__ void __launch_bounds__( kBlock )
                          int32_t const *__restrict__ rows,
                          int32_t const *__restrict__ n_rows, int kk_uniform,
                          int rbf, int geometry, int truncation, double rcond,
-                         int max_sweeps,
+                         int max_sweeps, double *__restrict__ coeffs,
+                         float *__restrict__ coeffs32,
+                         double *__restrict__ tangents,
                          unsigned long long *__restrict__ counters,
                          bool by_distance,
                          int32_t *__restrict__ refine_rows,
                          int32_t *__restrict__ n_refine,
                          int32_t *__restrict__ full_rows,
-                         int32_t *__restrict__ n_full )
+                         int32_t *__restrict__ n_full,
+                         int32_t *__restrict__ queue )
 {
     using S = SymIdx<M>;
-    // the trip count is uniform over the block (the wave-wide vote); tiles
-    // in dispatch order spread the list's first tiles over the XCDs
+    double *const mine =
+        tangents + (int64_t)blockIdx.x * kKeptSweeps * rotations<M> * kLanes +
+        threadIdx.x;
+    // tiles in dispatch order spread the list's first tiles over the XCDs; a
+    // block's next one comes from the queue (uniform over the block: the
+    // wave-wide vote needs every lane), which ends with the list
     int64_t const n = *n_rows;
-    for ( int64_t tile = blockIdx.x; tile * kBlock < n; tile += gridDim.x )
+    auto next = [&]() {
+        int t = 0;
+        if ( threadIdx.x == 0 )
+            t = atomicAdd( queue, 1 );
+        return (int64_t)gridDim.x + __builtin_amdgcn_readfirstlane( t );
+    };
+    for ( int64_t tile = blockIdx.x; tile * kBlock < n; tile = next() )
     {
         int64_t const li = tile * kBlock + threadIdx.x;
         bool const valid = li < n;
         int64_t const slot = valid ? rows[li] : 0;
         double A[S::size];
-        (void)system_moments<M, F32>( valid, slot, src, tgt, indices, order,
-                                      row_off, kk_uniform, rbf, geometry,
-                                      by_distance, A );
+        SystemRow const sr = system_moments<M, F32>(
+            valid, slot, src, tgt, indices, order, row_off, kk_uniform, rbf,
+            geometry, by_distance, A );
         double no_v[1];
-        int sweeps = 0;
+        int sweeps = 0, pass = 0;
         bool done = !valid || converged<M>( A );
-        for ( int pass = 0; !__all( done ) && pass < max_sweeps; ++pass )
+        for ( ; !__all( done ) && pass < max_sweeps; ++pass )
         {
-            sweep_all<M, 0>( A, no_v, done );
+            int const keep = pass < kKeptSweeps ? pass : kKeptSweeps - 1;
+            sweep_all<M, 0, true>( A, no_v, done,
+                                   mine + keep * rotations<M> * kLanes );
             sweeps += done ? 0 : 1;
             done = done || converged<M>( A );
         }
-        if ( !valid )
-            continue;
         double thr;
-        if ( truncated<M>( A, truncation, rcond, thr ) )
-            full_rows[atomicAdd( n_full, 1 )] = (int32_t)slot;
-        else
-        {
+        bool const under = valid && truncated<M>( A, truncation, rcond, thr );
+        bool finite = true;
+#pragma unroll
+        for ( int k = 0; k < M; ++k )
+            finite = finite && fabs( A[S::at( k, k )] ) <= DBL_MAX;
+        bool const here = under && finite && sweeps < kKeptSweeps;
+        if ( valid && !under )
             refine_rows[atomicAdd( n_refine, 1 )] = (int32_t)slot;
-            if ( counters )
+        if ( under && !here )
+            full_rows[atomicAdd( n_full, 1 )] = (int32_t)slot;
+        if ( counters && valid && ( here || !under ) )
+        {
+            if ( under )
+                atomicAdd( counters + 0, 1ull );
+            if ( !done )
+                atomicAdd( counters + 1, 1ull );
+            atomicAdd( counters + 2, (unsigned long long)sweeps );
+        }
+        if ( !here )
+            continue;
+        double lambda[M], x[M];
+#pragma unroll
+        for ( int k = 0; k < M; ++k )
+            lambda[k] = A[S::at( k, k )];
+        {
+            double V[M * M];
+#pragma unroll
+            for ( int e = 0; e < M * M; ++e )
+                V[e] = e / M == e % M ? 1.0 : 0.0;
+            for ( int p = 0; p < sweeps; ++p )
+                sweep_vectors<M>( V, mine + p * rotations<M> * kLanes );
+#pragma unroll
+            for ( int r = 0; r < M; ++r )
+                x[r] = 0.0;
+#pragma unroll
+            for ( int k = 0; k < M; ++k )
             {
-                if ( !done )
-                    atomicAdd( counters + 1, 1ull );
-                atomicAdd( counters + 2, (unsigned long long)sweeps );
+                double const w = fabs( lambda[k] ) >= thr ? V[k] / lambda[k] : 0.0;
+#pragma unroll
+                for ( int r = 0; r < M; ++r )
+                    x[r] = fma( w, V[r * M + k], x[r] );
             }
+        }
+        for ( int l = 0; l < sr.kk; ++l )
+        {
+            double P[M];
+            double const phi = nbr_row<M, F32>( geometry, rbf, sr.radius,
+                                                src[sr.nbr[l]], sr.tp, P );
+            double acc = 0.0;
+#pragma unroll
+            for ( int j = 0; j < M; ++j )
+                acc = fma( x[j], P[j], acc );
+            if constexpr ( F32 )
+                coeffs32[sr.rbeg + l] = (float)( acc * phi );
+            else
+                coeffs[sr.rbeg + l] = acc * phi;
         }
     }
 }
 
 } // namespace
 
-void setup_screen( double4 const *src, double4 const *tgt, int64_t n_tgt,
+void setup_listed( double4 const *src, double4 const *tgt, int64_t n_tgt,
                    int32_t const *indices, int32_t const *order,
-                   SetupParams const &p, bool f32, int32_t *full_rows,
-                   int32_t *n_full, unsigned long long *counters,
-                   hipStream_t s )
+                   SetupParams const &p, double *coeffs, float *coeffs32,
+                   int32_t *full_rows, int32_t *n_full, int32_t *queue,
+                   unsigned long long *counters, hipStream_t s )
 {
     DTKX_REQUIRE( p.rows && p.n_rows && p.refine_rows && p.n_refine,
                   DTKX_ERR_INVALID_ARGUMENT );
     if ( n_tgt <= p.row0 )
         return;
     int const sweeps = p.max_rot > 0 ? static_cast<int>( p.max_rot ) : 30;
-    // one wave a block and up to three waves a SIMD: a grid of 2,048
-    // blocks would leave the SIMDs two waves each
-    int64_t blocks = ceil_div( n_tgt - p.row0, kBlock );
-    blocks = blocks < kScreenBlocks ? blocks : kScreenBlocks;
+    int64_t const blocks = std::min<int64_t>(
+        ceil_div( n_tgt - p.row0, kBlock ), kListedBlocks );
     auto run = [&]( auto m, auto f32 ) {
-        eigen_screen_kernel<decltype( m )::value, decltype( f32 )::value>
+        constexpr int kM = decltype( m )::value;
+        DeviceBuffer<double> tangents(
+            std::max<std::size_t>(
+                blocks * kKeptSweeps * rotations<kM> * kLanes, 1 ),
+            s );
+        eigen_listed_kernel<kM, decltype( f32 )::value>
             <<<blocks, kBlock, 0, s>>>(
                 src, tgt, indices, order, p.row_off, p.rows, p.n_rows, p.kk,
-                p.rbf, p.geometry, p.truncation, p.rcond, sweeps, counters,
-                p.by_distance, p.refine_rows, p.n_refine, full_rows, n_full );
+                p.rbf, p.geometry, p.truncation, p.rcond, sweeps, coeffs,
+                coeffs32, tangents.get(), counters, p.by_distance, p.refine_rows,
+                p.n_refine, full_rows, n_full, queue );
     };
     using T = std::true_type;
     using F = std::false_type;
@@ -506,11 +565,11 @@ void setup_screen( double4 const *src, double4 const *tgt, int64_t n_tgt,
     using M4 = std::integral_constant<int, 4>;
     using M10 = std::integral_constant<int, 10>;
     if ( p.m == 1 )
-        f32 ? run( M1{}, T{} ) : run( M1{}, F{} );
+        coeffs32 ? run( M1{}, T{} ) : run( M1{}, F{} );
     else if ( p.m == 4 )
-        f32 ? run( M4{}, T{} ) : run( M4{}, F{} );
+        coeffs32 ? run( M4{}, T{} ) : run( M4{}, F{} );
     else if ( p.m == 10 )
-        f32 ? run( M10{}, T{} ) : run( M10{}, F{} );
+        coeffs32 ? run( M10{}, T{} ) : run( M10{}, F{} );
     else
         DTKX_REQUIRE( p.m == 1 || p.m == 4 || p.m == 10,
                       DTKX_ERR_INVALID_ARGUMENT );

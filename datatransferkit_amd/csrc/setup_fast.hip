@@ -368,54 +368,44 @@ void setup_fast( double4 const *src, double4 const *tgt, int64_t n_tgt,
                       pinv, counters, s );
         return;
     }
-    // otherwise their eigenvalues first: the rows with none below the
-    // threshold have A^+ = A^-1 and are solved again by Cholesky, the
-    // others by the eigen-solver with eigenvectors, on a forked stream at
-    // the same time (disjoint rows); rows whose Cholesky meets a
-    // non-positive pivot go to the eigen-solver afterwards. Each row ends
-    // as it did when the eigen-solver ran over the whole list before the
-    // Cholesky of its untruncated rows.
+    // otherwise by their eigenvalues: the rows with one below the threshold
+    // are set up where these are found, those with none have A^+ = A^-1 and
+    // are solved again by Cholesky, and the few that neither can take (the
+    // one lists them, and the other the rows whose Cholesky meets a
+    // non-positive pivot) go to the eigen-solver with eigenvectors.
     int64_t const nl = n_tgt - p.row0;
-    DeviceBuffer<int32_t> rlist( nl, s ), tlist( nl, s ), flist( nl, s ),
-        counts( 3, s ); // refine, truncated, refine failures
+    DeviceBuffer<int32_t> rlist( nl, s ), flist( nl, s ),
+        counts( 3, s ); // refine, left over, queue
     zero_async( counts.get(), 3 * sizeof( int32_t ), s );
     q.refine_rows = rlist.get();
     q.n_refine = counts.get();
-    setup_screen( src, tgt, n_tgt, indices, order, q, coeffs32 != nullptr,
-                  tlist.get(), counts.get() + 1, counters, s );
+    setup_listed( src, tgt, n_tgt, indices, order, q, coeffs, coeffs32,
+                  flist.get(), counts.get() + 1, counts.get() + 2, counters, s );
+    int64_t const blocks =
+        std::min<int64_t>( ceil_div( nl, kBlock ), kRefineBlocks );
+    auto refine = [&]( auto m, auto f32 ) {
+        refine_kernel<decltype( m )::value, decltype( f32 )::value>
+            <<<blocks, kBlock, 0, s>>>(
+                src, tgt, indices, order, p.row_off, p.kk, p.rbf, p.geometry,
+                rlist.get(), counts.get(), coeffs, coeffs32, p.by_distance,
+                flist.get(), counts.get() + 1 );
+    };
+    using T = std::true_type;
+    using F = std::false_type;
+    using M1 = std::integral_constant<int, 1>;
+    using M4 = std::integral_constant<int, 4>;
+    using M10 = std::integral_constant<int, 10>;
+    if ( p.m == 1 )
+        coeffs32 ? refine( M1{}, T{} ) : refine( M1{}, F{} );
+    else if ( p.m == 4 )
+        coeffs32 ? refine( M4{}, T{} ) : refine( M4{}, F{} );
+    else
+        coeffs32 ? refine( M10{}, T{} ) : refine( M10{}, F{} );
+    DTKX_HIP( hipGetLastError() );
     SetupParams f = p;
     f.screened = true;
-    {
-        Fork fork( s );
-        f.rows = tlist.get();
-        f.n_rows = counts.get() + 1;
-        setup_cyclic( src, tgt, n_tgt, indices, order, f, coeffs, coeffs32,
-                      nullptr, counters, fork.side() );
-        int64_t const blocks = std::min<int64_t>(
-            ceil_div( n_tgt - p.row0, kBlock ), kRefineBlocks );
-        auto refine = [&]( auto m, auto f32 ) {
-            refine_kernel<decltype( m )::value, decltype( f32 )::value>
-                <<<blocks, kBlock, 0, s>>>(
-                    src, tgt, indices, order, p.row_off, p.kk, p.rbf,
-                    p.geometry, rlist.get(), counts.get(), coeffs, coeffs32,
-                    p.by_distance, flist.get(), counts.get() + 2 );
-        };
-        using T = std::true_type;
-        using F = std::false_type;
-        using M1 = std::integral_constant<int, 1>;
-        using M4 = std::integral_constant<int, 4>;
-        using M10 = std::integral_constant<int, 10>;
-        if ( p.m == 1 )
-            coeffs32 ? refine( M1{}, T{} ) : refine( M1{}, F{} );
-        else if ( p.m == 4 )
-            coeffs32 ? refine( M4{}, T{} ) : refine( M4{}, F{} );
-        else
-            coeffs32 ? refine( M10{}, T{} ) : refine( M10{}, F{} );
-        DTKX_HIP( hipGetLastError() );
-        fork.join();
-    }
     f.rows = flist.get();
-    f.n_rows = counts.get() + 2;
+    f.n_rows = counts.get() + 1;
     setup_cyclic( src, tgt, n_tgt, indices, order, f, coeffs, coeffs32,
                   nullptr, counters, s );
 }
