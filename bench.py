@@ -748,10 +748,8 @@ def bench_nn(args):
 def bench_knn(args):
     """The k-nearest-neighbour search on its own (the reference's ArborX
     build and query, DTK_MovingLeastSquaresOperator_def.hpp:47-60): per
-    step, the hierarchy over n float sources and the query of n targets,
-    each row ascending by (distance, index); rows of more than 32
-    neighbours are collected unordered and sorted by a kernel of their
-    own. A sample of rows is checked against the oracle's k-d tree search,
+    step, the boxes over n float sources and the query of n targets,
+    each row ascending by (distance, index). A sample of rows is checked against the oracle's k-d tree search,
     which is also timed on the host as the baseline."""
     import numpy as np
     import torch
