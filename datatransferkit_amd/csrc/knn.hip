@@ -236,7 +236,7 @@ constexpr int kSrcPasses = ( kSrcKeyBits + 7 ) / 8;
 constexpr int kTgtPasses = ( kTgtKeyBits + 7 ) / 8;
 constexpr int kHistWords = ( kSrcPasses + kTgtPasses ) * rsort::kDigits;
 
-// Hilbert codes of the sources (63-bit) and of the targets (top 30 bits) in
+// Hilbert codes of the sources (63-bit) and of the targets (top 48 bits) in
 // one launch, one sort tile of points a block (blocks [0, src_blocks) take
 // the sources), with the digit counts of every radix pass added into hist
 // (sources' passes first, zero on entry). src_prob / tgt_prob (nullable, a batch):
