@@ -230,7 +230,9 @@ __device__ inline uint64_t hilbert_code( uint32_t const *q )
 // targets' top 48 bits (a cell of 1.5e-5 of the scene: a group of targets
 // must be close together in terms of the sources around it. With 30 bits,
 // cells of 1e-3, the targets inside a cluster of that size were in no order,
-// and half of the rows of 1M points in 200 such clusters were left over).
+// and half of the rows of 1M points in 200 such clusters were left over. 39
+// bits, one pass less: 1M x 1M nearest 471 -> 465 us, but in clusters of 1e-4
+// k = 10 took 1.69 ms instead of 1.15).
 constexpr int kSrcKeyBits = 63, kTgtLevels = 16, kTgtKeyBits = 3 * kTgtLevels;
 constexpr int kSrcPasses = ( kSrcKeyBits + 7 ) / 8;
 constexpr int kTgtPasses = ( kTgtKeyBits + 7 ) / 8;
