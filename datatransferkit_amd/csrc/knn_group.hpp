@@ -16,7 +16,10 @@
 //      by counting (a ballot and a population count a chunk). The target is
 //      done if t (with the margin of the rounded root below) does not reach
 //      past R; else the group's unfinished targets are gathered again with
-//      the larger radius that the count names.
+//      the larger radius that the count names. Where distances are tied the
+//      counts may jump from below kk to above S (on a lattice 7 and 19 around
+//      a node, 8 and 32 around a cell's centre): then the kk-th distance
+//      itself is found, and at it the lowest source indices.
 //   3. sort: the selected candidates of 16 targets are sorted together, four
 //      lanes a row, and the first kk of each row written.
 // R starts from the size of the 64-point node nearest the wave's first
@@ -532,10 +535,13 @@ struct GroupArgs
 
 // Row slots S of a search for kk results: room for the count to land in
 // [kk, S] after one or two tries (a count that must hit a narrow window
-// takes more), at least one and a half times kk.
+// takes more), at least one and a half times kk. (k = 8 takes 32: with 16,
+// the counts 7 and 19 around a lattice's node leave every row to the kk-th
+// distance itself, 1.80 ms of query against 0.68 at 1M nodes; uniform points
+// 0.42 either way.)
 constexpr int group_slots( int kk )
 {
-    return kk <= 8 ? 16 : ( kk <= 20 ? 32 : ( kk <= 42 ? 64 : 128 ) );
+    return kk <= 7 ? 16 : ( kk <= 20 ? 32 : ( kk <= 42 ? 64 : 128 ) );
 }
 
 template <typename T>
@@ -560,6 +566,9 @@ struct GroupShape
 };
 
 constexpr int kGroupTries = 256; // gathers of a wave before rows are left over
+// counts of a target on the way to a threshold (one or two find it on evenly
+// spread points), before its kk-th distance itself is looked for
+constexpr int kSteps = 8;
 
 // Squared radius expected to hold kk sources around q (uniform): from the
 // boxes of the 64- and 512-point nodes that hold q (or of the nearest node,
@@ -686,20 +695,19 @@ __global__ void __launch_bounds__( 64 )
     // and too many
     T r2_few = T( 0 ), r2_full = type_max<T>();
     int last_prob = -1, tries = 0, shrinks = 0;
+    int steps = kSteps; // counts of a target: one after a group of ties
     int kk = a.kk;
     // the next group's R^2 over this one's: the k-th distances' spread grows
     // as k falls
     float const slack = 1.08f + 0.4f * g.root_k;
     int64_t beg = 0, end = a.n_src;
-    // counts grow with the 3/2 power of the squared distance; logarithms of
-    // kk and of the count that a first threshold aims at, times 2/3
+    // counts grow with the 3/2 power of the squared distance; the logarithm
+    // of the count that a first threshold aims at, times 2/3
     constexpr float kPower = 0.6666667f;
-    float log_kk = 0.f, log_aim = 0.f, to_aim = 1.f;
+    float log_aim = 0.f;
     auto set_k = [&]() {
-        log_kk = kPower * __builtin_amdgcn_logf( (float)kk );
         log_aim = kPower *
                   __builtin_amdgcn_logf( (float)kk + 0.375f * (float)( S - kk ) );
-        to_aim = __builtin_amdgcn_exp2f( log_aim - log_kk );
     };
     set_k();
 
@@ -718,6 +726,7 @@ __global__ void __launch_bounds__( 64 )
         group = uniform( group );
         last_prob = uniform( last_prob );
         shrinks = uniform( shrinks );
+        steps = uniform( steps );
         guessed = uniform( (int)guessed ) != 0;
         tries = uniform( tries );
         if ( ++tries > kGroupTries )
@@ -953,21 +962,17 @@ __global__ void __launch_bounds__( 64 )
         // 2. select. t_max: the largest threshold whose margin ends within R
         constexpr T kMargin =
             sizeof( T ) == 4 ? (T)1.0000019073486328 : (T)( 1.0 + 1e-14 );
-        T const t_max = all ? type_max<T>()
+        T const t_max = all ? type_max<T>() * T( 0.9999 )
                             : r2 * ( sizeof( T ) == 4 ? (T)0.99999618530273
                                                       : (T)( 1.0 - 2e-14 ) );
-        uint64_t done = 0, lost = 0;
+        uint64_t done = 0, lost = 0, hard = 0;
         T need = T( 0 ), widest = T( 0 );
         int n_rows = 0;
         int row_lane = first; // the wave's lane of the target of this lane's row
-        for ( uint64_t left = sub; left; left &= left - 1 )
-        {
-            left = uniform( left );
-            n_rows = uniform( n_rows );
-            int const i = __builtin_ctzll( left );
+        T row_top = T( 0 );
+        auto distances = [&]( int i, T ( &d2 )[C] ) {
             T const qt[3] = {lane_value( q[0], i ), lane_value( q[1], i ),
                              lane_value( q[2], i )};
-            T d2[C];
 #pragma unroll
             for ( int c = 0; c < C; ++c )
             {
@@ -976,17 +981,72 @@ __global__ void __launch_bounds__( 64 )
                 T const b[3] = {px[c], py[c], pz[c]};
                 d2[c] = point_sq( qt, b );
             }
-            auto count = [&]( T t ) {
-                int n = 0;
+        };
+        auto count_to = [&]( T const ( &d )[C], T t ) {
+            int n = 0;
 #pragma unroll
-                for ( int c = 0; c < C; ++c )
+            for ( int c = 0; c < C; ++c )
+            {
+                if ( c >= chunks )
+                    break;
+                n += __popcll( __ballot( d[c] <= t ) );
+            }
+            return n;
+        };
+        // target i's candidates with d <= t into row n_rows; how many. The
+        // sort key is d in steps of t 2^-kDistBits (a reciprocal to one unit:
+        // 64 steps of room), then the slot
+        auto fill_row = [&]( T const ( &d )[C], T t ) {
+            T const scale = t > T( 1e-30 )
+                                ? (T)( ( 1u << Sh::kDistBits ) - 64u ) *
+                                      reciprocal( t )
+                                : T( 0 );
+            for ( int s = lane; s < S; s += 64 )
+                rkey[n_rows * Sh::kPitch + s] = ~0u;
+            wave_sync();
+            int at = 0;
+#pragma unroll
+            for ( int c = 0; c < C; ++c )
+            {
+                if ( c >= chunks )
+                    break;
+                bool const in = d[c] <= t;
+                uint64_t const m = __ballot( in );
+                // (past the row's end: its padding)
+                uint32_t const slot =
+                    min( __builtin_amdgcn_mbcnt_hi(
+                             (uint32_t)( m >> 32 ),
+                             __builtin_amdgcn_mbcnt_lo( (uint32_t)m, at ) ),
+                         (uint32_t)( Sh::kPitch - 1 ) );
+                if ( in )
                 {
-                    if ( c >= chunks )
-                        break;
-                    n += __popcll( __ballot( d2[c] <= t ) );
+                    rkey[n_rows * Sh::kPitch + slot] =
+                        ( (uint32_t)( d[c] * scale ) << Sh::kSlotBits ) | slot;
+                    rpos[n_rows * Sh::kPitch + slot] = pp[c];
                 }
-                return n;
-            };
+                at += __popcll( m );
+            }
+            return at;
+        };
+        // target i's row is filled with n candidates up to the squared
+        // distance t; top: what its sort keys are fractions of
+        auto keep_row = [&]( int i, T t, int n, T top ) {
+            done |= 1ull << i;
+            row_lane = lane / W == n_rows ? i : row_lane;
+            row_top = lane / W == n_rows ? top : row_top;
+            // the next target's first threshold aims at the window's middle
+            t_last = uniform(
+                t * (T)__builtin_amdgcn_exp2f(
+                        log_aim - kPower * __builtin_amdgcn_logf( (float)n ) ) );
+            ++n_rows;
+        };
+        for ( uint64_t left = sub; left; left &= left - 1 )
+        {
+            left = uniform( left );
+            n_rows = uniform( n_rows );
+            int const i = __builtin_ctzll( left );
+            T d2[C];
+            distances( i, d2 );
             // a threshold with kk to S candidates at or below it
             T below = T( -1 ), above = type_max<T>();
             T limit = t_max;
@@ -994,12 +1054,11 @@ __global__ void __launch_bounds__( 64 )
             t = uniform( t < t_max ? t : t_max );
             bool found = false, beyond = false;
             int n = 0;
-            for ( int it = 0; it < 40; ++it )
+            for ( int it = 0; it < steps; ++it )
             {
                 t = uniform( t );
-                n = uniform( count( t ) );
-                // (four places for squared distances within the margin)
-                if ( n >= kk && n <= S - 4 )
+                n = uniform( count_to( d2, t ) );
+                if ( n >= kk && n <= S )
                 {
                     found = true;
                     break;
@@ -1022,7 +1081,7 @@ __global__ void __launch_bounds__( 64 )
                 float const f = __builtin_amdgcn_exp2f(
                     log_aim - kPower * __builtin_amdgcn_logf( (float)n + 0.5f ) );
                 T u = t * (T)f;
-                if ( !( u > below && u < above ) || it >= 6 )
+                if ( !( u > below && u < above ) )
                     u = above < type_max<T>()
                             ? T( 0.5 ) * ( below > T( 0 ) ? below : T( 0 ) ) +
                                   T( 0.5 ) * above
@@ -1033,80 +1092,147 @@ __global__ void __launch_bounds__( 64 )
                     break;
                 t = u;
             }
-            n = uniform( n );
-            if ( uniform( (int)( !found || beyond ) ) )
+            if ( uniform( (int)( found && !beyond ) ) )
             {
-                if ( found )
-                    need = need > t ? need : t;
-                else if ( n >= kk )
-                {
-                    // no such threshold: too many equal distances
-                    leave( 1ull << i );
-                    done |= 1ull << i;
-                    continue;
-                }
+                // squared distances whose root may round as the kk-th's
+                // stay in
+                n = uniform( n );
+                if ( uniform( fill_row( d2, t * kMargin ) ) <= S )
+                    keep_row( i, t, n, t );
                 else
-                {
-                    T u = r2 * T( 2.25 );
-                    if ( __popcll( sub ) == 1 )
-                    {
-                        r2_few = r2;
-                        u = r2_full < type_max<T>()
-                                ? T( 0.5 ) * ( r2_few + r2_full )
-                                : u;
-                    }
-                    need = need > u ? need : u;
-                }
-                lost |= 1ull << i;
+                    hard |= 1ull << i;
                 continue;
             }
-            // squared distances whose root may round as the kk-th's stay in
-            T const t_all = t * kMargin;
-            // (a reciprocal to one unit: 64 steps of room)
-            T const scale =
-                t_all > T( 1e-30 )
-                    ? (T)( ( 1u << Sh::kDistBits ) - 64u ) * reciprocal( t_all )
-                    : T( 0 );
-            for ( int s = lane; s < S; s += 64 )
-                rkey[n_rows * Sh::kPitch + s] = ~0u;
-            wave_sync();
-            int at = 0;
+            above = uniform( above );
+            if ( uniform( (int)!( found || beyond ||
+                                  above < type_max<T>() ) ) )
+                // no step came above: does R hold enough?
+                beyond = uniform( count_to( d2, t_max ) ) < kk;
+            if ( uniform( (int)!beyond ) )
+            {
+                hard |= 1ull << i;
+                continue;
+            }
+            T u = found ? t : above;
+            if ( !( u < type_max<T>() ) )
+            {
+                u = r2 * T( 2.25 );
+                if ( __popcll( sub ) == 1 )
+                {
+                    r2_few = r2;
+                    u = r2_full < type_max<T>()
+                            ? T( 0.5 ) * ( r2_few + r2_full )
+                            : u;
+                }
+            }
+            need = need > u ? need : u;
+            lost |= 1ull << i;
+        }
+        // Targets that R serves but no threshold does (distances tied on a
+        // lattice or among copies of a point: the counts jump over the
+        // window): the kk-th distance itself, from the rounded roots and
+        // without margins, and at it the lowest indices.
+        for ( uint64_t left = hard; left; left &= left - 1 )
+        {
+            left = uniform( left );
+            n_rows = uniform( n_rows );
+            int const i = __builtin_ctzll( left );
+            T const qt[3] = {lane_value( q[0], i ), lane_value( q[1], i ),
+                             lane_value( q[2], i )};
+            // (past the candidates: infinite)
+            T r[C];
 #pragma unroll
             for ( int c = 0; c < C; ++c )
             {
-                if ( c >= chunks )
-                    break;
-                bool const in = d2[c] <= t_all;
-                uint64_t const m = __ballot( in );
-                // (past the row's end: its padding)
-                uint32_t const slot = min(
-                    __builtin_amdgcn_mbcnt_hi(
-                        (uint32_t)( m >> 32 ),
-                        __builtin_amdgcn_mbcnt_lo( (uint32_t)m, at ) ),
-                    (uint32_t)( Sh::kPitch - 1 ) );
-                if ( in )
-                {
-                    rkey[n_rows * Sh::kPitch + slot] =
-                        ( (uint32_t)( d2[c] * scale ) << Sh::kSlotBits ) |
-                        slot;
-                    rpos[n_rows * Sh::kPitch + slot] = pp[c];
-                }
-                at += __popcll( m );
+                T const b[3] = {px[c], py[c], pz[c]};
+                r[c] = sqrt_rn( point_sq( qt, b ) );
+                // (one root at a time: their temporaries are many)
+                __builtin_amdgcn_sched_barrier( 0 );
             }
-            done |= 1ull << i;
-            if ( at > S )
+            auto count_roots = [&]( T t ) {
+                int m = 0;
+#pragma unroll
+                for ( int c = 0; c < C; ++c )
+                    m += __popcll( __ballot( r[c] <= t ) );
+                return m;
+            };
+            // a root with kk to S candidates at or below it, or the kk-th
+            // itself: lo < root <= hi, narrowed between the candidates' own
+            // values, so that each count rules one out
+            T lo = T( -1 ), hi = uniform( sqrt_rn( t_max ) ), root = hi;
+            int n = 0;
+            bool tied = false;
+            while ( !tied )
             {
-                leave( 1ull << i );
-                continue;
+                lo = uniform( lo );
+                hi = uniform( hi );
+                T v_min = T( INFINITY ), v_max = T( -1 );
+#pragma unroll
+                for ( int c = 0; c < C; ++c )
+                {
+                    bool const in = r[c] > lo && r[c] <= hi;
+                    v_min = fmin( v_min, in ? r[c] : T( INFINITY ) );
+                    v_max = fmax( v_max, in ? r[c] : T( -1 ) );
+                }
+                v_min = uniform( wave_min( v_min ) );
+                v_max = uniform( wave_max( v_max ) );
+                tied = uniform( (int)!( v_min < v_max ) ) != 0;
+                T m = v_max > T( 4 ) * v_min ? sqrt_rn( v_min * v_max )
+                                             : v_min + T( 0.5 ) * ( v_max - v_min );
+                m = tied ? v_max : ( m > v_min && m < v_max ? m : v_min );
+                root = m = uniform( m );
+                n = uniform( count_roots( m ) );
+                if ( n < kk )
+                    lo = m;
+                else if ( n <= S )
+                    break;
+                else
+                    hi = m;
             }
-            row_lane = lane / W == n_rows ? i : row_lane;
-            T const w =
-                t * (T)__builtin_amdgcn_exp2f(
-                        log_kk - kPower * __builtin_amdgcn_logf( (float)n ) );
+            if ( n > S )
+            {
+                // more at the kk-th distance than fit: of the lowest indices
+                // (they are distinct: some cut leaves just kk)
+                auto id = [&]( int c ) {
+                    return r[c] == root ? g.ids[pp[c]] : INT32_MAX;
+                };
+                auto count_ids = [&]( int cut ) {
+                    int m = 0;
+#pragma unroll
+                    for ( int c = 0; c < C; ++c )
+                        m += __popcll( __ballot( r[c] < root || id( c ) <= cut ) );
+                    return m;
+                };
+                int lo_id = INT32_MAX, hi_id = INT32_MAX;
+#pragma unroll
+                for ( int c = 0; c < C; ++c )
+                {
+                    int const v = id( c );
+                    lo_id = min( lo_id, v );
+                    hi_id = min( hi_id, v < INT32_MAX ? ~v : INT32_MAX );
+                }
+                lo_id = uniform( wave_min_int( lo_id ) ) - 1;
+                hi_id = ~uniform( wave_min_int( hi_id ) );
+                while ( hi_id - lo_id > 1 )
+                {
+                    int const m = lo_id + ( hi_id - lo_id ) / 2;
+                    n = uniform( count_ids( m ) );
+                    if ( n < kk )
+                        lo_id = uniform( m );
+                    else
+                        hi_id = uniform( m );
+                    if ( n >= kk && n <= S )
+                        break;
+                }
+#pragma unroll
+                for ( int c = 0; c < C; ++c )
+                    if ( r[c] == root && id( c ) > hi_id )
+                        r[c] = T( INFINITY );
+            }
+            fill_row( r, root );
+            T const w = root * root;
             widest = widest > w ? widest : w;
-            // the next target's first threshold aims at the window's middle
-            t_last = uniform( w * (T)to_aim );
-            ++n_rows;
+            keep_row( i, w, n, T( 0 ) );
         }
 
         // 3. sort
@@ -1129,6 +1255,17 @@ __global__ void __launch_bounds__( 64 )
             // results of this lane's keys
             int mine = ( valid ? kk : 0 ) - sl * E;
             sort_rows<W, E>( key, sl );
+            // the largest kk-th squared distance, for the next group's R
+            uint32_t kth = key[0];
+#pragma unroll
+            for ( int e = 1; e < E; ++e )
+                kth = ( kk - 1 ) % E == e ? key[e] : kth;
+            T const w = uniform( wave_max(
+                valid && sl == ( kk - 1 ) / E
+                    ? row_top * (T)( kth >> Sh::kSlotBits ) *
+                          (T)( 1. / ( 1u << Sh::kDistBits ) )
+                    : T( 0 ) ) );
+            widest = widest > w ? widest : w;
             // neighbours of a row within the root's rounding (or the key's
             // step), the one past the last result included
             constexpr uint32_t kNear =
@@ -1185,10 +1322,47 @@ __global__ void __launch_bounds__( 64 )
                 if ( e < mine )
                     out[e] = pos[e];
 
-            // the close rows by the full (distance, index) keys, one row at
-            // a time over the wave (a few in a thousand rows of scattered
-            // points, every row of a lattice)
-            for ( uint64_t left = closes; left; )
+            // the close rows by the full (distance, index) keys: a few in a
+            // thousand rows of scattered points, one row at a time over the
+            // wave; every row of a lattice, all rows together where their
+            // keys fit the registers
+            bool together = false;
+            if constexpr ( S <= 32 )
+            {
+                together = __popcll( closes ) > 4;
+                if ( together )
+                {
+                    V const tq = a.tgt[rt];
+                    T const qq[3] = {tq.x, tq.y, tq.z};
+                    typename SK::type fk[E];
+#pragma unroll
+                    for ( int e = 0; e < E; ++e )
+                    {
+                        int const at = row * Sh::kPitch + sl * E + e;
+                        fk[e] = SK::none();
+                        if ( valid && rkey[at] != ~0u )
+                        {
+                            int32_t const ps = rpos[at];
+                            V const p = g.pts[ps];
+                            T const b[3] = {p.x, p.y, p.z};
+                            fk[e] = SK::make( sqrt_rn( point_sq( qq, b ) ),
+                                              g.ids[ps] );
+                        }
+                    }
+                    sort_rows<W, E>( fk, sl );
+#pragma unroll
+                    for ( int e = 0; e < E; ++e )
+                        if ( valid && sl * E + e < kk )
+                        {
+                            int32_t const id = SK::index( fk[e] );
+                            out[e] = a.src_pos ? a.src_pos[id] : id;
+                            if ( a.out_dist )
+                                a.out_dist[base + sl * E + e] =
+                                    SK::distance( fk[e] );
+                        }
+                }
+            }
+            for ( uint64_t left = together ? 0 : closes; left; )
             {
                 int const fl = __builtin_ctzll( left );
                 int const cr = fl / W;
@@ -1238,6 +1412,7 @@ __global__ void __launch_bounds__( 64 )
         todo &= ~done;
         if ( done )
         {
+            steps = hard ? 1 : kSteps;
             r2_few = T( 0 );
             r2_full = type_max<T>();
             shrinks = 0;

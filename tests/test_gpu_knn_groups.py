@@ -68,3 +68,44 @@ def test_hard_clouds(dtk, oracle_lib, geometry):
                               rng.random((400, 3)), 30 * rng.random((50, 3))])
         for k in (4, 10, 32, 64):
             check(dtk, oracle_lib, src, tgt, k, geometry)
+
+
+TIED = {
+    # counts around a cell's centre: 8, 32, 56, ...; around a node: 1, 7, 19, 27
+    "cells": (lambda n: (grid_points((n, n, n), (0, 0, 0)),
+                         grid_points((n - 1, n - 1, n - 1), (0.5, 0.5, 0.5))), (8, 10, 16, 20)),
+    "nodes": (lambda n: (grid_points((n, n, n), (0, 0, 0)),) * 2, (8, 10, 16, 20)),
+    # a spacing that rounds: the same shells a few units of rounding thick
+    "rounded": (lambda n: (grid_points((n, n, n), (0, 0, 0)) / (n + 0.7),
+                           grid_points((n - 1, n - 1, n - 1), (0.5, 0.5, 0.5)) / (n + 0.7)),
+                (10, 16, 20)),
+    # every node eight times, as the corners of hexahedra give them
+    "copies": (lambda n: (np.repeat(grid_points((n // 2,) * 3, (0, 0, 0)), 8, axis=0),
+                          grid_points((n // 2 - 1,) * 3, (0.5, 0.5, 0.5))), (1, 10, 32, 64)),
+}
+
+
+@pytest.mark.parametrize("geometry", ["float", "double"])
+@pytest.mark.parametrize("n", [12, 64])
+@pytest.mark.parametrize("cloud", list(TIED))
+def test_tied_distances_stay_in_the_groups(dtk, oracle_lib, cloud, n, geometry):
+    """Where the number of sources within a distance jumps over the row's
+    slots no threshold fits them; the rows are finished all the same, none is
+    left to the tree search."""
+    make, ks = TIED[cloud]
+    src, tgt = make(n)
+    rng = np.random.default_rng(n)
+    src = np.ascontiguousarray(src[rng.permutation(len(src))])
+    sample = rng.permutation(len(tgt))[:4000]
+    d_src, d_tgt = torch.as_tensor(src).cuda(), torch.as_tensor(tgt).cuda()
+    for k in ks:
+        print(f"ties: {cloud} {len(src)} -> {len(tgt)}, k={k}, {geometry}", flush=True)
+        op = dtk.MovingLeastSquaresOperator(d_src, d_tgt, basis="constant", k=k,
+                                            geometry=geometry)
+        assert op.stats()["n_stack_overflow"] == 0
+        gi, gd = oracle_lib.knn(src, tgt[sample], k, geometry=0 if geometry == "float" else 1)
+        idx, dist = dtk.knn(d_src, d_tgt, k, geometry=geometry, with_distances=True)
+        assert np.array_equal(idx.cpu().numpy()[sample], gi)
+        assert np.array_equal(dist.cpu().numpy()[sample].view(np.uint64),
+                              np.ascontiguousarray(gd).view(np.uint64))
+        assert np.array_equal(op.graph()[1].cpu().numpy(), idx.cpu().numpy())
