@@ -154,23 +154,32 @@ __device__ inline uint64_t expand21( uint32_t v )
     return x;
 }
 
-// The 2^21 grid of a scene box (box[0..2] = lower corner, box[3..5] = upper
-// corner): cell = (p - lo) scale. One division an axis and box, not a point.
+// The largest extent of a scene box (box[0..2] = lower corner, box[3..5] =
+// upper corner).
+template <typename T>
+__device__ inline double scene_extent( T const *box )
+{
+    double e = 0;
+    for ( int d = 0; d < 3; ++d )
+        e = fmax( e, (double)box[3 + d] - (double)box[d] );
+    return e;
+}
+
+// The 2^21 grid of a scene box, of cubic cells over its largest extent: cell
+// = (p - lo) scale. One division a box, not a point. (With the grid stretched
+// over each extent, 64 consecutive points of a box of 1 x 0.01 x 0.0001 lay
+// within 0.04 x 0.0004 x 4e-6: k = 32 for 1M points took 41 ms with the group
+// search and 11.5 with a tree search a lane.)
 struct CurveFrame
 {
-    double lo[3], scale[3];
+    double lo[3], scale;
 };
 template <typename T>
 __device__ inline CurveFrame curve_frame( T const *box )
 {
-    CurveFrame f;
-    for ( int d = 0; d < 3; ++d )
-    {
-        f.lo[d] = box[d];
-        double const ext = (double)box[3 + d] - f.lo[d];
-        f.scale[d] = ext > 0 ? 2097151.0 / ext : 0.0;
-    }
-    return f;
+    double const ext = scene_extent( box );
+    return {{(double)box[0], (double)box[1], (double)box[2]},
+            ext > 0 ? 2097151.0 / ext : 0.0};
 }
 
 // Cell of p on the grid of f.
@@ -180,7 +189,7 @@ __device__ inline void curve_cell( V p, CurveFrame const &f, uint32_t *q )
     double const c[3] = {(double)p.x, (double)p.y, (double)p.z};
     for ( int d = 0; d < 3; ++d )
     {
-        double u = ( c[d] - f.lo[d] ) * f.scale[d];
+        double u = ( c[d] - f.lo[d] ) * f.scale;
         u = u < 0 ? 0 : ( u > 2097151.0 ? 2097151.0 : u );
         q[d] = (uint32_t)u;
     }
@@ -358,13 +367,14 @@ __device__ inline void cell_box( uint32_t const *qb, uint32_t const *qm,
         n_diff += (int)diff[d];
     }
     bool const cut = part == 2 || ( part == 1 && n_diff == 2 );
+    double const ext = scene_extent( scene );
+    double const h = ext / 2097151.0;
+    double const margin = 1e-9 * ext + 1e-300;
     for ( int d = 0; d < 3; ++d )
     {
         int const s = cut && !diff[d] ? sh - 1 : sh;
         uint32_t const qmin = ( qb[d] >> s ) << s;
-        double const s0 = scene[d], ext = (double)scene[3 + d] - s0;
-        double const h = ext / 2097151.0;
-        double const margin = 1e-9 * ext + 1e-300;
+        double const s0 = scene[d];
         double l = s0 + qmin * h - margin;
         double u = s0 + ( (double)qmin + (double)( 1u << s ) ) * h + margin;
         if ( sizeof( T ) == 4 )

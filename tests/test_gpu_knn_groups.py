@@ -109,3 +109,22 @@ def test_tied_distances_stay_in_the_groups(dtk, oracle_lib, cloud, n, geometry):
         assert np.array_equal(dist.cpu().numpy()[sample].view(np.uint64),
                               np.ascontiguousarray(gd).view(np.uint64))
         assert np.array_equal(op.graph()[1].cpu().numpy(), idx.cpu().numpy())
+
+
+@pytest.mark.parametrize("geometry", ["float", "double"])
+@pytest.mark.parametrize("box", [(1, 1e-2, 1e-4), (1e-4, 1, 1e-2), (3e-9, 3e-5, 3e-7)])
+def test_thin_boxes_stay_in_the_groups(dtk, oracle_lib, box, geometry):
+    """Clouds much thinner in some directions: the curve's cells are cubes
+    (the grid is as wide as the longest side), so that groups of its points
+    stay round and are finished without the tree search."""
+    rng = np.random.default_rng(8)
+    src, tgt = rng.random((60_000, 3)) * np.array(box), rng.random((30_000, 3)) * np.array(box)
+    d_src, d_tgt = torch.as_tensor(src).cuda(), torch.as_tensor(tgt).cuda()
+    sample = rng.permutation(len(tgt))[:2000]
+    for k in (1, 10, 64):
+        print(f"thin box {box} k={k} {geometry}", flush=True)
+        op = dtk.MovingLeastSquaresOperator(d_src, d_tgt, basis="constant", k=k,
+                                            geometry=geometry)
+        assert op.stats()["n_stack_overflow"] == 0
+        gi, _ = oracle_lib.knn(src, tgt[sample], k, geometry=0 if geometry == "float" else 1)
+        assert np.array_equal(op.graph()[1].cpu().numpy()[sample], gi)
