@@ -11,17 +11,22 @@
 // 0.72 ms, k = 1 0.65 ms (one tree traversal a lane over the hierarchy below
 // took 2.14, 1.00 and 0.64).
 //
-// The rows that the groups leave, and searches with fewer than 64 sources,
+// The rows that the groups leave (targets far outside the sources' box or in
+// the middle of a hollow cloud, where a sphere that holds k sources holds
+// hundreds a little further on), and searches with fewer than 64 sources,
 // go to a tree search: a Karras hierarchy over the sorted codes (duplicate
 // codes split by index), in which each internal node also writes both child
 // boxes: exact for small children, the curve cell of the child's common
-// prefix for large ones (a conservative box needs no bottom-up pass). One
-// lane per target; a per-lane stack in LDS, or in global memory; the k best
-// candidates stay sorted in registers as 64-bit keys (float distance bits
-// << 32 | index), so the ordering is (distance, index) with one integer
-// compare. Pruning uses squared distances against a threshold slightly above
+// prefix, cut to the boxes of the runs that hold its points, for large ones.
+// One lane per target; a per-lane stack in LDS, its deeper entries in global
+// memory; for small k the best candidates stay sorted in registers as 64-bit
+// keys (float distance bits << 32 | index), so the ordering is (distance,
+// index) with one integer compare, for larger k a second traversal collects
+// them. Pruning uses squared distances against a threshold slightly above
 // the square of the current k-th distance, which never drops a candidate
-// that could tie or beat it.
+// that could tie or beat it. 1M x 1M, k = 10, build and query: targets 2 box
+// sides away 1.52 ms (9.4 by groups alone), in a box 3 times as wide 1.59
+// (8.9).
 #include "knn.hpp"
 #include "radix_sort.hpp"
 
@@ -57,6 +62,24 @@ struct alignas( 16 ) Node
     T lo[2][3];
     T hi[2][3];
     int32_t child[2];
+};
+
+// A node's box; entry 3 of each corner is unused (two 16-byte loads).
+template <typename T>
+struct alignas( 16 ) CurveBox
+{
+    T lo[4];
+    T hi[4];
+};
+
+// Boxes of the sorted sources: node i of level l covers the sources
+// [i 8^(l+1), (i + 1) 8^(l+1)).
+constexpr int kMaxBoxLevels = 10;
+template <typename T>
+struct BoxLevels
+{
+    CurveBox<T> *level[kMaxBoxLevels] = {};
+    int n_levels = 0;
 };
 
 constexpr int kBlock = 256;
@@ -247,8 +270,45 @@ constexpr int kSrcPasses = ( kSrcKeyBits + 7 ) / 8;
 constexpr int kTgtPasses = ( kTgtKeyBits + 7 ) / 8;
 constexpr int kHistWords = ( kSrcPasses + kTgtPasses ) * rsort::kDigits;
 
-// Hilbert codes of the sources (63-bit) and of the targets (top 48 bits) in
-// one launch, one sort tile of points a block (blocks [0, src_blocks) take
+// Key of a target (kTgtKeyBits bits). Outside the grid: by the side or corner
+// of the grid that it lies beyond, then the code of its mirror image inside (a
+// coarser one), so that consecutive targets are close in all three directions.
+// Inside: after all those (a wave of a few scattered targets is done while the
+// others run; as the last one it made the query of 1M uniform targets 20 us
+// longer), the top bits of its code. (Clamped to the
+// grid, targets 2 to 3 box sides away followed each other at random depths, in
+// the order in which the curve visits the face: tree search of 1M x 1M such
+// points, k = 10, 1.06 ms.)
+template <typename V>
+__device__ inline uint64_t target_key( V p, CurveFrame const &f )
+{
+    constexpr double kMax = 2097151.0;
+    double const c[3] = {(double)p.x, (double)p.y, (double)p.z};
+    uint32_t q[3];
+    uint32_t image = 0;
+    for ( int d = 0; d < 3; ++d )
+    {
+        double u = ( c[d] - f.lo[d] ) * f.scale;
+        uint32_t const side = u < 0 ? 1u : ( u > kMax ? 2u : 0u );
+        image = image * 3u + side;
+        if ( side )
+        {
+            double const x = fabs( u ) * ( 1.0 / kMax );
+            double const y = x - 2.0 * floor( 0.5 * x ); // [0, 2)
+            u = kMax * ( y > 1.0 ? 2.0 - y : y );
+            u = u >= 0 && u <= kMax ? u : 0.0; // (not finite)
+        }
+        q[d] = (uint32_t)u;
+    }
+    constexpr int kOuter = kTgtLevels - 2; // 1 + 5 bits name the image
+    int const cut = image ? 21 - kOuter : 21 - kTgtLevels;
+    uint32_t const top[3] = {q[0] >> cut, q[1] >> cut, q[2] >> cut};
+    uint64_t const code = hilbert_code<kTgtLevels>( top );
+    return image ? ( (uint64_t)image << ( 3 * kOuter ) ) | code
+                 : ( 1ull << ( kTgtKeyBits - 1 ) ) | code >> 1;
+}
+
+// Hilbert codes of the sources (63-bit) and keys of the targets in one launch, one sort tile of points a block (blocks [0, src_blocks) take
 // the sources), with the digit counts of every radix pass added into hist
 // (sources' passes first, zero on entry). src_prob / tgt_prob (nullable, a batch):
 // each point's problem, whose scene box is box + 6 problem.
@@ -279,10 +339,10 @@ __global__ void __launch_bounds__( rsort::kThreads )
             break;
         if ( prob )
             frame = curve_frame( box + 6 * prob[i] );
-        uint32_t q[3];
-        curve_cell( pts[i], frame, q );
         if ( is_src )
         {
+            uint32_t q[3];
+            curve_cell( pts[i], frame, q );
             uint64_t const code = hilbert_code<21>( q );
             scodes[i] = code;
 #pragma unroll
@@ -292,10 +352,7 @@ __global__ void __launch_bounds__( rsort::kThreads )
         }
         else
         {
-            // the top bits of the full code
-            constexpr int kCut = 21 - kTgtLevels;
-            uint32_t const cut[3] = {q[0] >> kCut, q[1] >> kCut, q[2] >> kCut};
-            uint64_t const c = hilbert_code<kTgtLevels>( cut );
+            uint64_t const c = target_key( pts[i], frame );
             tcodes[i] = c;
 #pragma unroll
             for ( int p = 0; p < kTgtPasses; ++p )
@@ -322,6 +379,20 @@ namespace dtkx
 {
 namespace
 {
+
+// The rows that a search leaves to the tree search are listed in eight parts,
+// by the XCD that leaves them, their counts kListPad apart: an atomic on one
+// counter takes some 10 ns, which 31,000 waves that each leave rows wait for
+// one after the other.
+constexpr int kListParts = 8, kListPad = 32;
+__device__ inline int left_total( int32_t const *count )
+{
+    int n = 0;
+#pragma unroll
+    for ( int p = 0; p < kListParts; ++p )
+        n += count[p * kListPad];
+    return n;
+}
 
 // ------------------------------------------------------ Karras hierarchy
 // delta(i, j): common prefix length of keys i and j, with the index used
@@ -393,7 +464,9 @@ __device__ inline void cell_box( uint32_t const *qb, uint32_t const *qm,
 // Children of internal node i: ranges, codes, parents and child boxes.
 // A child that is a leaf gets its point as a degenerate box and the code
 // ~source_index; an internal child covering at most kTight points gets its
-// exact box, a larger one the curve cell of its common prefix.
+// exact box, a larger one the curve cell of its common prefix, cut to the
+// boxes of the group search where there are any (without them 1M x 1M searches
+// of targets 20 box sides away took 2.1 ms at k = 10, with them 1.4).
 #ifndef DTKX_KNN_TIGHT
 #define DTKX_KNN_TIGHT 16
 #endif
@@ -418,7 +491,7 @@ __device__ inline int node_problem( int32_t const *src_off, int n_prob,
 }
 
 // One problem (src_off null): n points, internal nodes [0, n - 1).
-// wanted (nullable): nothing is built when it is 0 (no query is left to the
+// left_count (nullable): nothing is built if all parts are empty (no row left to the
 // hierarchy). Batch: n_int internal nodes in all; node i belongs to problem p, whose
 // sorted points are [src_off[p], src_off[p + 1]) with scene box scene + 6 p;
 // the hierarchy of each problem is built over its own range (child node
@@ -427,10 +500,10 @@ template <typename T, typename V>
 __global__ void __launch_bounds__( kBlock )
     karras_kernel( uint64_t const *codes_all, int32_t const *sorted_all,
                    V const *pts, V const *sorted_pts_all, int64_t n_int,
-                   T const *scenes, int32_t const *src_off, int n_prob,
-                   Node<T> *nodes, int32_t *sizes, int32_t const *wanted )
+                   T const *scenes, BoxLevels<T> const boxes,
+                   int32_t const *src_off, int n_prob, Node<T> *nodes, int32_t *sizes, int32_t const *left_count )
 {
-    if ( wanted && *wanted == 0 )
+    if ( left_count && left_total( left_count ) == 0 )
         return;
     int64_t const gi = blockIdx.x * (int64_t)kBlock + threadIdx.x;
     if ( gi >= n_int )
@@ -524,6 +597,33 @@ __global__ void __launch_bounds__( kBlock )
             curve_cell( point( e ), frame, qe );
             cell_box<T>( qb, qm, qe, prefix_delta( codes, n, b, e ), scene,
                          nd.lo[c], nd.hi[c] );
+            if ( boxes.n_levels > 0 )
+            {
+                // and the boxes of the (at most 12) runs that hold the points
+                int l = 0;
+                while ( ( ( so + e ) >> ( 3 * l + 3 ) ) -
+                                ( ( so + b ) >> ( 3 * l + 3 ) ) >=
+                            12 &&
+                        l + 1 < boxes.n_levels )
+                    ++l;
+                T lo[3] = {INFINITY, INFINITY, INFINITY};
+                T hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+                for ( int64_t q = ( so + b ) >> ( 3 * l + 3 );
+                      q <= ( so + e ) >> ( 3 * l + 3 ); ++q )
+                {
+                    CurveBox<T> const r = boxes.level[l][q];
+                    for ( int x = 0; x < 3; ++x )
+                    {
+                        lo[x] = fmin( lo[x], r.lo[x] );
+                        hi[x] = fmax( hi[x], r.hi[x] );
+                    }
+                }
+                for ( int x = 0; x < 3; ++x )
+                {
+                    nd.lo[c][x] = fmax( nd.lo[c][x], lo[x] );
+                    nd.hi[c][x] = fmin( nd.hi[c][x], hi[x] );
+                }
+            }
         }
     }
     nodes[gi] = nd;
@@ -752,11 +852,11 @@ constexpr int kQueryBlock = 64;
 #endif
 constexpr bool kSeed = DTKX_KNN_SEED != 0;
 
-// Queries run with an LDS stack of kLdsStack entries (14 waves per CU); the
-// rare one whose descent needs more is re-run with a global stack of
-// kMaxDepth entries. With the seeded k-th distance (seed_far_sq) a descent
-// pushes only far children inside the seed's bound, so shallow stacks
-// suffice.
+// A lane's traversal stack holds its first kLdsStack entries in LDS (14 waves
+// per CU). With the seeded k-th distance (seed_far_sq) a descent pushes only
+// far children inside the seed's bound, so shallow stacks almost always
+// suffice. Deeper entries go to global memory where rows come from a list;
+// a launch over all rows lists the rare row that needs them.
 // Every level of the hierarchy lengthens the common prefix of the node's
 // keys (63 curve bits, then 32 index bits for equal codes), so no path
 // from the root has more than 96 internal levels.
@@ -765,6 +865,23 @@ constexpr bool kSeed = DTKX_KNN_SEED != 0;
 #endif
 constexpr int kLdsStack = DTKX_KNN_LDS_STACK;
 constexpr int kMaxDepth = 97;
+// stack entries of the fixed-radius pass of a two-pass search when its row
+// is collected in the LDS stack's other slots (its radius is final, so it
+// descends far less deep than the first pass)
+constexpr int kPass2Stack = 12;
+// global stack entries a lane
+constexpr int kSpill = kMaxDepth - kPass2Stack;
+// the largest K whose two-pass rows are sorted by their own lane
+constexpr int kFusedSortK = 32;
+// The smallest K searched in two passes (below). 1M uniform sources and
+// targets, one pass against two: float coordinates 1.54 / 1.75 ms at k = 24,
+// 2.21 / 2.12 at k = 32; double coordinates, whose (distance, index)
+// comparisons cost three operations, 4.2 / 3.2 at k = 16, 11.9 / 5.1 at 32.
+template <typename T>
+constexpr int two_pass_k()
+{
+    return sizeof( T ) == 4 ? 32 : 16;
+}
 
 // Arguments of a query launch. One problem: rows [row0, row0 + n_rows) of
 // the Hilbert-ordered targets against n_src sources, kk results per row.
@@ -790,28 +907,34 @@ struct QueryArgs
     double *out_dist = nullptr;
     // curve layout: row r written at row r with indices as positions
     int32_t const *src_pos = nullptr;
-    // LDS-stack launch: rows whose descent would push past the LDS stack
-    // are listed here (and written by the re-run) instead of finished
-    int32_t *overflow_rows = nullptr;
-    int32_t *n_overflow = nullptr;
-    // global-stack re-run: rows rows[i] for i < *n_rows_dev, taken by the
-    // grid's n_rows lanes in turn, a stack of kMaxDepth entries per lane
-    // laid out [level][lane] (stride gstride)
-    int32_t const *rows = nullptr;
-    int32_t const *n_rows_dev = nullptr;
-    // nullable: the re-run adds the list's length here (one lane)
+    // rows left over: part p's are left_rows[p left_cap + i] for i <
+    // left_count[p kListPad]
+    int32_t *left_rows = nullptr, *left_count = nullptr;
+    int64_t left_cap = 0;
+    // launch over those rows: the tiles taken of each part (as left_count,
+    // zero before), the nodes of kSpill deeper stack entries per lane laid
+    // out [level][lane] (stride gstride)
+    int32_t *taken = nullptr;
+    // nullable: the list's length is added here (one lane)
     int32_t *n_rows_total = nullptr;
-    int2 *gstack = nullptr;
+    int32_t *gstack = nullptr;
     int64_t gstride = 0;
 };
 
-// One row of the tree search: lane qi (its global-stack slot), row r;
-// st_node and st_d are the block's LDS stack. STACK > 0: an LDS stack of
-// that many entries per lane (a query that would need more is listed for
-// the re-run); STACK == 0: a per-lane stack in global memory (gstack, laid
-// out [level][lane]) deep enough for any tree.
-template <typename T, int K, int STACK>
-__device__ inline void query_row( QueryArgs<T> const &a, int64_t const qi,
+template <typename T>
+__device__ inline void leave_row( QueryArgs<T> const &a, int64_t r )
+{
+    int const p = blockIdx.x % kListParts;
+    a.left_rows[p * a.left_cap + atomicAdd( a.left_count + p * kListPad, 1 )] =
+        (int32_t)r;
+}
+
+// One row of a one-pass search: row r, st_node and st_d the block's LDS
+// stack, spill the lane's slot in global memory. LIST: deeper entries go
+// there (nodes only: they are tested again when taken); else a row that needs
+// them is listed. Whether the row is written.
+template <typename T, int K, bool LIST>
+__device__ inline bool query_row( QueryArgs<T> const &a, int64_t const spill,
                                  int64_t const r, int32_t *st_node, T *st_d )
 {
     int32_t const t = a.order[r];
@@ -871,24 +994,17 @@ __device__ inline void query_row( QueryArgs<T> const &a, int64_t const qi,
                 int32_t far = near0 ? c1 : c0;
                 T fs = near0 ? s1 : s0;
                 next = near0 ? c0 : c1;
-                if ( STACK > 0 )
+                if ( sp < kLdsStack )
                 {
-                    if ( sp == STACK )
-                    {
-                        // deeper than the LDS stack: left to the re-run
-                        a.overflow_rows[atomicAdd( a.n_overflow, 1 )] =
-                            (int32_t)r;
-                        return;
-                    }
                     st_node[sp * kQueryBlock + threadIdx.x] = far;
                     st_d[sp * kQueryBlock + threadIdx.x] = fs;
                 }
+                else if ( LIST )
+                    a.gstack[( sp - kLdsStack ) * a.gstride + spill] = far;
                 else
                 {
-                    int2 e;
-                    e.x = far;
-                    e.y = __float_as_int( (float)fs );
-                    a.gstack[sp * a.gstride + qi] = e;
+                    leave_row( a, r );
+                    return false;
                 }
                 ++sp;
             }
@@ -901,25 +1017,14 @@ __device__ inline void query_row( QueryArgs<T> const &a, int64_t const qi,
                 while ( sp > 0 )
                 {
                     --sp;
-                    int32_t cand;
-                    T cs;
-                    if ( STACK > 0 )
+                    if ( LIST && sp >= kLdsStack )
                     {
-                        cand = st_node[sp * kQueryBlock + threadIdx.x];
-                        cs = st_d[sp * kQueryBlock + threadIdx.x];
+                        next = a.gstack[( sp - kLdsStack ) * a.gstride + spill];
+                        break;
                     }
-                    else
+                    if ( st_d[sp * kQueryBlock + threadIdx.x] <= thr )
                     {
-                        int2 e = a.gstack[sp * a.gstride + qi];
-                        cand = e.x;
-                        // the float copy of a double bound is rounded; a
-                        // rounded-down copy could prune wrongly, so it is
-                        // only used to order, never to prune, for double
-                        cs = sizeof( T ) == 4 ? (T)__int_as_float( e.y ) : 0;
-                    }
-                    if ( cs <= thr )
-                    {
-                        next = cand;
+                        next = st_node[sp * kQueryBlock + threadIdx.x];
                         break;
                     }
                 }
@@ -940,31 +1045,76 @@ __device__ inline void query_row( QueryArgs<T> const &a, int64_t const qi,
             if ( a.out_dist )
                 a.out_dist[base + j] = best.distance( j );
         }
+    return true;
 }
 
-template <typename T, int K, int STACK>
-__global__ void __launch_bounds__( kQueryBlock )
-    knn_query_kernel( QueryArgs<T> const a )
+// ------------------------------------------------- two-pass k-best search
+// For larger k the sorted (distance, index) list costs five operations per
+// slot for every candidate, and a wave runs it whenever any of its lanes
+// meets one. Two traversals do the same work with fewer operations:
+// pass 1 keeps only the k smallest SQUARED distances, a sorted register
+// array updated with one median-of-three per slot; its last entry s_k gives
+// the k-th distance d_k = sqrt(s_k) (a correctly rounded square root is
+// monotone, so it maps order statistics to order statistics). Exactly the
+// pass-1 entries whose root is below d_k are sources at distance < d_k, say
+// c_lt of them. Pass 2 is a fixed-radius traversal that writes those c_lt
+// sources and the k - c_lt smallest indices among the sources at distance
+// == d_k to the row; the row is then sorted by (distance, index) in
+// registers. The result is the set and order the sorted list gives.
+template <typename T>
+__device__ inline T med3( T a, T b, T c );
+template <>
+__device__ inline float med3( float a, float b, float c )
 {
-    constexpr int LS = STACK > 0 ? STACK : 1;
-    __shared__ int32_t st_node[LS * kQueryBlock];
-    __shared__ T st_d[LS * kQueryBlock];
-    int64_t const qi = xcd_tile<0>() * kQueryBlock + threadIdx.x;
-    if constexpr ( STACK == 0 )
+    return __builtin_amdgcn_fmed3f( a, b, c );
+}
+template <>
+__device__ inline double med3( double a, double b, double c )
+{
+    return fmin( c, fmax( a, b ) ); // a <= c
+}
+
+// The k smallest squared distances, ascending. Slots below K - kk hold -1,
+// so the last slot is the kk-th smallest for any kk <= K.
+template <typename T, int K>
+struct KthList
+{
+    T d[K];
+    __device__ void init( int kk )
     {
-        // listed rows: the grid's n_rows lanes stride over the list, whose
-        // length only the device knows
-        int64_t const n = *a.n_rows_dev;
-        if ( a.n_rows_total && qi == 0 )
-            atomicAdd( a.n_rows_total, (int32_t)n );
-        for ( int64_t i = qi; i < n; i += a.n_rows )
-            query_row<T, K, STACK>( a, qi, a.rows[i], st_node, st_d );
-        return;
+#pragma unroll
+        for ( int j = 0; j < K; ++j )
+            d[j] = j < K - kk ? T( -1 ) : T( INFINITY );
     }
-    // LDS-stack launches run rows [row0, row0 + n_rows), one per lane
-    if ( qi >= a.n_rows )
-        return;
-    query_row<T, K, STACK>( a, qi, a.row0 + qi, st_node, st_d );
+    // new d[j] = clamp(s, d[j - 1], d[j]): the j-th of the sorted union
+    __device__ void insert( T s )
+    {
+#pragma unroll
+        for ( int j = K - 1; j > 0; --j )
+            d[j] = med3( d[j - 1], s, d[j] );
+        d[0] = fmin( d[0], s );
+    }
+    __device__ T last() const { return d[K - 1]; }
+    // kk entries of value b (padding stays -1): b acts as kk candidates
+    // at squared distance b, so the list ends at the true kk-th value
+    // whenever at least kk sources lie at or below b
+    __device__ void seed( int kk, T b )
+    {
+#pragma unroll
+        for ( int j = 0; j < K; ++j )
+            if ( j >= K - kk )
+                d[j] = b;
+    }
+};
+
+// A squared-distance bound above every s whose rounded root is <= w.
+__device__ inline float root_bound( float w )
+{
+    return w * w * 1.00000095367431640625f; // (1 + 2^-20)
+}
+__device__ inline double root_bound( double w )
+{
+    return w * w * 1.0000000000000009; // (1 + 2^-50)
 }
 
 // (distance, index) keys
@@ -1005,6 +1155,281 @@ struct SortKey<double>
     __device__ static double distance( type a ) { return a.d; }
 };
 
+constexpr int pow2_at_least( int k )
+{
+    int n = 1;
+    while ( n < k )
+        n <<= 1;
+    return n;
+}
+
+// ascending bitonic sorting network, all indices compile-time constants
+template <typename T, int N>
+__device__ inline void bitonic_sort( typename SortKey<T>::type ( &a )[N] )
+{
+    using SK = SortKey<T>;
+#pragma unroll
+    for ( int k = 2; k <= N; k <<= 1 )
+#pragma unroll
+        for ( int j = k >> 1; j > 0; j >>= 1 )
+#pragma unroll
+            for ( int i = 0; i < N; ++i )
+            {
+                int const l = i ^ j;
+                if ( l > i )
+                {
+                    bool const up = ( i & k ) == 0;
+                    auto const x = a[i], y = a[l];
+                    bool const swap = up ? SK::less( y, x ) : SK::less( x, y );
+                    a[i] = swap ? y : x;
+                    a[l] = swap ? x : y;
+                }
+            }
+}
+
+// One row of a two-pass search (query_row's arguments). Rows of K >
+// kFusedSortK are written unordered, as source indices.
+template <typename T, int K, bool LIST>
+__device__ inline bool query2_row( QueryArgs<T> const &a, int64_t const spill,
+                                  int64_t const r, int32_t *st_node, T *st_d )
+{
+    using SK = SortKey<T>;
+    int32_t const t = a.order[r];
+    int64_t so = 0, np = a.n_src;
+    int32_t root = 0;
+    int kk = a.kk;
+    if ( a.src_off )
+    {
+        int const pb = a.tgt_prob[t];
+        so = a.src_off[pb];
+        np = a.src_off[pb + 1] - so;
+        root = (int32_t)( so - pb );
+        kk = a.kk_prob[pb];
+    }
+    typename Vec4<T>::type qp = a.tgt[t];
+    T const q[3] = {qp.x, qp.y, qp.z};
+    int64_t const base =
+        a.row_off ? a.row_off[r] : ( a.src_pos ? r : (int64_t)t ) * kk;
+    int32_t *row = a.out_idx + base;
+
+    // pass 1: the kk-th smallest squared distance
+    KthList<T, K> list;
+    list.init( kk );
+    if ( a.node_size && np > 1 )
+        // pruning starts at the seed, so the descent pushes no far child
+        // beyond it
+        list.seed( kk, root_bound( sqrt_rn(
+                           seed_far_sq( a.nodes, a.node_size, root, q, kk ) ) ) );
+    if ( np == 1 )
+    {
+        typename Vec4<T>::type sp0 = a.src[so];
+        T const b[3] = {sp0.x, sp0.y, sp0.z};
+        list.insert( box_sq( q, b, b ) );
+    }
+    else
+    {
+        T thr = list.last();
+        int sp = 0;
+        int32_t node = root;
+        while ( node >= 0 )
+        {
+            Node<T> const nd = a.nodes[node];
+            T const s0 = box_sq( q, nd.lo[0], nd.hi[0] );
+            T const s1 = box_sq( q, nd.lo[1], nd.hi[1] );
+            int32_t const c0 = nd.child[0], c1 = nd.child[1];
+            // an entry equal to the bound leaves the list's values unchanged
+            if ( c0 < 0 && s0 < thr )
+            {
+                list.insert( s0 );
+                thr = list.last();
+            }
+            if ( c1 < 0 && s1 < thr )
+            {
+                list.insert( s1 );
+                thr = list.last();
+            }
+            bool const g0 = c0 >= 0 && s0 < thr;
+            bool const g1 = c1 >= 0 && s1 < thr;
+            int32_t next = -1;
+            if ( g0 && g1 )
+            {
+                bool const near0 = s0 <= s1;
+                int32_t const far = near0 ? c1 : c0;
+                T const fs = near0 ? s1 : s0;
+                next = near0 ? c0 : c1;
+                if ( sp < kLdsStack )
+                {
+                    st_node[sp * kQueryBlock + threadIdx.x] = far;
+                    st_d[sp * kQueryBlock + threadIdx.x] = fs;
+                }
+                else if ( LIST )
+                    a.gstack[( sp - kLdsStack ) * a.gstride + spill] = far;
+                else
+                {
+                    leave_row( a, r );
+                    return false;
+                }
+                ++sp;
+            }
+            else if ( g0 )
+                next = c0;
+            else if ( g1 )
+                next = c1;
+            else
+            {
+                while ( sp > 0 )
+                {
+                    --sp;
+                    if ( LIST && sp >= kLdsStack )
+                    {
+                        next = a.gstack[( sp - kLdsStack ) * a.gstride + spill];
+                        break;
+                    }
+                    if ( st_d[sp * kQueryBlock + threadIdx.x] < thr )
+                    {
+                        next = st_node[sp * kQueryBlock + threadIdx.x];
+                        break;
+                    }
+                }
+            }
+            node = next;
+        }
+    }
+
+    // pass 2: the sources at distance < d_k, and the smallest indices among
+    // those at distance == d_k, written to the row unordered
+    T const dk = sqrt_rn( list.last() );
+    int c_lt = 0;
+#pragma unroll
+    for ( int j = 0; j < K; ++j )
+        c_lt += ( list.d[j] >= 0 && sqrt_rn( list.d[j] ) < dk ) ? 1 : 0;
+    T const s_hi = root_bound( dk );
+    // The row is collected in LDS when it fits beside pass 2's stack (whose
+    // pass-1 distances are dead): the stack keeps the first kPass2Stack node
+    // slots, the row takes the distance slots (as ints) and the node slots
+    // above. Scattered 4-byte stores to the row in global memory, spread
+    // over the traversal, would leave partly written lines for the L2 to
+    // evict (8 times the row's bytes, measured).
+    constexpr int kDistSlots = kLdsStack * (int)( sizeof( T ) / 4 );
+    constexpr bool kRowLds = K <= kFusedSortK &&
+                             K <= kDistSlots + kLdsStack - kPass2Stack;
+    constexpr int kStack2 = kRowLds ? kPass2Stack : kLdsStack;
+    int32_t *const ids_d = reinterpret_cast<int32_t *>( st_d );
+    auto slot = [&]( int j ) -> int32_t & {
+        if constexpr ( kRowLds )
+        {
+            if ( j < kDistSlots )
+                return ids_d[j * kQueryBlock + threadIdx.x];
+            return st_node[( kPass2Stack + j - kDistSlots ) * kQueryBlock +
+                           threadIdx.x];
+        }
+        else
+            return row[j];
+    };
+    int n_lt = 0, n_eq = 0;
+    auto take = [&]( T s, int32_t id ) {
+        T const d = sqrt_rn( s );
+        if ( d < dk )
+        {
+            if ( n_lt < c_lt )
+                slot( n_lt++ ) = id;
+        }
+        else if ( d == dk )
+        {
+            if ( c_lt + n_eq < kk )
+                slot( c_lt + n_eq++ ) = id;
+            else
+            {
+                // all tie slots taken: replace the largest index if larger
+                int jm = c_lt;
+                for ( int j = c_lt + 1; j < kk; ++j )
+                    jm = slot( j ) > slot( jm ) ? j : jm;
+                if ( id < slot( jm ) )
+                    slot( jm ) = id;
+            }
+        }
+    };
+    if ( np == 1 )
+    {
+        typename Vec4<T>::type sp0 = a.src[so];
+        T const b[3] = {sp0.x, sp0.y, sp0.z};
+        take( box_sq( q, b, b ), (int32_t)so );
+    }
+    else
+    {
+        int sp = 0;
+        int32_t node = root;
+        while ( node >= 0 )
+        {
+            Node<T> const nd = a.nodes[node];
+            T const s0 = box_sq( q, nd.lo[0], nd.hi[0] );
+            T const s1 = box_sq( q, nd.lo[1], nd.hi[1] );
+            int32_t const c0 = nd.child[0], c1 = nd.child[1];
+            if ( c0 < 0 && s0 <= s_hi )
+                take( s0, ~c0 );
+            if ( c1 < 0 && s1 <= s_hi )
+                take( s1, ~c1 );
+            bool const g0 = c0 >= 0 && s0 <= s_hi;
+            bool const g1 = c1 >= 0 && s1 <= s_hi;
+            int32_t next = -1;
+            if ( g0 && g1 )
+            {
+                next = c0;
+                if ( sp < kStack2 )
+                    st_node[sp * kQueryBlock + threadIdx.x] = c1;
+                else if ( LIST )
+                    a.gstack[( sp - kStack2 ) * a.gstride + spill] = c1;
+                else
+                {
+                    leave_row( a, r );
+                    return false;
+                }
+                ++sp;
+            }
+            else if ( g0 )
+                next = c0;
+            else if ( g1 )
+                next = c1;
+            else if ( sp > 0 )
+            {
+                --sp;
+                next = sp < kStack2
+                           ? st_node[sp * kQueryBlock + threadIdx.x]
+                           : a.gstack[( sp - kStack2 ) * a.gstride + spill];
+            }
+            node = next;
+        }
+    }
+    if constexpr ( K <= kFusedSortK )
+    {
+        constexpr int N = pow2_at_least( K );
+        typename SK::type key[N];
+#pragma unroll
+        for ( int j = 0; j < N; ++j )
+        {
+            key[j] = SK::none();
+            if ( j < kk )
+            {
+                int32_t const id = slot( j );
+                typename Vec4<T>::type const p = a.src[id];
+                T const b[3] = {p.x, p.y, p.z};
+                key[j] = SK::make( sqrt_rn( box_sq( q, b, b ) ), id );
+            }
+        }
+        bitonic_sort<T, N>( key );
+#pragma unroll
+        for ( int j = 0; j < K; ++j )
+            if ( j < kk )
+            {
+                int32_t const id = SK::index( key[j] );
+                row[j] = a.src_pos ? a.src_pos[id] : id;
+                if ( a.out_dist )
+                    a.out_dist[base + j] = SK::distance( key[j] );
+            }
+    }
+    return true;
+}
+
 // a < b and (c ? a : b) field by field, without short-circuit branches
 __device__ inline bool key_less( DKey const &a, DKey const &b )
 {
@@ -1029,34 +1454,127 @@ namespace dtkx
 namespace
 {
 
+// The unordered rows of a wave's lanes (K > kFusedSortK; has: the lane has
+// one, row r) sorted by (distance, index), a row at a time over the wave.
+template <typename T>
+__device__ inline void sort_lane_rows( QueryArgs<T> const &a, int64_t r, bool has )
+{
+    using SK = SortKey<T>;
+    int const lane = threadIdx.x;
+    __threadfence_block(); // the lanes' rows are read by other lanes
+    for ( uint64_t left = __ballot( has ); left; left &= left - 1 )
+    {
+        int const l = __builtin_ctzll( left );
+        int64_t const rr = a.row0 + __builtin_amdgcn_readlane(
+                                        (int)( r - a.row0 ), l );
+        int32_t const t = a.order[rr];
+        int const kk = a.src_off ? a.kk_prob[a.tgt_prob[t]] : a.kk;
+        int64_t const base =
+            a.row_off ? a.row_off[rr] : ( a.src_pos ? rr : (int64_t)t ) * kk;
+        typename SK::type key[1] = {SK::none()};
+        if ( lane < kk )
+        {
+            typename Vec4<T>::type const qp = a.tgt[t];
+            T const q[3] = {qp.x, qp.y, qp.z};
+            int32_t const id = a.out_idx[base + lane];
+            typename Vec4<T>::type const p = a.src[id];
+            T const b[3] = {p.x, p.y, p.z};
+            key[0] = SK::make( sqrt_rn( box_sq( q, b, b ) ), id );
+        }
+        sort_wave<1, 64>( key, lane );
+        if ( lane < kk )
+        {
+            int32_t const id = SK::index( key[0] );
+            a.out_idx[base + lane] = a.src_pos ? a.src_pos[id] : id;
+            if ( a.out_dist )
+                a.out_dist[base + lane] = SK::distance( key[0] );
+        }
+    }
+}
+
+// The tree search, one row a lane. LIST: the listed rows, whose number only
+// the device knows; else rows [row0, row0 + n_rows), a block each 64.
+template <typename T, int K, bool LIST>
+__global__ void __launch_bounds__( kQueryBlock )
+    knn_query_kernel( QueryArgs<T> const a )
+{
+    __shared__ int32_t st_node[kLdsStack * kQueryBlock];
+    __shared__ T st_d[kLdsStack * kQueryBlock];
+    auto tile = [&]( int64_t r, bool has ) {
+        constexpr bool kTwo = K >= two_pass_k<T>();
+        int64_t const spill = blockIdx.x * (int64_t)kQueryBlock + threadIdx.x;
+        if ( has )
+        {
+            if constexpr ( kTwo )
+                has = query2_row<T, K, LIST>( a, spill, r, st_node, st_d );
+            else
+                has = query_row<T, K, LIST>( a, spill, r, st_node, st_d );
+        }
+        if constexpr ( kTwo && K > kFusedSortK )
+            sort_lane_rows( a, r, has );
+    };
+    if constexpr ( LIST )
+    {
+        int const total = left_total( a.left_count );
+        if ( total == 0 )
+            return;
+        if ( a.n_rows_total && blockIdx.x == 0 && threadIdx.x == 0 )
+            atomicAdd( a.n_rows_total, total );
+        // A block takes tiles of the part that its XCD left (consecutive on
+        // the curve: its L2 then holds their subtrees), and then of the
+        // others: a queue each, which every block sees empty before it ends.
+        for ( int j = 0; j < kListParts; ++j )
+        {
+            int const p = ( blockIdx.x + j ) % kListParts;
+            int const n = a.left_count[p * kListPad];
+            while ( n > 0 )
+            {
+                int i = 0;
+                if ( threadIdx.x == 0 )
+                    i = atomicAdd( a.taken + p * kListPad, 1 );
+                i = __builtin_amdgcn_readfirstlane( i ) * kQueryBlock;
+                if ( i >= n )
+                    break;
+                i += threadIdx.x;
+                tile( i < n ? a.left_rows[p * a.left_cap + i] : 0, i < n );
+            }
+        }
+    }
+    else
+    {
+        int64_t const i = xcd_tile<0>() * kQueryBlock + threadIdx.x;
+        tile( a.row0 + i, i < a.n_rows );
+    }
+}
+
 template <typename T>
 struct QueryLauncher
 {
-    template <int K>
-    static void run( int stack, QueryArgs<T> const &a, hipStream_t s )
-    {
-        dim3 grid( ceil_div( a.n_rows, kQueryBlock ) ), block( kQueryBlock );
-        if ( stack == kLdsStack )
-            knn_query_kernel<T, K, kLdsStack><<<grid, block, 0, s>>>( a );
-        else
-            knn_query_kernel<T, K, 0><<<grid, block, 0, s>>>( a );
-        DTKX_HIP( hipGetLastError() );
-    }
     // k: the largest number of results of a row in this launch
-    static void dispatch( int k, int stack, QueryArgs<T> const &a,
-                          hipStream_t s )
+    static void dispatch( int k, bool list, int64_t blocks,
+                          QueryArgs<T> const &a, hipStream_t s )
     {
-        if ( a.n_rows == 0 )
+        if ( blocks == 0 )
             return;
+        dim3 const grid( blocks ), block( kQueryBlock );
 #define DTKX_KNN_CASE( KV )                                                    \
     if ( k <= KV )                                                             \
     {                                                                          \
-        run<KV>( stack, a, s );                                                \
+        if ( list )                                                            \
+            knn_query_kernel<T, KV, true><<<grid, block, 0, s>>>( a );         \
+        else                                                                   \
+            knn_query_kernel<T, KV, false><<<grid, block, 0, s>>>( a );        \
+        DTKX_HIP( hipGetLastError() );                                         \
         return;                                                                \
     }
+        DTKX_KNN_CASE( 1 )
         DTKX_KNN_CASE( 4 )
+        DTKX_KNN_CASE( 8 )
+        DTKX_KNN_CASE( 10 )
         DTKX_KNN_CASE( 16 )
+        DTKX_KNN_CASE( 24 )
         DTKX_KNN_CASE( 32 )
+        DTKX_KNN_CASE( 48 )
         DTKX_KNN_CASE( 64 )
 #undef DTKX_KNN_CASE
         DTKX_REQUIRE( k <= knn_max_k, DTKX_ERR_UNSUPPORTED );
@@ -1140,32 +1658,39 @@ void build_boxes( V const *pts, int32_t const *ids, V *sorted, int64_t n,
 // the smallest source set searched by groups: one 64-point node
 constexpr int64_t kGroupSources = 64;
 
-// blocks of the global-stack re-run (at most 131k lanes, 102 MB of stack:
-// clouds with hundreds of copies of a point leave every row near them to it)
-constexpr int64_t kRerunBlocks = 2048;
+// Blocks of the launch over the rows left over: 14 a CU, as their LDS stacks
+// allow (float coordinates; 78 MB of deeper stack entries at most).
+constexpr int64_t kListBlocks = 3584;
 
 // The queries of a search, in launches of rows with up to kmax results.
 // With boxes, rows are searched by groups of targets (knn_group.hpp);
 // without, the tree search with its LDS stack runs over every row. Rows that
-// either leaves (too many sources at equal distances for the groups'
-// registers, a descent past the LDS stack) are run again by the tree search
-// with a global stack. After the groups the hierarchy is built only if there
+// either leaves are run by the tree search over a list, with deeper stacks in
+// global memory. After the groups the hierarchy is built only if there
 // are such rows: the device decides, the launch returns at once otherwise
 // (5 us, where the hierarchy of 1M sources takes 80).
-// build_tree( wanted ): launches karras_kernel, for *wanted != 0 if given.
+// build_tree( left_count ): launches karras_kernel, for rows left if given.
 template <typename T, typename BuildTree>
 void run_queries( std::vector<KnnBatch::Launch> const &launches,
                   QueryArgs<T> qa, int64_t n_tgt, double per_target,
                   BoxLevels<T> const *boxes, typename Vec4<T>::type const *pts,
-                  int32_t const *ids, BuildTree &&build_tree, KnnInfo *info,
-                  hipStream_t s )
+                  int32_t const *ids, T const *scene, BuildTree &&build_tree,
+                  KnnInfo *info, hipStream_t s )
 {
     if ( n_tgt == 0 )
         return;
-    DeviceBuffer<int32_t> rows( n_tgt, s ), count( 1, s );
-    zero_async( count.get(), sizeof( int32_t ), s );
-    qa.overflow_rows = rows.get();
-    qa.n_overflow = count.get();
+    // the rows left over (a part's blocks hold an eighth of each launch's
+    // rows and a block or two more), their counts and the tiles taken
+    qa.left_cap = 0;
+    for ( auto const &l : launches )
+        qa.left_cap += ( l.end - l.begin ) / kListParts + 2 * kQueryBlock;
+    DeviceBuffer<int32_t> rows( kListParts * qa.left_cap, s );
+    constexpr int kCounts = kListParts * kListPad;
+    DeviceBuffer<int32_t> count( 2 * kCounts, s );
+    zero_async( count.get(), 2 * kCounts * sizeof( int32_t ), s );
+    qa.left_rows = rows.get();
+    qa.left_count = count.get();
+    qa.taken = count.get() + kCounts;
     int kmax = 1;
     for ( auto const &l : launches )
         kmax = std::max( kmax, l.kmax );
@@ -1180,6 +1705,7 @@ void run_queries( std::vector<KnnBatch::Launch> const &launches,
             g.boxes = *boxes;
             g.pts = pts;
             g.ids = ids;
+            g.scene = scene;
             if ( g.a.n_rows == 0 )
                 continue;
             switch ( group_slots( l.kmax ) )
@@ -1206,35 +1732,35 @@ void run_queries( std::vector<KnnBatch::Launch> const &launches,
         {
             qa.row0 = l.begin;
             qa.n_rows = l.end - l.begin;
-            QueryLauncher<T>::dispatch( l.kmax, kLdsStack, qa, s );
+            QueryLauncher<T>::dispatch( l.kmax, false,
+                                        ceil_div( qa.n_rows, kQueryBlock ), qa,
+                                        s );
         }
     }
-    // The re-run is launched without reading the list's length back (a
+    // The launch over the list is made without reading its length back (a
     // stream synchronisation, 60 us of idle GPU at 1M x 1M): a bounded grid
-    // whose lanes stride over the list, each with its own global stack.
+    // whose blocks stride over the list, each lane with its own deeper stack.
     // Almost always the list is empty and the launch costs a few us.
-    int64_t const lanes =
-        std::min<int64_t>( ceil_div( n_tgt, kQueryBlock ), kRerunBlocks ) *
-        kQueryBlock;
-    DeviceBuffer<int2> gstack( static_cast<std::size_t>( kMaxDepth ) * lanes,
-                               s );
+    int64_t const blocks =
+        std::min<int64_t>( ceil_div( n_tgt, kQueryBlock ), kListBlocks );
+    DeviceBuffer<int32_t> gstack(
+        static_cast<std::size_t>( kSpill ) * blocks * kQueryBlock, s );
     QueryArgs<T> ra = qa;
-    ra.overflow_rows = nullptr;
-    ra.n_overflow = nullptr;
-    ra.rows = rows.get();
-    ra.n_rows_dev = count.get();
-    ra.n_rows = lanes;
+    ra.row0 = 0;
     ra.gstack = gstack.get();
-    ra.gstride = lanes;
+    ra.gstride = blocks * kQueryBlock;
     if ( info && info->n_overflow_dev )
         ra.n_rows_total = info->n_overflow_dev;
-    QueryLauncher<T>::dispatch( kmax, 0, ra, s );
+    QueryLauncher<T>::dispatch( kmax, true, blocks, ra, s );
     if ( info && !info->n_overflow_dev )
     {
-        int32_t n_over = 0;
-        DTKX_HIP( hipMemcpyAsync( &n_over, count.get(), sizeof( int32_t ),
+        int32_t left[kCounts];
+        DTKX_HIP( hipMemcpyAsync( left, count.get(), sizeof( left ),
                                   hipMemcpyDeviceToHost, s ) );
         DTKX_HIP( hipStreamSynchronize( s ) );
+        int32_t n_over = 0;
+        for ( int p = 0; p < kListParts; ++p )
+            n_over += left[p * kListPad];
         info->n_overflow += n_over;
     }
 }
@@ -1401,20 +1927,19 @@ void knn_impl( void const *src_v, int64_t n_src, void const *tgt_v,
     int64_t const n_int = n_src - 1;
     DeviceBuffer<Node<T>> nodes( std::max<int64_t>( n_int, 1 ), s );
     DeviceBuffer<int32_t> sizes( std::max<int64_t>( n_int, 1 ), s );
-    auto build_tree = [&]( int32_t const *wanted ) {
-        if ( n_int == 0 )
-            return;
-        karras_kernel<T, V><<<ceil_div( n_int, kBlock ), kBlock, 0, s>>>(
-            scodes.get(), ids_sorted, src, spts, n_int, box.get(), nullptr, 1,
-            nodes.get(), sizes.get(), wanted );
-        DTKX_HIP( hipGetLastError() );
-    };
     bool const grouped = n_src >= kGroupSources;
     DeviceBuffer<CurveBox<T>> box_buf;
     BoxLevels<T> boxes;
     if ( grouped )
         build_boxes<T, V>( spts, nullptr, nullptr, n_src, box_buf, boxes, s );
-
+    auto build_tree = [&]( int32_t const *left_count ) {
+        if ( n_int == 0 )
+            return;
+        karras_kernel<T, V><<<ceil_div( n_int, kBlock ), kBlock, 0, s>>>(
+            scodes.get(), ids_sorted, src, spts, n_int, box.get(), boxes,
+            nullptr, 1, nodes.get(), sizes.get(), left_count );
+        DTKX_HIP( hipGetLastError() );
+    };
     QueryArgs<T> qa;
     qa.nodes = nodes.get();
     qa.node_size = kSeed ? sizes.get() : nullptr;
@@ -1429,8 +1954,8 @@ void knn_impl( void const *src_v, int64_t n_src, void const *tgt_v,
     if ( info && info->query_begin )
         DTKX_HIP( hipEventRecord( info->query_begin, s ) );
     run_queries<T>( {{0, n_tgt, kk}}, qa, n_tgt, (double)n_src / (double)n_tgt,
-                    grouped ? &boxes : nullptr, spts, ids_sorted, build_tree,
-                    info, s );
+                    grouped ? &boxes : nullptr, spts, ids_sorted, box.get(),
+                    build_tree, info, s );
     if ( info && info->query_end )
         DTKX_HIP( hipEventRecord( info->query_end, s ) );
     // buffers are released at scope exit, ordered on the stream
@@ -1705,12 +2230,19 @@ void knn_batched_impl( void const *src_v, int64_t n_src, void const *tgt_v,
     int64_t const n_int = n_src - P;
     DeviceBuffer<Node<T>> nodes( std::max<int64_t>( n_int, 1 ), s );
     DeviceBuffer<int32_t> sizes( std::max<int64_t>( n_int, 1 ), s );
-    auto build_tree = [&]( int32_t const *wanted ) {
+    bool const grouped = n_src >= kGroupSources;
+    DeviceBuffer<V> spts( grouped ? n_src : 0, s );
+    DeviceBuffer<CurveBox<T>> box_buf;
+    BoxLevels<T> levels;
+    if ( grouped )
+        build_boxes<T, V>( src, out.src_perm, spts.get(), n_src, box_buf, levels,
+                           s );
+    auto build_tree = [&]( int32_t const *left_count ) {
         if ( n_int == 0 )
             return;
         karras_kernel<T, V><<<ceil_div( n_int, kBlock ), kBlock, 0, s>>>(
             codes_sorted.get(), out.src_perm, src, nullptr, n_int,
-            boxes.get(), b.src_off, P, nodes.get(), sizes.get(), wanted );
+            boxes.get(), levels, b.src_off, P, nodes.get(), sizes.get(), left_count );
         DTKX_HIP( hipGetLastError() );
     };
 
@@ -1719,14 +2251,6 @@ void knn_batched_impl( void const *src_v, int64_t n_src, void const *tgt_v,
         out.order, b.tgt_prob, b.row_base, b.row_start, b.kk_prob, n_tgt,
         b.nnz, out.row_off );
     DTKX_HIP( hipGetLastError() );
-
-    bool const grouped = n_src >= kGroupSources;
-    DeviceBuffer<V> spts( grouped ? n_src : 0, s );
-    DeviceBuffer<CurveBox<T>> box_buf;
-    BoxLevels<T> levels;
-    if ( grouped )
-        build_boxes<T, V>( src, out.src_perm, spts.get(), n_src, box_buf, levels,
-                           s );
 
     if ( info && info->query_begin )
         DTKX_HIP( hipEventRecord( info->query_begin, s ) );
@@ -1744,7 +2268,7 @@ void knn_batched_impl( void const *src_v, int64_t n_src, void const *tgt_v,
     qa.src_pos = out.src_pos;
     run_queries<T>( b.launches, qa, n_tgt, (double)n_src / (double)n_tgt,
                     grouped ? &levels : nullptr, spts.get(), out.src_perm,
-                    build_tree, info, s );
+                    boxes.get(), build_tree, info, s );
     if ( info && info->query_end )
         DTKX_HIP( hipEventRecord( info->query_end, s ) );
 }

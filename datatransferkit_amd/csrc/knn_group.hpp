@@ -54,24 +54,6 @@ namespace dtkx
 namespace
 {
 
-// A node's box; entry 3 of each corner is unused (two 16-byte loads).
-template <typename T>
-struct alignas( 16 ) CurveBox
-{
-    T lo[4];
-    T hi[4];
-};
-
-// Boxes of the sorted sources: node i of level l covers the sources
-// [i 8^(l+1), (i + 1) 8^(l+1)).
-constexpr int kMaxBoxLevels = 10;
-template <typename T>
-struct BoxLevels
-{
-    CurveBox<T> *level[kMaxBoxLevels] = {};
-    int n_levels = 0;
-};
-
 // Levels up to the first of at most 64 nodes (at least two), and the node
 // count of each.
 inline int box_levels( int64_t n, int64_t *count )
@@ -527,6 +509,7 @@ struct GroupArgs
     BoxLevels<T> boxes;
     typename Vec4<T>::type const *pts = nullptr; // sources in sorted order
     int32_t const *ids = nullptr;                // sorted position -> source
+    T const *scene = nullptr; // the sources' box, six values a problem
     int per_wave = 64; // targets a wave
     int group = 16;    // targets gathered together, at most
     float spacing = 1.f; // source spacing over the k-th distance, k^(-1/3)
@@ -565,17 +548,41 @@ struct GroupShape
     static constexpr int kDistBits = 32 - kSlotBits < 26 ? 32 - kSlotBits : 26;
 };
 
-constexpr int kGroupTries = 256; // gathers of a wave before rows are left over
+// Gathers of a wave that finish no target before its rows are left over:
+// kGroupTries where kManyLeft rows of its part of the list are left already
+// (the tree search has work then), kMaxTries where not (the hierarchy and the
+// longest descent of a few rows take 400 us).
+constexpr int kGroupTries = 8, kMaxTries = 96, kManyLeft = 512;
+// Targets this many expected k-th distances outside the sources' box are
+// left over at once where half of a wave of kFarWave or more are: a few such
+// targets are found sooner than the tree is built, and a wave a target finds
+// 3000 of them 2 box sides away in a third of the tree search's time.
+constexpr float kFar = 4.f;
+constexpr int kFarWave = 4;
 // counts of a target on the way to a threshold (one or two find it on evenly
 // spread points), before its kk-th distance itself is looked for
 constexpr int kSteps = 8;
 
+// Radius expected to hold the part `part` of a box's points (sides x, y, z),
+// read as an evenly filled volume, or as a surface or curve where those give
+// the larger radius.
+__device__ inline float even_radius( float x, float y, float z, float part )
+{
+    float const e0 = fmaxf( fmaxf( x, y ), z ), e2 = fminf( fminf( x, y ), z ),
+                e1 = __builtin_amdgcn_fmed3f( x, y, z );
+    return fmaxf(
+        __builtin_amdgcn_exp2f(
+            0.33333334f *
+            __builtin_amdgcn_logf( 0.23873f * e0 * e1 * e2 * part ) ),
+        fmaxf( 0.95f * __builtin_amdgcn_sqrtf( 0.31831f * e0 * e1 * part ),
+               0.45f * e0 * part ) );
+}
+
 // Squared radius expected to hold kk sources around q (uniform): from the
 // boxes of the 64- and 512-point nodes that hold q (or of the nearest node,
-// and then the distance to it too), read as evenly filled volumes, or as
-// surfaces or curves where those give the larger radius; the smallest of
-// the nodes' radii (a run's box may have corners that the run does not
-// fill), and a tenth more. One round of 64 boxes a level: the children of up
+// and then the distance to it too), read as evenly filled (even_radius); the
+// smallest of the nodes' radii (a run's box may have corners that the run
+// does not fill), and a tenth more. One round of 64 boxes a level: the children of up
 // to 8 nodes.
 template <typename T>
 __device__ inline T first_radius_sq( BoxLevels<T> const &boxes, int64_t beg,
@@ -598,23 +605,13 @@ __device__ inline T first_radius_sq( BoxLevels<T> const &boxes, int64_t beg,
         {
             CurveBox<T> const b = boxes.level[l][i];
             s = (float)gap_sq( q, q, b.lo, b.hi );
-            float const x = (float)( b.hi[0] - b.lo[0] ),
-                        y = (float)( b.hi[1] - b.lo[1] ),
-                        z = (float)( b.hi[2] - b.lo[2] );
-            float const e0 = fmaxf( fmaxf( x, y ), z ),
-                        e2 = fminf( fminf( x, y ), z ),
-                        e1 = __builtin_amdgcn_fmed3f( x, y, z );
-            float const part =
-                (float)kk *
-                __builtin_amdgcn_rcpf(
-                    (float)( min( end, (int64_t)( i + 1 ) << sh ) -
-                             max( beg, (int64_t)i << sh ) ) );
-            r = fmaxf( __builtin_amdgcn_exp2f(
-                           0.33333334f * __builtin_amdgcn_logf(
-                                             0.23873f * e0 * e1 * e2 * part ) ),
-                       fmaxf( 0.95f * __builtin_amdgcn_sqrtf(
-                                          0.31831f * e0 * e1 * part ),
-                              0.45f * e0 * part ) );
+            r = even_radius( (float)( b.hi[0] - b.lo[0] ),
+                             (float)( b.hi[1] - b.lo[1] ),
+                             (float)( b.hi[2] - b.lo[2] ),
+                             (float)kk *
+                                 __builtin_amdgcn_rcpf( (float)(
+                                     min( end, (int64_t)( i + 1 ) << sh ) -
+                                     max( beg, (int64_t)i << sh ) ) ) );
         }
         uint64_t hits = __ballot( s <= 0.f );
         gap = 0.f;
@@ -687,6 +684,48 @@ __global__ void __launch_bounds__( 64 )
     }
 
     uint64_t todo = n_here == 64 ? ~0ull : ( 1ull << n_here ) - 1;
+    auto leave = [&]( uint64_t which ) {
+        // rows that this search does not finish: the tree search's
+        if ( ( which >> lane ) & 1 )
+            leave_row( a, my_row );
+    };
+    {
+        // Far outside the sources' box a sphere around a target that holds kk
+        // sources holds many more a little further on: no radius serves.
+        T box[6];
+        float part;
+        if ( a.src_off )
+        {
+#pragma unroll
+            for ( int d = 0; d < 6; ++d )
+                box[d] = g.scene[6 * my_prob + d];
+            part = (float)a.kk_prob[my_prob] *
+                   __builtin_amdgcn_rcpf( (float)( a.src_off[my_prob + 1] -
+                                                   a.src_off[my_prob] ) );
+        }
+        else
+        {
+#pragma unroll
+            for ( int d = 0; d < 6; ++d )
+                box[d] = g.scene[d];
+            part = (float)a.kk * __builtin_amdgcn_rcpf( (float)a.n_src );
+        }
+        float const gap = (float)gap_sq( q, q, box, box + 3 );
+        uint64_t out = uniform( (uint64_t)( todo & __ballot( gap > 0.f ) ) );
+        if ( out )
+        {
+            float const r =
+                kFar * even_radius( (float)( box[3] - box[0] ),
+                                    (float)( box[4] - box[1] ),
+                                    (float)( box[5] - box[2] ), part );
+            out = uniform( (uint64_t)( out & __ballot( gap > r * r ) ) );
+            if ( g.per_wave >= kFarWave && 2 * __popcll( out ) >= g.per_wave )
+            {
+                leave( out );
+                todo &= ~out;
+            }
+        }
+    }
     int group = g.group; // at most kRows: a group's rows are sorted together
     T r2 = T( -1 );    // squared gather radius, negative: not known
     T t_last = T( 0 ); // the last target's threshold
@@ -697,9 +736,10 @@ __global__ void __launch_bounds__( 64 )
     int last_prob = -1, tries = 0, shrinks = 0;
     int steps = kSteps; // counts of a target: one after a group of ties
     int kk = a.kk;
-    // the next group's R^2 over this one's: the k-th distances' spread grows
-    // as k falls
-    float const slack = 1.08f + 0.4f * g.root_k;
+    // the next group's R^2 over this one's largest: the k-th distances' spread
+    // grows as k falls (1M uniform points, k = 10 / 32: 1.2 + 0.4 k^-1/2 432 /
+    // 580 us, 1.15 + 0.4 k^-1/2 438 / 596, 1 + 0.15 k^-1/2 469 / 624)
+    float const slack = 1.2f + 0.4f * g.root_k;
     int64_t beg = 0, end = a.n_src;
     // counts grow with the 3/2 power of the squared distance; the logarithm
     // of the count that a first threshold aims at, times 2/3
@@ -710,12 +750,6 @@ __global__ void __launch_bounds__( 64 )
                   __builtin_amdgcn_logf( (float)kk + 0.375f * (float)( S - kk ) );
     };
     set_k();
-
-    auto leave = [&]( uint64_t which ) {
-        // rows that this search does not finish: the tree search's
-        if ( ( which >> lane ) & 1 )
-            a.overflow_rows[atomicAdd( a.n_overflow, 1 )] = (int32_t)my_row;
-    };
 
     // (the search's state is the same in every lane: saying so where it
     // enters a loop keeps its control flow scalar)
@@ -729,7 +763,11 @@ __global__ void __launch_bounds__( 64 )
         steps = uniform( steps );
         guessed = uniform( (int)guessed ) != 0;
         tries = uniform( tries );
-        if ( ++tries > kGroupTries )
+        if ( tries > kGroupTries &&
+             ( tries > kMaxTries ||
+               uniform( __hip_atomic_load(
+                   a.left_count + blockIdx.x % kListParts * kListPad,
+                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT ) ) > kManyLeft ) )
         {
             leave( todo );
             break;
@@ -922,7 +960,12 @@ __global__ void __launch_bounds__( 64 )
             if ( guessed && ++shrinks <= 3 )
                 r2 *= T( 0.6 );
             else if ( n_sub > 1 )
+            {
                 group = ( n_sub + 1 ) / 2;
+                // (targets much sparser than the sources)
+                if ( 8 * group <= g.group && __popcll( todo ) > 8 )
+                    tries = max( tries, kGroupTries );
+            }
             else
             {
                 r2_full = r2;
@@ -936,6 +979,7 @@ __global__ void __launch_bounds__( 64 )
                     r2_full = type_max<T>();
                 }
             }
+            ++tries;
             wave_sync();
             continue;
         }
@@ -1073,6 +1117,7 @@ __global__ void __launch_bounds__( 64 )
                             break;
                         beyond = true;
                         limit = type_max<T>();
+                        it -= 2 * kSteps;
                     }
                     below = t;
                 }
@@ -1410,6 +1455,7 @@ __global__ void __launch_bounds__( 64 )
             }
         }
         todo &= ~done;
+        tries += done ? 0 : 1;
         if ( done )
         {
             steps = hard ? 1 : kSteps;

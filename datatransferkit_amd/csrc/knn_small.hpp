@@ -101,9 +101,8 @@ __global__ void __launch_bounds__( kSmallThreads )
         {
             uint32_t q[3];
             curve_cell( pts[i], frame, q );
-            key[s] = hilbert_code<21>( q );
-            if ( !is_src )
-                key[s] >>= kSrcKeyBits - kTgtKeyBits;
+            key[s] = is_src ? hilbert_code<21>( q )
+                            : target_key( pts[i], frame );
         }
     }
     for ( int shift = 0; shift < bits; shift += 8 )

@@ -128,3 +128,67 @@ def test_thin_boxes_stay_in_the_groups(dtk, oracle_lib, box, geometry):
         assert op.stats()["n_stack_overflow"] == 0
         gi, _ = oracle_lib.knn(src, tgt[sample], k, geometry=0 if geometry == "float" else 1)
         assert np.array_equal(op.graph()[1].cpu().numpy()[sample], gi)
+
+
+def outside(rng, n, where):
+    """Targets of the unit box: inside it, beside it, in a box around it."""
+    t = rng.random((n, 3))
+    if where == "beside":
+        t[:, 0] += 2.0
+    return 3.0 * t - 1.0 if where == "around" else t
+
+
+@pytest.mark.parametrize("geometry", ["float", "double"])
+@pytest.mark.parametrize("where", ["beside", "around"])
+def test_targets_outside_cost_no_more_than_their_tree_search(dtk, oracle_lib, where, geometry):
+    """No radius that holds k sources holds few more for a target far outside
+    the sources' box; gathered one at a time such targets took 10 to 20 times
+    the query of targets inside. They go to the tree search at once: at most 6
+    times (1.8 to 3 measured), with the oracle's rows."""
+    rng = np.random.default_rng(11)
+    src, n = rng.random((300_000, 3)), 300_000
+    sample = rng.permutation(n)[:2000]
+    d_src = torch.as_tensor(src).cuda()
+
+    def query(tgt, k):
+        ops = [dtk.MovingLeastSquaresOperator(d_src, torch.as_tensor(tgt).cuda(),
+                                              basis="constant", k=k, geometry=geometry)
+               for _ in range(4)]
+        return ops[0], min(op.stats()["ms_knn_query"] for op in ops)
+
+    for k in (1, 10, 24):
+        print(f"outside: {where} k={k} {geometry}", flush=True)
+        tgt = outside(rng, n, where)
+        _, inside = query(outside(rng, n, "inside"), k)
+        op, ms = query(tgt, k)
+        print(f"  {inside:.3f} ms inside, {ms:.3f} {where}", flush=True)
+        gi, _ = oracle_lib.knn(src, tgt[sample], k, geometry=0 if geometry == "float" else 1)
+        assert np.array_equal(op.graph()[1].cpu().numpy()[sample], gi)
+        assert ms <= 6 * inside
+
+
+@pytest.mark.parametrize("geometry", ["float", "double"])
+@pytest.mark.parametrize("n_tgt", [1, 65, 300, 513, 9000, 140_001])
+@pytest.mark.parametrize("k", [1, 4, 9, 10, 17, 32, 33, 64])
+def test_rows_left_to_the_tree_search(dtk, oracle_lib, k, n_tgt, geometry):
+    """Clouds whose rows the groups leave (more sources at one distance than
+    a wave holds), at list lengths from one row to more than the lanes of the
+    launch over the list, for every form of the tree search."""
+    rng = np.random.default_rng(k)
+    near = rng.standard_normal((900, 3))
+    src = np.concatenate([np.repeat([[0.5, 0.5, 0.5]], 700, axis=0),
+                          4.0 * near / np.linalg.norm(near, axis=1)[:, None]])
+    unique = 0.5 + 1e-3 * rng.standard_normal((min(n_tgt, 500), 3))
+    tgt = unique[np.arange(n_tgt) % len(unique)]
+    print(f"left rows: k={k} n={n_tgt} {geometry}", flush=True)
+    op = dtk.MovingLeastSquaresOperator(torch.as_tensor(src).cuda(), torch.as_tensor(tgt).cuda(),
+                                        basis="constant", k=k, geometry=geometry)
+    assert op.stats()["n_stack_overflow"] == n_tgt
+    idx, dist = dtk.knn(torch.as_tensor(src).cuda(), torch.as_tensor(tgt).cuda(), k,
+                        geometry=geometry, with_distances=True)
+    gi, gd = oracle_lib.knn(src, unique, k, geometry=0 if geometry == "float" else 1)
+    at = np.arange(n_tgt) % len(unique)
+    assert np.array_equal(idx.cpu().numpy(), gi[at])
+    assert np.array_equal(dist.cpu().numpy().view(np.uint64),
+                          np.ascontiguousarray(gd)[at].view(np.uint64))
+    assert np.array_equal(op.graph()[1].cpu().numpy(), gi[at])
