@@ -1710,6 +1710,9 @@ void run_queries( std::vector<KnnBatch::Launch> const &launches,
                 continue;
             switch ( group_slots( l.kmax ) )
             {
+            case 1:
+                launch_group<T, 1>( g, per_target, l.kmax, s );
+                break;
             case 16:
                 launch_group<T, 16>( g, per_target, l.kmax, s );
                 break;

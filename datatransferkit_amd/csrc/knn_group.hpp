@@ -521,10 +521,10 @@ struct GroupArgs
 // takes more), at least one and a half times kk. (k = 8 takes 32: with 16,
 // the counts 7 and 19 around a lattice's node leave every row to the kk-th
 // distance itself, 1.80 ms of query against 0.68 at 1M nodes; uniform points
-// 0.42 either way.)
+// 0.42 either way.) The nearest source alone needs no row.
 constexpr int group_slots( int kk )
 {
-    return kk <= 7 ? 16 : ( kk <= 20 ? 32 : ( kk <= 42 ? 64 : 128 ) );
+    return kk <= 1 ? 1 : kk <= 7 ? 16 : ( kk <= 20 ? 32 : ( kk <= 42 ? 64 : 128 ) );
 }
 
 template <typename T>
@@ -536,7 +536,9 @@ constexpr T type_max()
 template <typename T, int S>
 struct GroupShape
 {
-    static constexpr int kLanes = S == 128 ? 8 : 4; // lanes a row in the sort
+    // lanes a row in the sort (k = 1 needs none: any target of the wave can
+    // be in one gather)
+    static constexpr int kLanes = S == 128 ? 8 : ( S == 1 ? 1 : 4 );
     static constexpr int kKeys = S / kLanes;
     static constexpr int kRows = 64 / kLanes;       // rows a sort
     static constexpr int kChunks = sizeof( T ) == 4 ? 8 : 6;
@@ -1084,6 +1086,87 @@ __global__ void __launch_bounds__( 64 )
                         log_aim - kPower * __builtin_amdgcn_logf( (float)n ) ) );
             ++n_rows;
         };
+        // The nearest source of each target: the least squared distance, and
+        // among those that the rounded root may tie the lowest index. Without
+        // rows a gather serves all 64 targets of a wave: 1M x 1M uniform points
+        // 357 -> 274 us, 3000 sources and 400,000 targets 109 -> 69.
+        if constexpr ( S == 1 )
+        {
+            int32_t my_pos = 0;
+            for ( uint64_t left = sub; left; left &= left - 1 )
+            {
+                left = uniform( left );
+                int const i = __builtin_ctzll( left );
+                T d2[C];
+                distances( i, d2 );
+                T m = T( INFINITY );
+#pragma unroll
+                for ( int c = 0; c < C; ++c )
+                {
+                    if ( c >= chunks )
+                        break;
+                    m = fmin( m, d2[c] );
+                }
+                m = uniform( wave_min( m ) );
+                if ( uniform( (int)!( m <= t_max ) ) )
+                {
+                    T const u = m < type_max<T>() ? m : r2 * T( 2.25 );
+                    need = need > u ? need : u;
+                    lost |= 1ull << i;
+                    continue;
+                }
+                T const limit = m * kMargin;
+                int n = 0;
+                int32_t v = -1;
+#pragma unroll
+                for ( int c = 0; c < C; ++c )
+                {
+                    if ( c >= chunks )
+                        break;
+                    bool const in = d2[c] <= limit;
+                    v = in ? pp[c] : v;
+                    n += __popcll( __ballot( in ) );
+                }
+                uint64_t who = __ballot( v >= 0 );
+                if ( uniform( n ) > 1 )
+                {
+                    T const root = sqrt_rn( m );
+                    int32_t id = INT32_MAX;
+#pragma unroll
+                    for ( int c = 0; c < C; ++c )
+                    {
+                        if ( c >= chunks )
+                            break;
+                        if ( d2[c] <= limit && sqrt_rn( d2[c] ) == root )
+                        {
+                            int32_t const o = g.ids[pp[c]];
+                            v = o < id ? pp[c] : v;
+                            id = o < id ? o : id;
+                        }
+                    }
+                    who = __ballot( id == wave_min_int( id ) );
+                }
+                int32_t const pos = __builtin_amdgcn_readlane(
+                    v, __builtin_ctzll( uniform( who ) ) );
+                my_pos = lane == i ? pos : my_pos;
+                done |= 1ull << i;
+                widest = widest > m ? widest : m;
+            }
+            if ( ( done >> lane ) & 1 )
+            {
+                int64_t const at = a.row_off ? a.row_off[my_row]
+                                             : ( a.src_pos ? my_row : (int64_t)my_t );
+                a.out_idx[at] = a.src_pos ? my_pos : g.ids[my_pos];
+                if ( a.out_dist )
+                {
+                    V const p = g.pts[my_pos];
+                    T const b[3] = {p.x, p.y, p.z};
+                    a.out_dist[at] = (double)sqrt_rn( point_sq( q, b ) );
+                }
+            }
+        }
+        // The k nearest.
+        if constexpr ( S > 1 )
         for ( uint64_t left = sub; left; left &= left - 1 )
         {
             left = uniform( left );
@@ -1177,7 +1260,7 @@ __global__ void __launch_bounds__( 64 )
         // lattice or among copies of a point: the counts jump over the
         // window): the kk-th distance itself, from the rounded roots and
         // without margins, and at it the lowest indices.
-        for ( uint64_t left = hard; left; left &= left - 1 )
+        for ( uint64_t left = S > 1 ? hard : 0; left; left &= left - 1 )
         {
             left = uniform( left );
             n_rows = uniform( n_rows );
@@ -1281,7 +1364,7 @@ __global__ void __launch_bounds__( 64 )
         }
 
         // 3. sort
-        if ( n_rows )
+        if ( S > 1 && n_rows )
         {
             wave_sync();
             int const ol = opaque_lane();
@@ -1478,7 +1561,10 @@ __global__ void __launch_bounds__( 64 )
         else if ( !all )
         {
             guessed = true;
-            r2 = uniform( widest * T( slack ) );
+            // (a gather of a chunk gains nothing from a smaller R: 3000 sources
+            // in 200 clusters of 1e-4, 400,000 targets, k = 10 541 -> 169 us)
+            T const next = widest * T( slack );
+            r2 = uniform( n_cand <= 64 && r2 > next ? r2 : next );
             if ( 5 * n_cand < 2 * Sh::kCand )
                 group = min( 2 * group, g.group );
             if ( !( r2 > T( 0 ) ) )
