@@ -739,17 +739,20 @@ __global__ void __launch_bounds__( 64 )
     int steps = kSteps; // counts of a target: one after a group of ties
     int kk = a.kk;
     // the next group's R^2 over this one's largest: the k-th distances' spread
-    // grows as k falls (1M uniform points, k = 10 / 32: 1.2 + 0.4 k^-1/2 432 /
-    // 580 us, 1.15 + 0.4 k^-1/2 438 / 596, 1 + 0.15 k^-1/2 469 / 624)
-    float const slack = 1.2f + 0.4f * g.root_k;
+    // grows as k falls (1M uniform points, k = 10 / 32 / 64: 1.2 + 0.4 k^-1/2
+    // 431 / 596 / 1175 us, 1.08 + 0.4 k^-1/2 435 / 589 / 1202, 1 + 0.4 k^-1/2
+    // 446 / 599 / 1237)
+    float const slack = 1.14f + 0.4f * g.root_k;
     int64_t beg = 0, end = a.n_src;
-    // counts grow with the 3/2 power of the squared distance; the logarithm
-    // of the count that a first threshold aims at, times 2/3
+    // counts grow with the 3/2 power of the squared distance; logarithms of
+    // kk and of the count that a first threshold aims at, times 2/3
     constexpr float kPower = 0.6666667f;
-    float log_aim = 0.f;
+    float log_kk = 0.f, to_aim = 1.f, log_aim = 0.f;
     auto set_k = [&]() {
+        log_kk = kPower * __builtin_amdgcn_logf( (float)kk );
         log_aim = kPower *
                   __builtin_amdgcn_logf( (float)kk + 0.375f * (float)( S - kk ) );
+        to_aim = __builtin_amdgcn_exp2f( log_aim - log_kk );
     };
     set_k();
 
@@ -1015,7 +1018,6 @@ __global__ void __launch_bounds__( 64 )
         T need = T( 0 ), widest = T( 0 );
         int n_rows = 0;
         int row_lane = first; // the wave's lane of the target of this lane's row
-        T row_top = T( 0 );
         auto distances = [&]( int i, T ( &d2 )[C] ) {
             T const qt[3] = {lane_value( q[0], i ), lane_value( q[1], i ),
                              lane_value( q[2], i )};
@@ -1074,16 +1076,13 @@ __global__ void __launch_bounds__( 64 )
             }
             return at;
         };
-        // target i's row is filled with n candidates up to the squared
-        // distance t; top: what its sort keys are fractions of
-        auto keep_row = [&]( int i, T t, int n, T top ) {
+        // target i's row is filled, its kk-th squared distance about w
+        auto keep_row = [&]( int i, T w ) {
             done |= 1ull << i;
             row_lane = lane / W == n_rows ? i : row_lane;
-            row_top = lane / W == n_rows ? top : row_top;
+            widest = widest > w ? widest : w;
             // the next target's first threshold aims at the window's middle
-            t_last = uniform(
-                t * (T)__builtin_amdgcn_exp2f(
-                        log_aim - kPower * __builtin_amdgcn_logf( (float)n ) ) );
+            t_last = uniform( w * (T)to_aim );
             ++n_rows;
         };
         // The nearest source of each target: the least squared distance, and
@@ -1226,7 +1225,9 @@ __global__ void __launch_bounds__( 64 )
                 // stay in
                 n = uniform( n );
                 if ( uniform( fill_row( d2, t * kMargin ) ) <= S )
-                    keep_row( i, t, n, t );
+                    keep_row( i, t * (T)__builtin_amdgcn_exp2f(
+                                         log_kk - kPower * __builtin_amdgcn_logf(
+                                                               (float)n ) ) );
                 else
                     hard |= 1ull << i;
                 continue;
@@ -1358,9 +1359,7 @@ __global__ void __launch_bounds__( 64 )
                         r[c] = T( INFINITY );
             }
             fill_row( r, root );
-            T const w = root * root;
-            widest = widest > w ? widest : w;
-            keep_row( i, w, n, T( 0 ) );
+            keep_row( i, root * root );
         }
 
         // 3. sort
@@ -1383,17 +1382,6 @@ __global__ void __launch_bounds__( 64 )
             // results of this lane's keys
             int mine = ( valid ? kk : 0 ) - sl * E;
             sort_rows<W, E>( key, sl );
-            // the largest kk-th squared distance, for the next group's R
-            uint32_t kth = key[0];
-#pragma unroll
-            for ( int e = 1; e < E; ++e )
-                kth = ( kk - 1 ) % E == e ? key[e] : kth;
-            T const w = uniform( wave_max(
-                valid && sl == ( kk - 1 ) / E
-                    ? row_top * (T)( kth >> Sh::kSlotBits ) *
-                          (T)( 1. / ( 1u << Sh::kDistBits ) )
-                    : T( 0 ) ) );
-            widest = widest > w ? widest : w;
             // neighbours of a row within the root's rounding (or the key's
             // step), the one past the last result included
             constexpr uint32_t kNear =
@@ -1488,6 +1476,15 @@ __global__ void __launch_bounds__( 64 )
                                 a.out_dist[base + sl * E + e] =
                                     SK::distance( fk[e] );
                         }
+                    // (tied counts do not follow the power law that estimated
+                    // the kk-th distances: the next group's R from the rows)
+                    T w = T( 0 );
+#pragma unroll
+                    for ( int e = 0; e < E; ++e )
+                        if ( valid && sl * E + e == kk - 1 )
+                            w = (T)SK::distance( fk[e] );
+                    w = uniform( wave_max( w ) );
+                    widest = widest > w * w ? widest : w * w;
                 }
             }
             for ( uint64_t left = together ? 0 : closes; left; )
