@@ -288,14 +288,6 @@ __device__ inline int opaque_lane()
     return l;
 }
 
-// order of a wave's own LDS accesses as written
-__device__ inline void wave_sync()
-{
-    __builtin_amdgcn_fence( __ATOMIC_RELEASE, "wavefront" );
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence( __ATOMIC_ACQUIRE, "wavefront" );
-}
-
 // ------------------------------------------------------------ row sort
 __device__ inline bool row_less( uint32_t a, uint32_t b ) { return a < b; }
 __device__ inline bool row_less( uint64_t a, uint64_t b ) { return a < b; }
@@ -628,10 +620,10 @@ __device__ inline T first_radius_sq( BoxLevels<T> const &boxes, int64_t beg,
         bool const mine = ( ( hits >> lane ) & 1 ) && at < 8;
         if ( l <= 2 )
             rad = fminf( rad, wave_min( mine ? r : INFINITY ) );
-        wave_sync();
+        rsort::wave_lds_order();
         if ( mine )
             queue[at] = i;
-        wave_sync();
+        rsort::wave_lds_order();
         n_in = min( __popcll( hits ), 8 );
     }
     T const w = (T)( __builtin_amdgcn_sqrtf( gap ) +
@@ -877,7 +869,7 @@ __global__ void __launch_bounds__( 64 )
                     queue[rsort::lanes_below( m )] = (int32_t)i;
                 n_in = __popcll( m );
             }
-            wave_sync();
+            rsort::wave_lds_order();
             int cur = 0;
             for ( int l = top - 1; l >= 0 && !full; --l )
             {
@@ -912,7 +904,7 @@ __global__ void __launch_bounds__( 64 )
                               rsort::lanes_below( m )] = child;
                     n_out += nm;
                 }
-                wave_sync();
+                rsort::wave_lds_order();
                 cur = Sh::kQueue - cur;
                 n_in = n_out;
             }
@@ -985,10 +977,10 @@ __global__ void __launch_bounds__( 64 )
                 }
             }
             ++tries;
-            wave_sync();
+            rsort::wave_lds_order();
             continue;
         }
-        wave_sync();
+        rsort::wave_lds_order();
         T px[C], py[C], pz[C];
         int32_t pp[C];
         int const chunks = ( n_cand + 63 ) / 64;
@@ -1006,7 +998,7 @@ __global__ void __launch_bounds__( 64 )
                 pp[c] = cpos[i];
             }
         }
-        wave_sync();
+        rsort::wave_lds_order();
 
         // 2. select. t_max: the largest threshold whose margin ends within R
         constexpr T kMargin =
@@ -1051,7 +1043,7 @@ __global__ void __launch_bounds__( 64 )
                                 : T( 0 );
             for ( int s = lane; s < S; s += 64 )
                 rkey[n_rows * Sh::kPitch + s] = ~0u;
-            wave_sync();
+            rsort::wave_lds_order();
             int at = 0;
 #pragma unroll
             for ( int c = 0; c < C; ++c )
@@ -1365,7 +1357,7 @@ __global__ void __launch_bounds__( 64 )
         // 3. sort
         if ( S > 1 && n_rows )
         {
-            wave_sync();
+            rsort::wave_lds_order();
             int const ol = opaque_lane();
             int const row = ol / W, sl = ol % W;
             bool const valid = row < n_rows;
@@ -1567,7 +1559,7 @@ __global__ void __launch_bounds__( 64 )
             if ( !( r2 > T( 0 ) ) )
                 r2 = T( -1 );
         }
-        wave_sync();
+        rsort::wave_lds_order();
     }
 }
 

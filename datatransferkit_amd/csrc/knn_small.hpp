@@ -111,6 +111,7 @@ __global__ void __launch_bounds__( kSmallThreads )
         uint32_t const mask = ( 1u << nbits ) - 1u;
         for ( int i = lane; i < kDigits; i += 64 )
             whist[w][i] = 0;
+        rsort::wave_lds_order();
 #pragma unroll
         for ( int s = 0; s < ITEMS; ++s )
         {
@@ -122,8 +123,10 @@ __global__ void __launch_bounds__( kSmallThreads )
             uint32_t prior = 0;
             if ( ok )
                 prior = whist[w][d];
+            rsort::wave_lds_order();
             if ( ok && below == 0 )
                 whist[w][d] = prior + (uint32_t)__popcll( m );
+            rsort::wave_lds_order();
             rank[s] = prior + below;
         }
         __syncthreads();

@@ -155,6 +155,18 @@ __device__ inline uint32_t lanes_below( uint64_t m )
         __builtin_amdgcn_mbcnt_lo( static_cast<uint32_t>( m ), 0u ) );
 }
 
+// Order of a wave's own LDS accesses as written: what its lanes wrote before
+// is read after, and what they read before is overwritten only after. (The
+// hardware takes a wave's LDS instructions in order; this keeps the compiler
+// from moving one lane's read past another's write, which in one lane's own
+// code do not depend on each other.)
+__device__ inline void wave_lds_order()
+{
+    __builtin_amdgcn_fence( __ATOMIC_RELEASE, "wavefront" );
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence( __ATOMIC_ACQUIRE, "wavefront" );
+}
+
 // The lanes among `ok` whose digit (8 bits) equals this lane's: one ballot a
 // bit, each taken as it is or inverted by the lane's own bit spread over a
 // word, so that a bit costs four vector instructions (a choice of the ballot
@@ -255,6 +267,7 @@ __device__ void sort_tile( Array const &A, int pass, int tile, Smem &sm )
 
     for ( int i = lane; i < kDigits; i += 64 )
         sm.whist[w][i] = 0;
+    wave_lds_order();
 
     Key key[kItems];
     int32_t val[kItems];
@@ -280,8 +293,11 @@ __device__ void sort_tile( Array const &A, int pass, int tile, Smem &sm )
         uint32_t prior = 0;
         if ( ok )
             prior = sm.whist[w][d];
+        // every lane of the digit has read the count that the first one adds to
+        wave_lds_order();
         if ( ok && below == 0 )
             sm.whist[w][d] = prior + static_cast<uint32_t>( __popcll( m ) );
+        wave_lds_order();
         rank[s] = prior + below;
     }
     __syncthreads();
