@@ -1608,10 +1608,23 @@ void enqueue_build( dtkx_mls_batch *b, StageEvents *ev )
     bool const f32 = o.precision == DTKX_PRECISION_FP32_BULK;
     bool const cyclic = f32 || o.solver != DTKX_SOLVER_CLASSICAL_JACOBI;
     int group_used = 0;
+    // one scratch for the groups' listed rows (their setups follow each other
+    // on the stream): a captured build keeps its temporaries for the graph's
+    // lifetime
+    dtkx::DeviceBuffer<double> tangents;
+    if ( cyclic && o.solver == DTKX_SOLVER_CHOLESKY )
+    {
+        std::size_t need = 1;
+        for ( auto const &g : b->groups )
+            need = std::max( need,
+                             dtkx::setup_listed_scratch( g.m, g.r1 - g.r0 ) );
+        tangents.resize( need, s );
+    }
     for ( auto &g : b->groups )
     {
         dtkx::SetupParams p;
         p.m = g.m;
+        p.tangents = tangents.get();
         p.kk = 0;
         p.rbf = o.rbf;
         p.geometry = o.geometry;

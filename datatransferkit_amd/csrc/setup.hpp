@@ -41,6 +41,10 @@ struct SetupParams
     // unconverged systems are counted for truncated rows only (it counted
     // the others)
     bool screened = false;
+    // Cholesky solver (nullable): its listed rows' scratch, of at least
+    // setup_listed_scratch( m, rows ) doubles, which setups of one stream may
+    // share; else it is allocated for the call
+    double *tangents = nullptr;
 };
 
 // counters[0] = n_underdetermined, [1] = n_unconverged, [2] = rotations
@@ -76,6 +80,7 @@ void setup_cyclic( double4 const *src, double4 const *tgt, int64_t n_tgt,
 // truncation test are appended to p.refine_rows; the others' coefficients
 // are written, but for the few appended to full_rows, which its counters
 // leave out. coeffs32 as in setup_cyclic; *queue is zero before.
+std::size_t setup_listed_scratch( int m, int64_t rows );
 void setup_listed( double4 const *src, double4 const *tgt, int64_t n_tgt,
                    int32_t const *indices, int32_t const *order,
                    SetupParams const &p, double *coeffs, float *coeffs32,

@@ -411,9 +411,17 @@ void launch_cyclic( double4 const *src, double4 const *tgt, int64_t n_tgt,
 // cost nothing beside the rotations; tiles from a queue instead of a stride
 // 797 -> 688 us of the kernel, as 4,688 tiles over 2,048 blocks leave some
 // with a third; gathers four neighbours at a time gave nothing.
-constexpr int kKeptSweeps = 10;
-// two waves a SIMD at this kernel's registers
+// Seven regions keep six sweeps: the shell's rows take 4.3 on average, and
+// seven regions measure as ten do (setup 1.04-1.06 ms), at 330 MB of scratch
+// instead of 472.
+constexpr int kKeptSweeps = 7;
+// two waves a SIMD at this kernel's registers (one: 1.21 ms)
 constexpr int kListedBlocks = 2048;
+
+int64_t listed_blocks( int64_t rows )
+{
+    return std::min<int64_t>( ceil_div( rows, kBlock ), kListedBlocks );
+}
 
 template <int M, bool F32>
 __global__ void __launch_bounds__( kBlock, 2 )
@@ -533,6 +541,13 @@ __global__ void __launch_bounds__( kBlock, 2 )
 
 } // namespace
 
+std::size_t setup_listed_scratch( int m, int64_t rows )
+{
+    int const n = m == 10 ? rotations<10> : ( m == 4 ? rotations<4> : 0 );
+    return static_cast<std::size_t>( listed_blocks( rows ) ) * kKeptSweeps * n *
+           kLanes;
+}
+
 void setup_listed( double4 const *src, double4 const *tgt, int64_t n_tgt,
                    int32_t const *indices, int32_t const *order,
                    SetupParams const &p, double *coeffs, float *coeffs32,
@@ -544,19 +559,23 @@ void setup_listed( double4 const *src, double4 const *tgt, int64_t n_tgt,
     if ( n_tgt <= p.row0 )
         return;
     int const sweeps = p.max_rot > 0 ? static_cast<int>( p.max_rot ) : 30;
-    int64_t const blocks = std::min<int64_t>(
-        ceil_div( n_tgt - p.row0, kBlock ), kListedBlocks );
+    int64_t const blocks = listed_blocks( n_tgt - p.row0 );
+    DeviceBuffer<double> owned;
+    double *tangents = p.tangents;
+    if ( !tangents )
+    {
+        owned.resize( std::max<std::size_t>(
+                          setup_listed_scratch( p.m, n_tgt - p.row0 ), 1 ),
+                      s );
+        tangents = owned.get();
+    }
     auto run = [&]( auto m, auto f32 ) {
         constexpr int kM = decltype( m )::value;
-        DeviceBuffer<double> tangents(
-            std::max<std::size_t>(
-                blocks * kKeptSweeps * rotations<kM> * kLanes, 1 ),
-            s );
         eigen_listed_kernel<kM, decltype( f32 )::value>
             <<<blocks, kBlock, 0, s>>>(
                 src, tgt, indices, order, p.row_off, p.rows, p.n_rows, p.kk,
                 p.rbf, p.geometry, p.truncation, p.rcond, sweeps, coeffs,
-                coeffs32, tangents.get(), counters, p.by_distance, p.refine_rows,
+                coeffs32, tangents, counters, p.by_distance, p.refine_rows,
                 p.n_refine, full_rows, n_full, queue );
     };
     using T = std::true_type;
