@@ -1,11 +1,13 @@
 """The search by groups of targets at the sizes where it changes: below and
 above the 64 sources it starts at, the source counts that it takes whole and
-the first ones it gathers, partial blocks, groups and waves, the neighbour
-counts at which the row slots change; and the clouds that drive its radius:
-copies of a point beyond a row's slots, lattices (every distance tied), tight
-clusters beside a thin background, targets outside the sources' box. Indices
-and distances equal the oracle's brute-force order bit for bit, in both
-geometries."""
+the first ones it gathers, partial blocks, the neighbour counts at which the
+row slots change; and the clouds that drive its radius: copies of a point
+beyond a row's slots, lattices (every distance tied), tight clusters beside a
+thin background, targets outside the sources' box. A wave takes fewer targets
+where a launch has few (one below 8,192), so these clouds run again at target
+counts that fill waves and groups, with a partial last wave, alone and in a
+batch. Indices and distances equal the oracle's brute-force order bit for bit,
+in both geometries."""
 import numpy as np
 import pytest
 
@@ -53,21 +55,98 @@ def test_target_counts(dtk, oracle_lib, geometry, n_tgt):
         check(dtk, oracle_lib, src, tgt, k, geometry)
 
 
-@pytest.mark.parametrize("geometry", ["float", "double"])
-def test_hard_clouds(dtk, oracle_lib, geometry):
-    rng = np.random.default_rng(5)
+def hard_sources(rng):
     lattice = grid_points((20, 20, 20), (0, 0, 0)) / 19.0
     flat = rng.random((6000, 3)) * np.array([1.0, 1.0, 0.0])
     line = rng.random((6000, 3)) * np.array([1.0, 0.0, 0.0])
     copies = np.repeat(rng.random((60, 3)), 150, axis=0)
     cluster = np.concatenate([0.5 + 1e-4 * rng.standard_normal((8000, 3)),
                               rng.random((300, 3))])
-    for src in (lattice, flat, line, copies, cluster):
-        near = src[rng.integers(0, len(src), 700)]
-        tgt = np.concatenate([near, near + 1e-5 * rng.standard_normal(near.shape),
-                              rng.random((400, 3)), 30 * rng.random((50, 3))])
+    return {"lattice": lattice, "flat": flat, "line": line, "copies": copies,
+            "cluster": cluster}
+
+
+def hard_targets(rng, src, n):
+    """About n targets: sources, points beside sources, in the box, beyond it."""
+    near = src[rng.integers(0, len(src), 3 * n // 8)]
+    return np.concatenate([near, near + 1e-5 * rng.standard_normal(near.shape),
+                           rng.random((n // 5, 3)), 30 * rng.random((n // 40 + 1, 3))])
+
+
+@pytest.mark.parametrize("geometry", ["float", "double"])
+def test_hard_clouds(dtk, oracle_lib, geometry):
+    rng = np.random.default_rng(5)
+    for src in hard_sources(rng).values():
+        tgt = hard_targets(rng, src, 1850)
         for k in (4, 10, 32, 64):
             check(dtk, oracle_lib, src, tgt, k, geometry)
+
+
+@pytest.mark.parametrize("geometry", ["float", "double"])
+@pytest.mark.parametrize("cloud", ["lattice", "flat", "line", "copies", "cluster"])
+def test_hard_clouds_in_full_groups(dtk, oracle_lib, cloud, geometry):
+    """64 targets a wave from 524,288 targets on for k <= 16, 32 from 262,144
+    for larger k: waves and groups of every kind of target, finished together,
+    in part or one by one."""
+    rng = np.random.default_rng(9)
+    src = hard_sources(rng)[cloud]
+    for n, ks in ((550_000, (1, 4, 10)), (280_000, (20, 32, 64))):
+        tgt = hard_targets(rng, src, n)
+        assert len(tgt) > (524_288 if ks[0] == 1 else 262_144) and len(tgt) % 64
+        sample = rng.permutation(len(tgt))[:3000]
+        d_src, d_tgt = torch.as_tensor(src).cuda(), torch.as_tensor(tgt).cuda()
+        for k in ks:
+            print(f"full groups: {cloud} {len(src)} -> {len(tgt)}, k={k}, {geometry}", flush=True)
+            idx, dist = dtk.knn(d_src, d_tgt, k, geometry=geometry, with_distances=True)
+            gi, gd = oracle_lib.knn(src, tgt[sample], k,
+                                    geometry=0 if geometry == "float" else 1)
+            assert np.array_equal(idx.cpu().numpy()[sample], gi)
+            assert np.array_equal(dist.cpu().numpy()[sample].view(np.uint64),
+                                  np.ascontiguousarray(gd).view(np.uint64))
+
+
+@pytest.mark.parametrize("k", [10, 33])
+@pytest.mark.parametrize("geometry", ["float", "double"])
+def test_hard_clouds_in_a_batch(dtk, k, geometry):
+    """Problems of hard clouds, small clouds and clouds of other scales in the
+    waves of one batch: each equals its own operator."""
+    rng = np.random.default_rng(12)
+    clouds = list(hard_sources(rng).values())
+    clouds += [rng.random((n, 3)) * s for n, s in ((70, 1.0), (200, 1e-7), (300, 1e6), (k, 1.0))]
+    probs = []
+    for i in range(27):
+        src = clouds[i % len(clouds)]
+        n = int(rng.integers(9000, 15000)) if i else 170_000
+        probs.append((torch.as_tensor(src).cuda(),
+                      torch.as_tensor(hard_targets(rng, src, n) * np.abs(src).max()).cuda()))
+    print(f"hard batch k={k} {geometry} {sum(len(t) for _, t in probs)}", flush=True)
+    batch = dtk.MovingLeastSquaresBatch([(s, t, "constant", k) for s, t in probs],
+                                        geometry=geometry)
+    xs = [torch.as_tensor(rng.random(len(s))).cuda() for s, _ in probs]
+    ys = [torch.zeros(len(t), dtype=torch.float64, device="cuda") for _, t in probs]
+    batch.rebuild()
+    batch.apply(xs, ys)
+    for (s, t), x, y in zip(probs, xs, ys):
+        op = dtk.MovingLeastSquaresOperator(s, t, basis="constant", k=k, geometry=geometry)
+        assert torch.equal(op.apply(x, torch.empty_like(y)), y)
+
+
+@pytest.mark.parametrize("geometry", ["float", "double"])
+@pytest.mark.parametrize("scale", [1e-9, 1e-7, 1.0, 1e6])
+def test_small_clouds_of_any_scale(dtk, oracle_lib, scale, geometry):
+    """Clouds that a wave takes whole, in other units: no row is left to the
+    tree search (its first threshold was a distance of 1)."""
+    rng = np.random.default_rng(4)
+    for n_src in (64, 192, 200, 256):
+        src, tgt = scale * rng.random((n_src, 3)), scale * rng.random((3000, 3))
+        d_src, d_tgt = torch.as_tensor(src).cuda(), torch.as_tensor(tgt).cuda()
+        for k in (1, 3, 16, 40):
+            print(f"scale {scale} {n_src} k={k} {geometry}", flush=True)
+            op = dtk.MovingLeastSquaresOperator(d_src, d_tgt, basis="constant", k=k,
+                                                geometry=geometry)
+            assert op.stats()["n_stack_overflow"] == 0
+            gi, _ = oracle_lib.knn(src, tgt, k, geometry=0 if geometry == "float" else 1)
+            assert np.array_equal(op.graph()[1].cpu().numpy(), gi)
 
 
 TIED = {

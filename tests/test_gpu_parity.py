@@ -10,10 +10,13 @@ Bars (integer/index work bit-exact; floating point per the plain FP64 form):
     are counted and bounded.
   * the reference's own MLS tests at their tolerances.
 """
+import os
+import re
+
 import numpy as np
 import pytest
 
-from conftest import c1_inputs, grid_points, load_golden, poly_for_basis
+from conftest import REPO, c1_inputs, grid_points, load_golden, poly_for_basis
 
 pytestmark = pytest.mark.gpu
 
@@ -188,8 +191,9 @@ def test_knn_deep_tree_overflow_rerun(dtk, oracle_lib, geometry):
 
 @pytest.mark.parametrize("geometry", ["float", "double"])
 def test_knn_overflow_rerun_strides_over_many_rows(dtk, oracle_lib, geometry):
-    """More overflowing queries (20,000) than the re-run has lanes (16,384),
-    so lanes take several listed rows and reuse their global stack.
+    """More overflowing queries (240,000) than the launch over the list has
+    lanes (3584 blocks of 64), so lanes take several listed rows and reuse
+    their global stack.
 
     Sources: pairs at (2^-i, 2^-i, 2^-i), i = 1..21, and 16 copies of the
     origin; k = all 58 sources; every query at the origin. The hierarchy is
@@ -198,13 +202,16 @@ def test_knn_overflow_rerun_strides_over_many_rows(dtk, oracle_lib, geometry):
     distance covers every pair, so each of the 21 levels pushes its pair,
     and the 16 duplicates (split by index, 4 levels at distance 0) push 3
     more: 24 entries, past the 22-entry LDS stack, for every query. So one
-    query gives a count of 1 and 20,000 give 20,000; the rows must equal
+    query gives a count of 1 and 240,000 give 240,000; the rows must equal
     the oracle's."""
     chain = np.repeat(np.array([[2.0 ** -i] * 3 for i in range(1, 22)]), 2, axis=0)
     src = np.concatenate([chain, np.zeros((16, 3))])
     k = len(src)
     g = 0 if geometry == "float" else 1
-    n = 20_000
+    n = 240_000
+    with open(os.path.join(REPO, "datatransferkit_amd", "csrc", "knn.hip")) as f:
+        blocks = int(re.search(r"kListBlocks = (\d+);", f.read()).group(1))
+    assert n > 64 * blocks, "no more rows than lanes"
     print(f"overflow rerun geometry={geometry} n_tgt={n} k={k}", flush=True)
 
     def make(t):

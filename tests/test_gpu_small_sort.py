@@ -21,8 +21,8 @@ def dtk():
 
 @pytest.mark.parametrize("geometry", ["float", "double"])
 @pytest.mark.parametrize("n_src,n_tgt", [
-    (1, 1), (64, 63), (2047, 2049), (2048, 65), (4096, 4097), (8193, 8192), (8192, 8190),
-    (12288, 12288), (12289, 900), (700, 12289)])
+    (1, 1), (64, 63), (2047, 2049), (2048, 65), (4096, 4097), (8193, 8192), (8192, 8192), (8192, 8193),
+    (12289, 900), (700, 12289)])
 def test_small_sorts(dtk, oracle_lib, geometry, n_src, n_tgt):
     rng = np.random.default_rng(n_src + n_tgt)
     src, tgt = rng.random((n_src, 3)), rng.random((n_tgt, 3))
