@@ -1077,6 +1077,15 @@ __global__ void __launch_bounds__( 64 )
             t_last = uniform( w * (T)to_aim );
             ++n_rows;
         };
+        // R^2 of the next gather where this one held too few and no candidate
+        // says how far the rest is
+        auto wider = [&]() {
+            if ( __popcll( sub ) > 1 )
+                return r2 * T( 2.25 );
+            r2_few = r2;
+            return r2_full < type_max<T>() ? T( 0.5 ) * ( r2_few + r2_full )
+                                           : r2 * T( 2.25 );
+        };
         // The nearest source of each target: the least squared distance, and
         // among those that the rounded root may tie the lowest index. Without
         // rows a gather serves all 64 targets of a wave: 1M x 1M uniform points
@@ -1101,7 +1110,7 @@ __global__ void __launch_bounds__( 64 )
                 m = uniform( wave_min( m ) );
                 if ( uniform( (int)!( m <= t_max ) ) )
                 {
-                    T const u = m < type_max<T>() ? m : r2 * T( 2.25 );
+                    T const u = m < type_max<T>() ? m : wider();
                     need = need > u ? need : u;
                     lost |= 1ull << i;
                     continue;
@@ -1236,16 +1245,7 @@ __global__ void __launch_bounds__( 64 )
             }
             T u = found ? t : above;
             if ( !( u < type_max<T>() ) )
-            {
-                u = r2 * T( 2.25 );
-                if ( __popcll( sub ) == 1 )
-                {
-                    r2_few = r2;
-                    u = r2_full < type_max<T>()
-                            ? T( 0.5 ) * ( r2_few + r2_full )
-                            : u;
-                }
-            }
+                u = wider();
             need = need > u ? need : u;
             lost |= 1ull << i;
         }
@@ -1550,10 +1550,10 @@ __global__ void __launch_bounds__( 64 )
         else if ( !all )
         {
             guessed = true;
-            // (a gather of a chunk gains nothing from a smaller R: 3000 sources
-            // in 200 clusters of 1e-4, 400,000 targets, k = 10 541 -> 169 us)
+            // (so small a gather gains nothing from a smaller R: 1M points on a line,
+            // k = 1 355 -> 285 us)
             T const next = widest * T( slack );
-            r2 = uniform( n_cand <= 64 && r2 > next ? r2 : next );
+            r2 = uniform( n_cand <= 32 && r2 > next ? r2 : next );
             if ( 5 * n_cand < 2 * Sh::kCand )
                 group = min( 2 * group, g.group );
             if ( !( r2 > T( 0 ) ) )
