@@ -180,7 +180,7 @@ __global__ void __launch_bounds__( kBlock )
 // whole-record reads. Stored straight from the rows, targets in random
 // caller order scatter one value per field and row: at 1M x 1M (k = 32,
 // 4 float fields) the apply took 0.211 ms against 0.142 ms for the same
-// targets given in Hilbert order, and 0.163 ms staged.
+// targets given in Morton order, and 0.163 ms staged.
 template <typename X, int NF>
 __global__ void __launch_bounds__( kBlock )
     records_to_caller_kernel( Pack<X, NF> const *__restrict__ rec,

@@ -221,10 +221,9 @@ void invert_permutation( int32_t const *perm, int64_t n, int32_t *inv,
 // hands consecutive workgroups to the 8 XCDs in turn (each XCD with its own
 // L2). A bijection of [0, gridDim.x) in one of two shapes:
 //  * kChunk = 0: each XCD takes one contiguous eighth of the tiles, so the
-//    spatially adjacent work of Hilbert-ordered rows shares an L2. The kNN
-//    queries use this: an XCD's L2 then holds the subtrees of its own region
-//    only (2.03 ms for the 1M x 1M, k = 32 query, against 2.06-2.13 ms with
-//    chunks of 32-512 tiles).
+//    spatially adjacent work of curve-ordered rows shares an L2. The kNN
+//    queries use this: an XCD's L2 then holds the nodes of its own region
+//    only.
 //  * kChunk > 0: the tiles are cut into chunks of kChunk consecutive tiles,
 //    and chunk j goes to XCD j mod 8, each XCD taking its chunks in order:
 //    adjacent work inside a chunk still shares an L2, and the eight XCDs

@@ -7,9 +7,9 @@
 // order) -> the boxes of 8, 64, 512, ... consecutive sources.
 // Query: groups of targets that are consecutive on the curve (knn_group.hpp).
 // The exact k smallest (distance, index) pairs of each target, as brute force
-// gives. 1M x 1M uniform points, build and query: k = 32 0.94 ms, k = 10
-// 0.72 ms, k = 1 0.65 ms (one tree traversal a lane over the hierarchy below
-// took 2.14, 1.00 and 0.64).
+// gives. 1M x 1M uniform points, build and query: k = 32 0.84 ms, k = 10
+// 0.69 ms, k = 1 0.54 ms (one tree traversal a lane over the hierarchy below
+// took 2.11, 1.00 and 0.64).
 //
 // The rows that the groups leave (targets far outside the sources' box or in
 // the middle of a hollow cloud, where a sphere that holds k sources holds
@@ -224,7 +224,7 @@ __device__ inline void curve_cell( V p, CurveFrame const &f, uint32_t *q )
 // then a Gray decode across the axes. The code of q >> s is the code of q
 // without its last 3 s bits, so a prefix of 3 L bits names an octree cell,
 // one further bit a half and two a quarter of one. Consecutive cells share
-// a face: a run of consecutive points, unlike one in Hilbert order, never
+// a face: a run of consecutive points, unlike one in Morton order, never
 // jumps, and its box stays small (the sources within the k-th distance of
 // 16 consecutive targets number 223 against 360, the 8-point blocks they
 // lie in 55 against 102: uniform points, k = 32).
@@ -2101,7 +2101,7 @@ void knn_batched_impl( void const *src_v, int64_t n_src, void const *tgt_v,
 
     // Two stable radix sorts of both point sets, in shared launches
     // (radix_sort.hpp): by Hilbert code in the problem's box (sources 63 bits,
-    // targets 30, as one problem's search orders them), then by the
+    // targets 48, as one problem's search orders them), then by the
     // problem's key (sources: the problem; targets: its row key). The second
     // sorts positions of the first, and its last pass gathers the first's
     // indices (and the sources' codes) into the final order.

@@ -30,11 +30,11 @@
 // with most lanes of its wave masked off, some 40,000 a target at k = 32.
 // Here a target costs about 16 a chunk of 64 candidates (four to five chunks
 // at k = 32), a sixteenth of the group's gather and of the sort. 1M x 1M
-// uniform points, the query alone: k = 32 0.64 ms against 1.97 ms, k = 10
-// 0.43 against 0.69, k = 1 0.37 against 0.34 (whose hierarchy took another
+// uniform points, the query alone: k = 32 0.59 ms against 1.82 ms, k = 10
+// 0.43 against 0.69, k = 1 0.27 against 0.32 (whose hierarchies took another
 // 0.08 to build); 9e4 x 1e5 with k = 64 0.23 against 0.57. What bounds it now
-// is instruction issue (16,400 vector and 11,000 scalar instructions a wave
-// of 64 targets at k = 32, four waves a SIMD): no HBM figure is near.
+// is instruction issue (7,450 vector and 4,950 scalar instructions a wave
+// of 32 targets at k = 32, four waves a SIMD): no HBM figure is near.
 //
 // Exactness: distances are formed in the operation order of box_sq, box
 // distances per axis from the same rounded differences, and rounding is

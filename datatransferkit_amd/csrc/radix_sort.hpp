@@ -34,7 +34,7 @@ namespace rsort
 
 // 16 waves of 8 keys a lane, 8192 keys a tile (112 KB of LDS, one block
 // per CU). Per pass at 2^20 source keys (with the targets' 2^20 in the
-// first four passes), with 4096-key tiles of 16 waves: 18-19 us alone,
+// passes that they share), with 4096-key tiles of 16 waves: 18-19 us alone,
 // 29-34 us with the targets; 4 waves of 16 keys took 29 / 38-46 us.
 // Fewer, larger tiles shorten the look-back chains, which outweighs the
 // CUs they leave idle: the kNN build (scene box to hierarchy, 1M x 1M)

@@ -158,9 +158,9 @@ typedef struct dtkx_mls_stats {
     double ms_knn;              /* stage times of the last create, measured */
     double ms_setup;            /* with HIP events on the handle's stream   */
     int32_t group_size_used;
-    int32_t n_stack_overflow;   /* kNN queries re-run by the tree search with
-                                   a global stack: deeper than the LDS one,
-                                   or left by the group search */
+    int32_t n_stack_overflow;   /* kNN queries left to the tree search over a
+                                   list: by the group search, or deeper than
+                                   the LDS stack */
     double ms_knn_query;        /* the kNN query kernels alone */
     int64_t n_eigen_fallback;   /* Cholesky solver: systems not certified,
                                    set up by the cyclic eigen-solver */
