@@ -279,8 +279,8 @@ APPLY_KERNELS = {
 
 def query_kernel(geo, k):
     """The query kernel the library launches for k results: the group search
-    with the row slots that k takes (16, 32, 64 or 128)."""
-    slots = 16 if k <= 8 else 32 if k <= 20 else 64 if k <= 42 else 128
+    with the row slots that k takes (1, 16, 32, 64 or 128)."""
+    slots = 1 if k <= 1 else 16 if k <= 7 else 32 if k <= 20 else 64 if k <= 42 else 128
     return f"knn_group_kernel<{geo},{slots}>"
 
 
