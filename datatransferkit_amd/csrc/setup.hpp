@@ -33,10 +33,6 @@ struct SetupParams
     int32_t const *n_rows = nullptr;
     // every row is in the search's order, ascending by distance
     bool by_distance = false;
-    // cyclic solver over a row list (nullable): rows whose eigenvalues all
-    // pass the truncation test are appended here (device count n_refine)
-    int32_t *refine_rows = nullptr;
-    int32_t *n_refine = nullptr;
     // cyclic solver over rows that setup_listed left: the sweeps and
     // unconverged systems are counted for truncated rows only (it counted
     // the others)
@@ -77,14 +73,16 @@ void setup_cyclic( double4 const *src, double4 const *tgt, int64_t n_tgt,
 // The listed rows p.rows[0 .. *p.n_rows) by their eigenvalues: the cyclic
 // Jacobi of setup_cyclic (the same rotations of A, so the same eigenvalues,
 // sweeps and convergence) without V. Rows whose eigenvalues all pass the
-// truncation test are appended to p.refine_rows; the others' coefficients
-// are written, but for the few appended to full_rows, which its counters
-// leave out. coeffs32 as in setup_cyclic; *queue is zero before.
+// truncation test are solved again by Cholesky, the others from their
+// rotations; the few that neither can take are appended to full_rows
+// (*n_full), and its counters leave out those of them with an eigenvalue
+// below the threshold. coeffs32 as in setup_cyclic; *n_full and the four
+// counts are zero before.
 std::size_t setup_listed_scratch( int m, int64_t rows );
 void setup_listed( double4 const *src, double4 const *tgt, int64_t n_tgt,
                    int32_t const *indices, int32_t const *order,
                    SetupParams const &p, double *coeffs, float *coeffs32,
-                   int32_t *full_rows, int32_t *n_full, int32_t *queue,
+                   int32_t *full_rows, int32_t *n_full, int32_t *counts,
                    unsigned long long *counters, hipStream_t s );
 
 // Certified Cholesky fast path (DTKX_SOLVER_CHOLESKY): each system is

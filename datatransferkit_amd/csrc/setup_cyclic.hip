@@ -33,9 +33,7 @@ namespace
 using namespace cyc;
 constexpr int kBlock = 64;
 
-// One listed or ranged row's neighbour list, target and radius
-// (row_reach), with its moments (upper triangle) written
-// to A. Shared by the eigen-solver's two kernels, so both form the same bits.
+// One listed or ranged row's neighbour list, target and radius (row_reach).
 struct SystemRow
 {
     int64_t rbeg;
@@ -47,15 +45,13 @@ struct SystemRow
 
 template <int M, bool F32>
 __device__ __forceinline__ SystemRow
-    system_moments( bool valid, int64_t slot, double4 const *__restrict__ src,
-                    double4 const *__restrict__ tgt,
-                    int32_t const *__restrict__ indices,
-                    int32_t const *__restrict__ order,
-                    int64_t const *__restrict__ row_off, int kk_uniform,
-                    int rbf, int geometry, bool by_distance,
-                    double *A )
+    system_row( bool valid, int64_t slot, double4 const *__restrict__ src,
+                double4 const *__restrict__ tgt,
+                int32_t const *__restrict__ indices,
+                int32_t const *__restrict__ order,
+                int64_t const *__restrict__ row_off, int kk_uniform,
+                int geometry, bool by_distance )
 {
-    using S = SymIdx<M>;
     int64_t const t = valid ? ( order ? order[slot] : slot ) : 0;
     int64_t const rbeg =
         valid ? ( row_off ? row_off[slot] : slot * kk_uniform ) : 0;
@@ -67,16 +63,35 @@ __device__ __forceinline__ SystemRow
 
     double const dmax = row_reach<M, F32>( geometry, by_distance, src, nbr, kk, tp );
     double const radius = F32 ? (double)( 1.1f * (float)dmax ) : 1.1 * dmax;
+    return SystemRow{rbeg, kk, nbr, tp, radius};
+}
+
+// A row with its moments (upper triangle) written to A. Shared by the
+// kernels below, so all form the same bits.
+template <int M, bool F32>
+__device__ __forceinline__ SystemRow
+    system_moments( bool valid, int64_t slot, double4 const *__restrict__ src,
+                    double4 const *__restrict__ tgt,
+                    int32_t const *__restrict__ indices,
+                    int32_t const *__restrict__ order,
+                    int64_t const *__restrict__ row_off, int kk_uniform,
+                    int rbf, int geometry, bool by_distance,
+                    double *A )
+{
+    using S = SymIdx<M>;
+    SystemRow const sr =
+        system_row<M, F32>( valid, slot, src, tgt, indices, order, row_off,
+                            kk_uniform, geometry, by_distance );
 
 #pragma unroll
     for ( int e = 0; e < S::size; ++e )
         A[e] = 0.0;
     if ( valid )
-        for ( int l = 0; l < kk; ++l )
+        for ( int l = 0; l < sr.kk; ++l )
         {
             double P[M];
-            double const phi =
-                nbr_row<M, F32>( geometry, rbf, radius, src[nbr[l]], tp, P );
+            double const phi = nbr_row<M, F32>( geometry, rbf, sr.radius,
+                                                src[sr.nbr[l]], sr.tp, P );
 #pragma unroll
             for ( int r = 0; r < M; ++r )
             {
@@ -86,7 +101,7 @@ __device__ __forceinline__ SystemRow
                     A[S::at( r, c )] = fma( pr, P[c], A[S::at( r, c )] );
             }
         }
-    return SystemRow{rbeg, kk, nbr, tp, radius};
+    return sr;
 }
 
 // Truncation threshold of a system's eigenvalues (DBL_EPSILON, or rcond
@@ -116,9 +131,6 @@ __device__ __forceinline__ bool truncated( double const *A, int truncation,
 // 256 VGPRs): every lane of the pair keeps the whole moment matrix and runs
 // the same rotations on it (identical values, so both agree), and owns
 // R = M / H rows of V.
-// refine_rows (the Cholesky setup's fallback rows, nullable): systems whose
-// eigenvalues all pass the truncation test are listed there, to be solved
-// again by Cholesky (setup_fast.hip, refine_kernel).
 template <int M, int H, bool F32, bool STORE>
 __device__ __forceinline__ void
     cyclic_system( int64_t const li, double4 const *__restrict__ src,
@@ -135,8 +147,7 @@ __device__ __forceinline__ void
                          double *__restrict__ pinv_out,
                          unsigned long long *__restrict__ counters,
                          bool by_distance,
-                         int32_t *__restrict__ refine_rows,
-                         int32_t *__restrict__ n_refine, bool screened )
+                         bool screened )
 {
     using S = SymIdx<M>;
     constexpr int R = M / H;
@@ -297,8 +308,6 @@ __device__ __forceinline__ void
             coeffs[rbeg + l] = acc * phi;
         }
     }
-    if ( refine_rows && h == 0 && !under )
-        refine_rows[atomicAdd( n_refine, 1 )] = (int32_t)slot;
     // (a screened list's untruncated rows had their sweeps counted by the
     // screen)
     if ( counters && h == 0 )
@@ -334,8 +343,7 @@ __global__ void __launch_bounds__( kBlock )
                          double *__restrict__ pinv_out,
                          unsigned long long *__restrict__ counters,
                          bool by_distance,
-                         int32_t *__restrict__ refine_rows,
-                         int32_t *__restrict__ n_refine, bool screened )
+                         bool screened )
 {
     constexpr int SPB = kBlock / H;
     auto one = [&]( int64_t tile ) {
@@ -343,7 +351,7 @@ __global__ void __launch_bounds__( kBlock )
             tile * SPB + threadIdx.x / H, src, tgt, n_tgt, indices, order, row0,
             row_off, rows, n_rows, kk_uniform, rbf, geometry, truncation, rcond,
             max_sweeps, coeffs, coeffs32, pinv_out, counters, by_distance,
-            refine_rows, n_refine, screened );
+            screened );
     };
     if constexpr ( LIST )
     {
@@ -381,8 +389,7 @@ void launch_cyclic( double4 const *src, double4 const *tgt, int64_t n_tgt,
                                      p.row_off, p.rows, p.n_rows, p.kk,
                                      p.rbf, p.geometry, p.truncation, p.rcond,
                                      sweeps, coeffs, coeffs32, pinv, counters,
-                                     p.by_distance, p.refine_rows, p.n_refine,
-                                     p.screened );
+                                     p.by_distance, p.screened );
     };
     using T = std::true_type;
     using F = std::false_type;
@@ -400,8 +407,11 @@ void launch_cyclic( double4 const *src, double4 const *tgt, int64_t n_tgt,
 // (kept for each wave and sweep; the last region takes all later sweeps and
 // is not read). The operations are cyclic_system's and a converged system's
 // rotations exact no-ops whatever its wave, so all results are its bit for
-// bit. Truncated rows that need more sweeps than are kept, or that hold a
-// value that is not finite, go to full_rows (cyclic_system, from their start).
+// bit. A wave with few truncated rows, or a row that took more sweeps than
+// are kept, leaves those to a second pass (listed_rest_kernel), where the
+// waves are full and ten regions kept; what still needs more there, or holds
+// a value that is not finite, goes to full_rows (cyclic_system, from their
+// start).
 //
 // Bound by the FP64 of the rotations (a division chain and 64 fused
 // operations on A, 45 a sweep). A and V together (155 doubles) took two lanes
@@ -415,6 +425,15 @@ void launch_cyclic( double4 const *src, double4 const *tgt, int64_t n_tgt,
 // seven regions measure as ten do (setup 1.04-1.06 ms), at 330 MB of scratch
 // instead of 472.
 constexpr int kKeptSweeps = 7;
+constexpr int kKeptAgain = 10;
+// Where the list is longer than a tile a block, a wave with less than a
+// quarter of its rows truncated leaves them to the second pass. Rows of 10
+// with the quadratic basis, of which half are listed and 5 % of those
+// truncated, 3 or 4 a wave, whose V nearly every wave formed: setup of 1M rows
+// (3.8 tiles a block) 1.46 -> 1.22 ms, of 300k (1.1) 590 -> 565 us; of 250k
+// (0.95) the second pass's own latency would cost 20 us. Where every row is
+// truncated (a shell) it would only repeat the sweeps. A share of 1/8 left
+// 1.27 ms, 1/2 as 1/4.
 // two waves a SIMD at this kernel's registers (one: 1.21 ms)
 constexpr int kListedBlocks = 2048;
 
@@ -423,119 +442,244 @@ int64_t listed_blocks( int64_t rows )
     return std::min<int64_t>( ceil_div( rows, kBlock ), kListedBlocks );
 }
 
+// blocks of the second pass that take truncated rows: their ten regions
+// within the first pass's scratch
+int64_t again_blocks( int64_t rows )
+{
+    return std::max<int64_t>( listed_blocks( rows ) * kKeptSweeps / kKeptAgain,
+                              1 );
+}
+
+struct Listed
+{
+    double4 const *src, *tgt;
+    int32_t const *indices, *order;
+    int64_t const *row_off;
+    int32_t const *rows, *n_rows;
+    int kk, rbf, geometry, truncation;
+    double rcond;
+    int max_sweeps;
+    bool by_distance;
+    double *coeffs;
+    float *coeffs32;
+    double *tangents;
+    unsigned long long *counters;
+    // rows for Cholesky from the front of refine_rows, rows for the second
+    // pass from its end (both together are at most the listed rows)
+    int32_t *refine_rows, *n_refine, *n_later;
+    int64_t refine_end;
+    int32_t *full_rows, *n_full, *queue, *refine_queue;
+};
+
+// the coefficients of a row whose a0 is x
 template <int M, bool F32>
-__global__ void __launch_bounds__( kBlock, 2 )
-    eigen_listed_kernel( double4 const *__restrict__ src,
-                         double4 const *__restrict__ tgt,
-                         int32_t const *__restrict__ indices,
-                         int32_t const *__restrict__ order,
-                         int64_t const *__restrict__ row_off,
-                         int32_t const *__restrict__ rows,
-                         int32_t const *__restrict__ n_rows, int kk_uniform,
-                         int rbf, int geometry, int truncation, double rcond,
-                         int max_sweeps, double *__restrict__ coeffs,
-                         float *__restrict__ coeffs32,
-                         double *__restrict__ tangents,
-                         unsigned long long *__restrict__ counters,
-                         bool by_distance,
-                         int32_t *__restrict__ refine_rows,
-                         int32_t *__restrict__ n_refine,
-                         int32_t *__restrict__ full_rows,
-                         int32_t *__restrict__ n_full,
-                         int32_t *__restrict__ queue )
+__device__ __forceinline__ void listed_coefficients( Listed const &a,
+                                                     double const *x,
+                                                     SystemRow const &sr )
+{
+    for ( int l = 0; l < sr.kk; ++l )
+    {
+        double P[M];
+        double const phi = nbr_row<M, F32>( a.geometry, a.rbf, sr.radius,
+                                            a.src[sr.nbr[l]], sr.tp, P );
+        double acc = 0.0;
+#pragma unroll
+        for ( int j = 0; j < M; ++j )
+            acc = fma( x[j], P[j], acc );
+        if constexpr ( F32 )
+            a.coeffs32[sr.rbeg + l] = (float)( acc * phi );
+        else
+            a.coeffs[sr.rbeg + l] = acc * phi;
+    }
+}
+
+// one row (every lane of the wave has to call: the vote); AGAIN: the second
+// pass, whose rows are all truncated; sparse: waves with few truncated rows
+// leave them to it
+template <int M, bool F32, bool AGAIN>
+__device__ __forceinline__ void listed_row( Listed const &a, bool valid,
+                                            int64_t slot, double *mine,
+                                            bool sparse )
 {
     using S = SymIdx<M>;
+    constexpr int kKept = AGAIN ? kKeptAgain : kKeptSweeps;
+    double A[S::size];
+    (void)system_moments<M, F32>( valid, slot, a.src, a.tgt, a.indices,
+                                  a.order, a.row_off, a.kk, a.rbf, a.geometry,
+                                  a.by_distance, A );
+    double no_v[1];
+    int sweeps = 0, pass = 0;
+    bool done = !valid || converged<M>( A );
+    for ( ; !__all( done ) && pass < a.max_sweeps; ++pass )
+    {
+        int const keep = pass < kKept ? pass : kKept - 1;
+        sweep_all<M, 0, true>( A, no_v, done,
+                               mine + keep * rotations<M> * kLanes );
+        sweeps += done ? 0 : 1;
+        done = done || converged<M>( A );
+    }
+    double thr;
+    bool const under = valid && truncated<M>( A, a.truncation, a.rcond, thr );
+    bool finite = true;
+#pragma unroll
+    for ( int k = 0; k < M; ++k )
+        finite = finite && fabs( A[S::at( k, k )] ) <= DBL_MAX;
+    bool here = under && finite && sweeps < kKept;
+    if constexpr ( !AGAIN )
+    {
+        int const formed = __popcll( __ballot( here ) );
+        int const rows = __popcll( __ballot( valid ) );
+        here = here && ( !sparse || 4 * formed >= rows );
+        if ( valid && !under )
+            a.refine_rows[atomicAdd( a.n_refine, 1 )] = (int32_t)slot;
+        if ( under && finite && !here )
+            a.refine_rows[a.refine_end - atomicAdd( a.n_later, 1 )] =
+                (int32_t)slot;
+    }
+    if ( under && !here && ( AGAIN || !finite ) )
+        a.full_rows[atomicAdd( a.n_full, 1 )] = (int32_t)slot;
+    if ( a.counters && valid && ( here || !under ) )
+    {
+        if ( under )
+            atomicAdd( a.counters + 0, 1ull );
+        if ( !done )
+            atomicAdd( a.counters + 1, 1ull );
+        atomicAdd( a.counters + 2, (unsigned long long)sweeps );
+    }
+    if ( !here )
+        return;
+    double lambda[M], x[M];
+#pragma unroll
+    for ( int k = 0; k < M; ++k )
+        lambda[k] = A[S::at( k, k )];
+    {
+        double V[M * M];
+#pragma unroll
+        for ( int e = 0; e < M * M; ++e )
+            V[e] = e / M == e % M ? 1.0 : 0.0;
+        for ( int p = 0; p < sweeps; ++p )
+            sweep_vectors<M>( V, mine + p * rotations<M> * kLanes );
+#pragma unroll
+        for ( int r = 0; r < M; ++r )
+            x[r] = 0.0;
+#pragma unroll
+        for ( int k = 0; k < M; ++k )
+        {
+            double const w = fabs( lambda[k] ) >= thr ? V[k] / lambda[k] : 0.0;
+#pragma unroll
+            for ( int r = 0; r < M; ++r )
+                x[r] = fma( w, V[r * M + k], x[r] );
+        }
+    }
+    // the row read again instead of held through the sweeps (its 14 registers
+    // were spilled there: 4.60 -> 4.48 ms for the 2M rows of a shell); the
+    // empty statement hides from the compiler that it is the same row
+    int32_t again = (int32_t)slot;
+    asm volatile( "" : "+v"( again ) );
+    listed_coefficients<M, F32>(
+        a, x,
+        system_row<M, F32>( true, again, a.src, a.tgt, a.indices, a.order,
+                            a.row_off, a.kk, a.geometry, a.by_distance ) );
+}
+
+template <int M, bool F32>
+__global__ void __launch_bounds__( kBlock, 2 ) eigen_listed_kernel( Listed a )
+{
     double *const mine =
-        tangents + (int64_t)blockIdx.x * kKeptSweeps * rotations<M> * kLanes +
+        a.tangents + (int64_t)blockIdx.x * kKeptSweeps * rotations<M> * kLanes +
         threadIdx.x;
     // tiles in dispatch order spread the list's first tiles over the XCDs; a
     // block's next one comes from the queue (uniform over the block: the
     // wave-wide vote needs every lane), which ends with the list
-    int64_t const n = *n_rows;
+    int64_t const n = *a.n_rows;
+    bool const sparse = n > (int64_t)gridDim.x * kBlock;
     auto next = [&]() {
         int t = 0;
         if ( threadIdx.x == 0 )
-            t = atomicAdd( queue, 1 );
+            t = atomicAdd( a.queue, 1 );
         return (int64_t)gridDim.x + __builtin_amdgcn_readfirstlane( t );
     };
     for ( int64_t tile = blockIdx.x; tile * kBlock < n; tile = next() )
     {
         int64_t const li = tile * kBlock + threadIdx.x;
         bool const valid = li < n;
-        int64_t const slot = valid ? rows[li] : 0;
-        double A[S::size];
-        SystemRow const sr = system_moments<M, F32>(
-            valid, slot, src, tgt, indices, order, row_off, kk_uniform, rbf,
-            geometry, by_distance, A );
-        double no_v[1];
-        int sweeps = 0, pass = 0;
-        bool done = !valid || converged<M>( A );
-        for ( ; !__all( done ) && pass < max_sweeps; ++pass )
+        listed_row<M, F32, false>( a, valid, valid ? a.rows[li] : 0, mine,
+                                   sparse );
+    }
+}
+
+// The untruncated rows again by Cholesky, one lane a row: the moments, their
+// inverse factor and the row's coefficients. A non-positive pivot sends the
+// row to full_rows.
+template <int M, bool F32>
+__device__ __forceinline__ void refine_row( Listed const &a, int64_t slot )
+{
+    using S = SymIdx<M>;
+    double A[S::size];
+    SystemRow const sr = system_moments<M, F32>(
+        true, slot, a.src, a.tgt, a.indices, a.order, a.row_off, a.kk, a.rbf,
+        a.geometry, a.by_distance, A );
+    if ( !cholesky_factor_inverse<M>( A ) )
+    {
+        a.full_rows[atomicAdd( a.n_full, 1 )] = (int32_t)slot;
+        return;
+    }
+    double x[M];
+#pragma unroll
+    for ( int i = 0; i < M; ++i )
+    {
+        double acc = 0.0;
+#pragma unroll
+        for ( int k = i; k < M; ++k )
+            acc = fma( A[S::at( i, k )], A[S::at( 0, k )], acc );
+        x[i] = acc;
+    }
+    listed_coefficients<M, F32>( a, x, sr );
+}
+
+// What the first pass left: its truncated rows, packed into full waves, over
+// the first n_again blocks, and the Cholesky rows beside them, tiles from a
+// queue that the blocks without truncated rows start on at once.
+template <int M, bool F32>
+__global__ void __launch_bounds__( kBlock, 2 )
+    listed_rest_kernel( Listed a, int n_again )
+{
+    int64_t const n_later = *a.n_later;
+    if ( (int)blockIdx.x < n_again )
+    {
+        double *const mine =
+            a.tangents +
+            (int64_t)blockIdx.x * kKeptAgain * rotations<M> * kLanes +
+            threadIdx.x;
+        for ( int64_t tile = blockIdx.x; tile * kBlock < n_later;
+              tile += n_again )
         {
-            int const keep = pass < kKeptSweeps ? pass : kKeptSweeps - 1;
-            sweep_all<M, 0, true>( A, no_v, done,
-                                   mine + keep * rotations<M> * kLanes );
-            sweeps += done ? 0 : 1;
-            done = done || converged<M>( A );
+            int64_t const li = tile * kBlock + threadIdx.x;
+            bool const valid = li < n_later;
+            listed_row<M, F32, true>(
+                a, valid, valid ? a.refine_rows[a.refine_end - li] : 0, mine,
+                false );
         }
-        double thr;
-        bool const under = valid && truncated<M>( A, truncation, rcond, thr );
-        bool finite = true;
-#pragma unroll
-        for ( int k = 0; k < M; ++k )
-            finite = finite && fabs( A[S::at( k, k )] ) <= DBL_MAX;
-        bool const here = under && finite && sweeps < kKeptSweeps;
-        if ( valid && !under )
-            refine_rows[atomicAdd( n_refine, 1 )] = (int32_t)slot;
-        if ( under && !here )
-            full_rows[atomicAdd( n_full, 1 )] = (int32_t)slot;
-        if ( counters && valid && ( here || !under ) )
-        {
-            if ( under )
-                atomicAdd( counters + 0, 1ull );
-            if ( !done )
-                atomicAdd( counters + 1, 1ull );
-            atomicAdd( counters + 2, (unsigned long long)sweeps );
-        }
-        if ( !here )
-            continue;
-        double lambda[M], x[M];
-#pragma unroll
-        for ( int k = 0; k < M; ++k )
-            lambda[k] = A[S::at( k, k )];
-        {
-            double V[M * M];
-#pragma unroll
-            for ( int e = 0; e < M * M; ++e )
-                V[e] = e / M == e % M ? 1.0 : 0.0;
-            for ( int p = 0; p < sweeps; ++p )
-                sweep_vectors<M>( V, mine + p * rotations<M> * kLanes );
-#pragma unroll
-            for ( int r = 0; r < M; ++r )
-                x[r] = 0.0;
-#pragma unroll
-            for ( int k = 0; k < M; ++k )
-            {
-                double const w = fabs( lambda[k] ) >= thr ? V[k] / lambda[k] : 0.0;
-#pragma unroll
-                for ( int r = 0; r < M; ++r )
-                    x[r] = fma( w, V[r * M + k], x[r] );
-            }
-        }
-        for ( int l = 0; l < sr.kk; ++l )
-        {
-            double P[M];
-            double const phi = nbr_row<M, F32>( geometry, rbf, sr.radius,
-                                                src[sr.nbr[l]], sr.tp, P );
-            double acc = 0.0;
-#pragma unroll
-            for ( int j = 0; j < M; ++j )
-                acc = fma( x[j], P[j], acc );
-            if constexpr ( F32 )
-                coeffs32[sr.rbeg + l] = (float)( acc * phi );
-            else
-                coeffs[sr.rbeg + l] = acc * phi;
-        }
+    }
+    // a block's first tile is its own (one atomic a block on a single word cost
+    // a short list 15 us), counted from the first block without truncated
+    // rows; later ones come from the queue
+    int64_t const n = *a.n_refine;
+    int64_t const tiles = ( n_later + kBlock - 1 ) / kBlock;
+    int64_t const busy = tiles < n_again ? tiles : n_again;
+    auto next = [&]() {
+        int t = 0;
+        if ( threadIdx.x == 0 )
+            t = atomicAdd( a.refine_queue, 1 );
+        return (int64_t)gridDim.x + __builtin_amdgcn_readfirstlane( t );
+    };
+    int64_t const first =
+        blockIdx.x + ( blockIdx.x < busy ? (int64_t)gridDim.x : 0 ) - busy;
+    for ( int64_t tile = first; tile * kBlock < n; tile = next() )
+    {
+        int64_t const li = tile * kBlock + threadIdx.x;
+        if ( li < n )
+            refine_row<M, F32>( a, a.refine_rows[li] );
     }
 }
 
@@ -544,39 +688,42 @@ __global__ void __launch_bounds__( kBlock, 2 )
 std::size_t setup_listed_scratch( int m, int64_t rows )
 {
     int const n = m == 10 ? rotations<10> : ( m == 4 ? rotations<4> : 0 );
-    return static_cast<std::size_t>( listed_blocks( rows ) ) * kKeptSweeps * n *
-           kLanes;
+    int64_t const regions = std::max<int64_t>(
+        listed_blocks( rows ) * kKeptSweeps, again_blocks( rows ) * kKeptAgain );
+    return static_cast<std::size_t>( regions ) * n * kLanes;
 }
 
 void setup_listed( double4 const *src, double4 const *tgt, int64_t n_tgt,
                    int32_t const *indices, int32_t const *order,
                    SetupParams const &p, double *coeffs, float *coeffs32,
-                   int32_t *full_rows, int32_t *n_full, int32_t *queue,
+                   int32_t *full_rows, int32_t *n_full, int32_t *counts,
                    unsigned long long *counters, hipStream_t s )
 {
-    DTKX_REQUIRE( p.rows && p.n_rows && p.refine_rows && p.n_refine,
-                  DTKX_ERR_INVALID_ARGUMENT );
+    DTKX_REQUIRE( p.rows && p.n_rows, DTKX_ERR_INVALID_ARGUMENT );
     if ( n_tgt <= p.row0 )
         return;
-    int const sweeps = p.max_rot > 0 ? static_cast<int>( p.max_rot ) : 30;
-    int64_t const blocks = listed_blocks( n_tgt - p.row0 );
+    int64_t const n = n_tgt - p.row0, blocks = listed_blocks( n );
+    DeviceBuffer<int32_t> rlist( n, s );
     DeviceBuffer<double> owned;
     double *tangents = p.tangents;
     if ( !tangents )
     {
-        owned.resize( std::max<std::size_t>(
-                          setup_listed_scratch( p.m, n_tgt - p.row0 ), 1 ),
+        owned.resize( std::max<std::size_t>( setup_listed_scratch( p.m, n ), 1 ),
                       s );
         tangents = owned.get();
     }
+    int const sweeps = p.max_rot > 0 ? static_cast<int>( p.max_rot ) : 30;
+    Listed const a{ src, tgt, indices, order, p.row_off, p.rows, p.n_rows, p.kk,
+                    p.rbf, p.geometry, p.truncation, p.rcond, sweeps,
+                    p.by_distance, coeffs, coeffs32, tangents, counters,
+                    rlist.get(), counts, counts + 1, n - 1,
+                    full_rows, n_full, counts + 2, counts + 3 };
     auto run = [&]( auto m, auto f32 ) {
         constexpr int kM = decltype( m )::value;
-        eigen_listed_kernel<kM, decltype( f32 )::value>
-            <<<blocks, kBlock, 0, s>>>(
-                src, tgt, indices, order, p.row_off, p.rows, p.n_rows, p.kk,
-                p.rbf, p.geometry, p.truncation, p.rcond, sweeps, coeffs,
-                coeffs32, tangents, counters, p.by_distance, p.refine_rows,
-                p.n_refine, full_rows, n_full, queue );
+        constexpr bool kF32 = decltype( f32 )::value;
+        eigen_listed_kernel<kM, kF32><<<blocks, kBlock, 0, s>>>( a );
+        listed_rest_kernel<kM, kF32><<<blocks, kBlock, 0, s>>>(
+            a, static_cast<int>( again_blocks( n ) ) );
     };
     using T = std::true_type;
     using F = std::false_type;

@@ -222,93 +222,6 @@ __global__ void __launch_bounds__( kBlock, 2 )
     }
 }
 
-// The eigen-solver's untruncated rows again, one lane per listed row: the
-// moments, their Cholesky inverse factor and the row's coefficients (a
-// non-positive pivot leaves the eigen-solver's coefficients in place). A
-// bounded grid strides over the list, whose length only the device knows.
-constexpr int kRefineBlocks = 1024;
-
-template <int M, bool F32>
-__global__ void __launch_bounds__( kBlock )
-    refine_kernel( double4 const *__restrict__ src,
-                   double4 const *__restrict__ tgt,
-                   int32_t const *__restrict__ indices,
-                   int32_t const *__restrict__ order,
-                   int64_t const *__restrict__ row_off, int kk_uniform,
-                   int rbf, int geometry, int32_t const *__restrict__ rows,
-                   int32_t const *__restrict__ n_rows,
-                   double *__restrict__ coeffs, float *__restrict__ coeffs32,
-                   bool by_distance,
-                   int32_t *__restrict__ full_rows,
-                   int32_t *__restrict__ n_full )
-{
-    using S = SymIdx<M>;
-    int64_t const n = *n_rows;
-    for ( int64_t li = blockIdx.x * (int64_t)kBlock + threadIdx.x; li < n;
-          li += (int64_t)gridDim.x * kBlock )
-    {
-        int64_t const slot = rows[li];
-        int64_t const t = order ? order[slot] : slot;
-        int64_t const rbeg = row_off ? row_off[slot] : slot * kk_uniform;
-        int const kk =
-            row_off ? (int)( row_off[slot + 1] - rbeg ) : kk_uniform;
-        int32_t const *nbr = indices + rbeg;
-        double4 const tp = tgt[t];
-        double const dmax =
-            row_reach<M, F32>( geometry, by_distance, src, nbr, kk, tp );
-        double const radius =
-            F32 ? (double)( 1.1f * (float)dmax ) : 1.1 * dmax;
-        double A[S::size];
-#pragma unroll
-        for ( int e = 0; e < S::size; ++e )
-            A[e] = 0.0;
-        for ( int l = 0; l < kk; ++l )
-        {
-            double P[M];
-            double const phi =
-                nbr_row<M, F32>( geometry, rbf, radius, src[nbr[l]], tp, P );
-#pragma unroll
-            for ( int r = 0; r < M; ++r )
-            {
-                double const pr = P[r] * phi;
-#pragma unroll
-                for ( int c = r; c < M; ++c )
-                    A[S::at( r, c )] = fma( pr, P[c], A[S::at( r, c )] );
-            }
-        }
-        if ( !cholesky_factor_inverse<M>( A ) )
-        {
-            // to the eigen-solver with eigenvectors, which runs next
-            full_rows[atomicAdd( n_full, 1 )] = (int32_t)slot;
-            continue;
-        }
-        double x[M];
-#pragma unroll
-        for ( int i = 0; i < M; ++i )
-        {
-            double acc = 0.0;
-#pragma unroll
-            for ( int k = i; k < M; ++k )
-                acc = fma( A[S::at( i, k )], A[S::at( 0, k )], acc );
-            x[i] = acc;
-        }
-        for ( int l = 0; l < kk; ++l )
-        {
-            double P[M];
-            double const phi =
-                nbr_row<M, F32>( geometry, rbf, radius, src[nbr[l]], tp, P );
-            double acc = 0.0;
-#pragma unroll
-            for ( int q = 0; q < M; ++q )
-                acc = fma( x[q], P[q], acc );
-            if constexpr ( F32 )
-                coeffs32[rbeg + l] = (float)( acc * phi );
-            else
-                coeffs[rbeg + l] = acc * phi;
-        }
-    }
-}
-
 template <int M>
 void launch_fast( double4 const *src, double4 const *tgt, int64_t n_tgt,
                   int32_t const *indices, int32_t const *order,
@@ -345,8 +258,10 @@ void setup_fast( double4 const *src, double4 const *tgt, int64_t n_tgt,
         return;
     DTKX_REQUIRE( p.m == 1 || p.m == 4 || p.m == 10,
                   DTKX_ERR_INVALID_ARGUMENT );
-    DeviceBuffer<int32_t> list( n_tgt - p.row0, s ), count( 1, s );
-    zero_async( count.get(), sizeof( int32_t ), s );
+    int64_t const nl = n_tgt - p.row0;
+    // listed rows, rows for the eigen-solver, and setup_listed's four
+    DeviceBuffer<int32_t> list( nl, s ), count( 6, s );
+    zero_async( count.get(), 6 * sizeof( int32_t ), s );
     if ( p.m == 1 )
         launch_fast<1>( src, tgt, n_tgt, indices, order, p, coeffs, coeffs32,
                         pinv, list.get(), count.get(), counters, s );
@@ -369,43 +284,16 @@ void setup_fast( double4 const *src, double4 const *tgt, int64_t n_tgt,
         return;
     }
     // otherwise by their eigenvalues: the rows with one below the threshold
-    // are set up where these are found, those with none have A^+ = A^-1 and
-    // are solved again by Cholesky, and the few that neither can take (the
-    // one lists them, and the other the rows whose Cholesky meets a
-    // non-positive pivot) go to the eigen-solver with eigenvectors.
-    int64_t const nl = n_tgt - p.row0;
-    DeviceBuffer<int32_t> rlist( nl, s ), flist( nl, s ),
-        counts( 3, s ); // refine, left over, queue
-    zero_async( counts.get(), 3 * sizeof( int32_t ), s );
-    q.refine_rows = rlist.get();
-    q.n_refine = counts.get();
+    // are set up from them, those with none have A^+ = A^-1 and are solved
+    // again by Cholesky, and the few that neither can take go to the
+    // eigen-solver with eigenvectors.
+    DeviceBuffer<int32_t> flist( nl, s );
     setup_listed( src, tgt, n_tgt, indices, order, q, coeffs, coeffs32,
-                  flist.get(), counts.get() + 1, counts.get() + 2, counters, s );
-    int64_t const blocks =
-        std::min<int64_t>( ceil_div( nl, kBlock ), kRefineBlocks );
-    auto refine = [&]( auto m, auto f32 ) {
-        refine_kernel<decltype( m )::value, decltype( f32 )::value>
-            <<<blocks, kBlock, 0, s>>>(
-                src, tgt, indices, order, p.row_off, p.kk, p.rbf, p.geometry,
-                rlist.get(), counts.get(), coeffs, coeffs32, p.by_distance,
-                flist.get(), counts.get() + 1 );
-    };
-    using T = std::true_type;
-    using F = std::false_type;
-    using M1 = std::integral_constant<int, 1>;
-    using M4 = std::integral_constant<int, 4>;
-    using M10 = std::integral_constant<int, 10>;
-    if ( p.m == 1 )
-        coeffs32 ? refine( M1{}, T{} ) : refine( M1{}, F{} );
-    else if ( p.m == 4 )
-        coeffs32 ? refine( M4{}, T{} ) : refine( M4{}, F{} );
-    else
-        coeffs32 ? refine( M10{}, T{} ) : refine( M10{}, F{} );
-    DTKX_HIP( hipGetLastError() );
+                  flist.get(), count.get() + 1, count.get() + 2, counters, s );
     SetupParams f = p;
     f.screened = true;
     f.rows = flist.get();
-    f.n_rows = counts.get() + 1;
+    f.n_rows = count.get() + 1;
     setup_cyclic( src, tgt, n_tgt, indices, order, f, coeffs, coeffs32,
                   nullptr, counters, s );
 }
