@@ -421,9 +421,11 @@ void launch_cyclic( double4 const *src, double4 const *tgt, int64_t n_tgt,
 // cost nothing beside the rotations; tiles from a queue instead of a stride
 // 797 -> 688 us of the kernel, as 4,688 tiles over 2,048 blocks leave some
 // with a third; gathers four neighbours at a time gave nothing.
-// Seven regions keep six sweeps: the shell's rows take 4.3 on average, and
-// seven regions measure as ten do (setup 1.04-1.06 ms), at 330 MB of scratch
-// instead of 472.
+// The full grid's blocks have seven regions each, for six sweeps: the shell's
+// rows take 4.3 on average, and at its size seven regions measure as ten do
+// (setup 1.04-1.06 ms), at 330 MB of scratch instead of 472. A smaller grid's
+// blocks share as many, up to ten each: there a few rows' second pass is a
+// tenth of the setup.
 constexpr int kKeptSweeps = 7;
 constexpr int kKeptAgain = 10;
 // Where the list is longer than a tile a block, a wave with less than a
@@ -442,12 +444,19 @@ int64_t listed_blocks( int64_t rows )
     return std::min<int64_t>( ceil_div( rows, kBlock ), kListedBlocks );
 }
 
+// regions of each block of the first pass
+int kept_regions( int64_t rows )
+{
+    return static_cast<int>( std::min<int64_t>(
+        kListedBlocks * kKeptSweeps / listed_blocks( rows ), kKeptAgain ) );
+}
+
 // blocks of the second pass that take truncated rows: their ten regions
 // within the first pass's scratch
 int64_t again_blocks( int64_t rows )
 {
-    return std::max<int64_t>( listed_blocks( rows ) * kKeptSweeps / kKeptAgain,
-                              1 );
+    return std::max<int64_t>(
+        listed_blocks( rows ) * kept_regions( rows ) / kKeptAgain, 1 );
 }
 
 struct Listed
@@ -463,6 +472,7 @@ struct Listed
     double *coeffs;
     float *coeffs32;
     double *tangents;
+    int kept;
     unsigned long long *counters;
     // rows for Cholesky from the front of refine_rows, rows for the second
     // pass from its end (both together are at most the listed rows)
@@ -502,7 +512,7 @@ __device__ __forceinline__ void listed_row( Listed const &a, bool valid,
                                             bool sparse )
 {
     using S = SymIdx<M>;
-    constexpr int kKept = AGAIN ? kKeptAgain : kKeptSweeps;
+    int const kept = AGAIN ? kKeptAgain : a.kept;
     double A[S::size];
     (void)system_moments<M, F32>( valid, slot, a.src, a.tgt, a.indices,
                                   a.order, a.row_off, a.kk, a.rbf, a.geometry,
@@ -512,7 +522,7 @@ __device__ __forceinline__ void listed_row( Listed const &a, bool valid,
     bool done = !valid || converged<M>( A );
     for ( ; !__all( done ) && pass < a.max_sweeps; ++pass )
     {
-        int const keep = pass < kKept ? pass : kKept - 1;
+        int const keep = pass < kept ? pass : kept - 1;
         sweep_all<M, 0, true>( A, no_v, done,
                                mine + keep * rotations<M> * kLanes );
         sweeps += done ? 0 : 1;
@@ -524,7 +534,7 @@ __device__ __forceinline__ void listed_row( Listed const &a, bool valid,
 #pragma unroll
     for ( int k = 0; k < M; ++k )
         finite = finite && fabs( A[S::at( k, k )] ) <= DBL_MAX;
-    bool here = under && finite && sweeps < kKept;
+    bool here = under && finite && sweeps < kept;
     if constexpr ( !AGAIN )
     {
         int const formed = __popcll( __ballot( here ) );
@@ -586,7 +596,7 @@ template <int M, bool F32>
 __global__ void __launch_bounds__( kBlock, 2 ) eigen_listed_kernel( Listed a )
 {
     double *const mine =
-        a.tangents + (int64_t)blockIdx.x * kKeptSweeps * rotations<M> * kLanes +
+        a.tangents + (int64_t)blockIdx.x * a.kept * rotations<M> * kLanes +
         threadIdx.x;
     // tiles in dispatch order spread the list's first tiles over the XCDs; a
     // block's next one comes from the queue (uniform over the block: the
@@ -688,8 +698,11 @@ __global__ void __launch_bounds__( kBlock, 2 )
 std::size_t setup_listed_scratch( int m, int64_t rows )
 {
     int const n = m == 10 ? rotations<10> : ( m == 4 ? rotations<4> : 0 );
-    int64_t const regions = std::max<int64_t>(
-        listed_blocks( rows ) * kKeptSweeps, again_blocks( rows ) * kKeptAgain );
+    if ( rows <= 0 )
+        return 0;
+    int64_t const regions =
+        std::max<int64_t>( listed_blocks( rows ) * kept_regions( rows ),
+                           again_blocks( rows ) * kKeptAgain );
     return static_cast<std::size_t>( regions ) * n * kLanes;
 }
 
@@ -715,7 +728,7 @@ void setup_listed( double4 const *src, double4 const *tgt, int64_t n_tgt,
     int const sweeps = p.max_rot > 0 ? static_cast<int>( p.max_rot ) : 30;
     Listed const a{ src, tgt, indices, order, p.row_off, p.rows, p.n_rows, p.kk,
                     p.rbf, p.geometry, p.truncation, p.rcond, sweeps,
-                    p.by_distance, coeffs, coeffs32, tangents, counters,
+                    p.by_distance, coeffs, coeffs32, tangents, kept_regions( n ), counters,
                     rlist.get(), counts, counts + 1, n - 1,
                     full_rows, n_full, counts + 2, counts + 3 };
     auto run = [&]( auto m, auto f32 ) {
