@@ -76,7 +76,7 @@ void setup_cyclic( double4 const *src, double4 const *tgt, int64_t n_tgt,
 // truncation test are solved again by Cholesky, the others from their
 // rotations; the few that neither can take are appended to full_rows
 // (*n_full), and its counters leave out those of them with an eigenvalue
-// below the threshold. coeffs32 as in setup_cyclic; *n_full and the four
+// below the threshold. coeffs32 as in setup_cyclic; *n_full and the five
 // counts are zero before.
 std::size_t setup_listed_scratch( int m, int64_t rows );
 void setup_listed( double4 const *src, double4 const *tgt, int64_t n_tgt,

@@ -404,8 +404,8 @@ void launch_cyclic( double4 const *src, double4 const *tgt, int64_t n_tgt,
 // rotations never read V. Rows whose eigenvalues all pass the truncation test
 // go to refine_rows (solved again by Cholesky). For the others V is formed
 // afterwards, in the registers that A leaves, from the rotations' tangents
-// (kept for each wave and sweep; the last region takes all later sweeps and
-// is not read). The operations are cyclic_system's and a converged system's
+// (kept for each wave and sweep; the last region takes all later sweeps,
+// which are not read). The operations are cyclic_system's and a converged system's
 // rotations exact no-ops whatever its wave, so all results are its bit for
 // bit. A wave with few truncated rows, or a row that took more sweeps than
 // are kept, leaves those to a second pass (listed_rest_kernel), where the
@@ -428,6 +428,11 @@ void launch_cyclic( double4 const *src, double4 const *tgt, int64_t n_tgt,
 // tenth of the setup.
 constexpr int kKeptSweeps = 7;
 constexpr int kKeptAgain = 10;
+// A block whose rows need more takes one of these further shares, of three
+// regions, if any is left: one wave with a seventh sweep would otherwise add
+// the second pass's whole latency (a shell of 130k rows 0.85 -> 1.04 ms).
+constexpr int kSpares = 128;
+constexpr int kSpareRegions = 3;
 // Where the list is longer than a tile a block, a wave with less than a
 // quarter of its rows truncated leaves them to the second pass. Rows of 10
 // with the quadratic basis, of which half are listed and 5 % of those
@@ -459,6 +464,13 @@ int64_t again_blocks( int64_t rows )
         listed_blocks( rows ) * kept_regions( rows ) / kKeptAgain, 1 );
 }
 
+// regions of the first pass, or of the second
+int64_t listed_regions( int64_t rows )
+{
+    return std::max<int64_t>( listed_blocks( rows ) * kept_regions( rows ),
+                              again_blocks( rows ) * kKeptAgain );
+}
+
 struct Listed
 {
     double4 const *src, *tgt;
@@ -471,14 +483,14 @@ struct Listed
     bool by_distance;
     double *coeffs;
     float *coeffs32;
-    double *tangents;
+    double *tangents, *spares;
     int kept;
     unsigned long long *counters;
     // rows for Cholesky from the front of refine_rows, rows for the second
     // pass from its end (both together are at most the listed rows)
     int32_t *refine_rows, *n_refine, *n_later;
     int64_t refine_end;
-    int32_t *full_rows, *n_full, *queue, *refine_queue;
+    int32_t *full_rows, *n_full, *queue, *refine_queue, *n_spares;
 };
 
 // the coefficients of a row whose a0 is x
@@ -503,16 +515,31 @@ __device__ __forceinline__ void listed_coefficients( Listed const &a,
     }
 }
 
+// a block's spare share: its number, none asked for yet, or none left
+constexpr int kNoSpare = -1;
+constexpr int kSparesGone = -2;
+
 // one row (every lane of the wave has to call: the vote); AGAIN: the second
 // pass, whose rows are all truncated; sparse: waves with few truncated rows
 // leave them to it
 template <int M, bool F32, bool AGAIN>
 __device__ __forceinline__ void listed_row( Listed const &a, bool valid,
                                             int64_t slot, double *mine,
-                                            bool sparse )
+                                            bool sparse, int &spare )
 {
     using S = SymIdx<M>;
+    constexpr int kStride = rotations<M> * kLanes;
     int const kept = AGAIN ? kKeptAgain : a.kept;
+    // where a sweep's tangents are (sweeps beyond the kept ones: the spare
+    // share if the block has one, else over the last region)
+    auto region = [&]( int pass ) {
+        int const last = ( !AGAIN && spare >= 0 ? kSpareRegions : 0 ) + kept - 1;
+        int const p = pass < last ? pass : last;
+        return p < kept ? mine + p * kStride
+                        : a.spares + threadIdx.x +
+                              ( (int64_t)spare * kSpareRegions + p - kept ) *
+                                  kStride;
+    };
     double A[S::size];
     (void)system_moments<M, F32>( valid, slot, a.src, a.tgt, a.indices,
                                   a.order, a.row_off, a.kk, a.rbf, a.geometry,
@@ -522,9 +549,16 @@ __device__ __forceinline__ void listed_row( Listed const &a, bool valid,
     bool done = !valid || converged<M>( A );
     for ( ; !__all( done ) && pass < a.max_sweeps; ++pass )
     {
-        int const keep = pass < kept ? pass : kept - 1;
-        sweep_all<M, 0, true>( A, no_v, done,
-                               mine + keep * rotations<M> * kLanes );
+        if constexpr ( !AGAIN )
+            if ( pass == kept && spare == kNoSpare )
+            {
+                int taken = 0;
+                if ( threadIdx.x == 0 )
+                    taken = atomicAdd( a.n_spares, 1 );
+                taken = __builtin_amdgcn_readfirstlane( taken );
+                spare = taken < kSpares ? taken : kSparesGone;
+            }
+        sweep_all<M, 0, true>( A, no_v, done, region( pass ) );
         sweeps += done ? 0 : 1;
         done = done || converged<M>( A );
     }
@@ -534,7 +568,11 @@ __device__ __forceinline__ void listed_row( Listed const &a, bool valid,
 #pragma unroll
     for ( int k = 0; k < M; ++k )
         finite = finite && fabs( A[S::at( k, k )] ) <= DBL_MAX;
-    bool here = under && finite && sweeps < kept;
+    // a sweep is kept if no later one was written over it
+    int const readable =
+        kept + ( !AGAIN && spare >= 0 ? kSpareRegions : 0 );
+    bool here =
+        under && finite && ( sweeps < readable || pass <= readable );
     if constexpr ( !AGAIN )
     {
         int const formed = __popcll( __ballot( here ) );
@@ -568,7 +606,7 @@ __device__ __forceinline__ void listed_row( Listed const &a, bool valid,
         for ( int e = 0; e < M * M; ++e )
             V[e] = e / M == e % M ? 1.0 : 0.0;
         for ( int p = 0; p < sweeps; ++p )
-            sweep_vectors<M>( V, mine + p * rotations<M> * kLanes );
+            sweep_vectors<M>( V, region( p ) );
 #pragma unroll
         for ( int r = 0; r < M; ++r )
             x[r] = 0.0;
@@ -603,6 +641,7 @@ __global__ void __launch_bounds__( kBlock, 2 ) eigen_listed_kernel( Listed a )
     // wave-wide vote needs every lane), which ends with the list
     int64_t const n = *a.n_rows;
     bool const sparse = n > (int64_t)gridDim.x * kBlock;
+    int spare = kNoSpare;
     auto next = [&]() {
         int t = 0;
         if ( threadIdx.x == 0 )
@@ -614,7 +653,7 @@ __global__ void __launch_bounds__( kBlock, 2 ) eigen_listed_kernel( Listed a )
         int64_t const li = tile * kBlock + threadIdx.x;
         bool const valid = li < n;
         listed_row<M, F32, false>( a, valid, valid ? a.rows[li] : 0, mine,
-                                   sparse );
+                                   sparse, spare );
     }
 }
 
@@ -661,6 +700,7 @@ __global__ void __launch_bounds__( kBlock, 2 )
             a.tangents +
             (int64_t)blockIdx.x * kKeptAgain * rotations<M> * kLanes +
             threadIdx.x;
+        int none = kSparesGone;
         for ( int64_t tile = blockIdx.x; tile * kBlock < n_later;
               tile += n_again )
         {
@@ -668,7 +708,7 @@ __global__ void __launch_bounds__( kBlock, 2 )
             bool const valid = li < n_later;
             listed_row<M, F32, true>(
                 a, valid, valid ? a.refine_rows[a.refine_end - li] : 0, mine,
-                false );
+                false, none );
         }
     }
     // a block's first tile is its own (one atomic a block on a single word cost
@@ -700,10 +740,9 @@ std::size_t setup_listed_scratch( int m, int64_t rows )
     int const n = m == 10 ? rotations<10> : ( m == 4 ? rotations<4> : 0 );
     if ( rows <= 0 )
         return 0;
-    int64_t const regions =
-        std::max<int64_t>( listed_blocks( rows ) * kept_regions( rows ),
-                           again_blocks( rows ) * kKeptAgain );
-    return static_cast<std::size_t>( regions ) * n * kLanes;
+    int64_t const regions = listed_regions( rows );
+    return static_cast<std::size_t>( regions + kSpares * kSpareRegions ) * n *
+           kLanes;
 }
 
 void setup_listed( double4 const *src, double4 const *tgt, int64_t n_tgt,
@@ -728,9 +767,11 @@ void setup_listed( double4 const *src, double4 const *tgt, int64_t n_tgt,
     int const sweeps = p.max_rot > 0 ? static_cast<int>( p.max_rot ) : 30;
     Listed const a{ src, tgt, indices, order, p.row_off, p.rows, p.n_rows, p.kk,
                     p.rbf, p.geometry, p.truncation, p.rcond, sweeps,
-                    p.by_distance, coeffs, coeffs32, tangents, kept_regions( n ), counters,
+                    p.by_distance, coeffs, coeffs32, tangents,
+                    tangents + listed_regions( n ) * p.m * ( p.m - 1 ) / 2 * kLanes,
+                    kept_regions( n ), counters,
                     rlist.get(), counts, counts + 1, n - 1,
-                    full_rows, n_full, counts + 2, counts + 3 };
+                    full_rows, n_full, counts + 2, counts + 3, counts + 4 };
     auto run = [&]( auto m, auto f32 ) {
         constexpr int kM = decltype( m )::value;
         constexpr bool kF32 = decltype( f32 )::value;

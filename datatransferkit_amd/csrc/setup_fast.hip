@@ -259,9 +259,9 @@ void setup_fast( double4 const *src, double4 const *tgt, int64_t n_tgt,
     DTKX_REQUIRE( p.m == 1 || p.m == 4 || p.m == 10,
                   DTKX_ERR_INVALID_ARGUMENT );
     int64_t const nl = n_tgt - p.row0;
-    // listed rows, rows for the eigen-solver, and setup_listed's four
-    DeviceBuffer<int32_t> list( nl, s ), count( 6, s );
-    zero_async( count.get(), 6 * sizeof( int32_t ), s );
+    // listed rows, rows for the eigen-solver, and setup_listed's five
+    DeviceBuffer<int32_t> list( nl, s ), count( 7, s );
+    zero_async( count.get(), 7 * sizeof( int32_t ), s );
     if ( p.m == 1 )
         launch_fast<1>( src, tgt, n_tgt, indices, order, p, coeffs, coeffs32,
                         pinv, list.get(), count.get(), counters, s );

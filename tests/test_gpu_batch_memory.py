@@ -1,7 +1,7 @@
 """Device memory that a batch's rebuild graph holds for the scratch of its
 listed rows: one share for all of its groups, of 6 kept sweeps and one more
-(2,048 blocks of 64 rows, 45 rotations, 7 regions of 8 bytes: 330 MB), not one
-for each basis."""
+(2,048 blocks of 64 rows, 45 rotations, 7 regions of 8 bytes: 330 MB, and 9 MB
+of spare regions), not one for each basis."""
 import numpy as np
 import pytest
 
